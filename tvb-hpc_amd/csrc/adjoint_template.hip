@@ -143,6 +143,10 @@ tvbx_adjoint(const tvbx_adj_args A) {
       const int j = __builtin_amdgcn_readfirstlane(j0);
       const size_t jp = (size_t)j * a.pitch + pb;
       if (!one_node) tvbx_load_row_of(ccol, crow, cw, j, crw);
+      if (!one_node || k == 0) {
+#pragma unroll
+        for (int q = 0; q < TVBX_IPL; ++q) tvbx_load_node(lp[q], a, j, pb + q);
+      }
       // the replay's recordings of step n, lambda (when it is not kept in
       // registers) and the forcing of n's sample do not depend on the
       // gathers: their loads are issued first and land while the gathers
@@ -373,7 +377,10 @@ tvbx_logp_grad(const tvbx_logp_args L) {
   const size_t ip = (size_t)i * a.pitch + pb;
   tvbx_lane_params lp[TVBX_IPL];
 #pragma unroll
-  for (int q = 0; q < TVBX_IPL; ++q) tvbx_load_lane(lp[q], a, pb + q);
+  for (int q = 0; q < TVBX_IPL; ++q) {
+    tvbx_load_lane(lp[q], a, pb + q);
+    tvbx_load_node(lp[q], a, i, pb + q);
+  }
   float gm_acc[TVBX_IPL][TVBX_NGM], gc_acc[TVBX_IPL][TVBX_NGC];
   float gm_err[TVBX_IPL][TVBX_NGM], gc_err[TVBX_IPL][TVBX_NGC];
 #pragma unroll

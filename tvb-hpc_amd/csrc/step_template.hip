@@ -16,7 +16,11 @@
 //   TVBX_PRIO        1: wave priority falls with a multi-step launch's progress
 //   TVBX_EMAJ        L > 0: blocked launches of up to L steps form all their
 //                    coupling sums first, edges outer and steps inner
-//   struct tvbx_lane_params + tvbx_load_lane()   per-instance parameters
+//   struct tvbx_lane_params + tvbx_load_lane() / tvbx_load_node(): the
+//                    per-instance parameters, and those of the node (and
+//                    instance), loaded once per node rather than at each
+//                    step, where the ring's stores keep the compiler from
+//                    hoisting the loads
 //   tvbx_pre(), tvbx_post(), tvbx_dfun(), tvbx_obsrv(), tvbx_wrap(),
 //   tvbx_ring_value(), tvbx_bold_step()
 //
@@ -611,7 +615,9 @@ __device__ __forceinline__ bool tvbx_group_redo(const float (&acc0)[TVBX_IPL],
 
 // Coupling sums c[q][kk] of node i at step n (ring slot t): the CSR row
 // reduction of network.py:115-136 over the edges in row order, with rec_sum
-// recording for the adjoint.
+// recording for the adjoint.  RAW: the accumulators go to csum instead, n
+// being the step's index within the launch.
+template <bool RAW = false>
 __device__ __forceinline__ void tvbx_coupling(
     const tvbx_step_args &a, const unsigned *__restrict__ cd,
     const float *__restrict__ wt, const tvbx_row &row,
@@ -751,6 +757,10 @@ __device__ __forceinline__ void tvbx_coupling(
 #undef TVBX_W1
 #undef TVBX_CDS
 #undef TVBX_WS
+    if (RAW) {
+      tvbx_stf(a.csum + ((size_t)n * TVBX_C + kk) * NP + ip, acc);
+      continue;
+    }
 #pragma unroll
     for (int q = 0; q < TVBX_IPL; ++q) {
       acc[q] = acc[q] * tvbx_acc_unscale(a);
@@ -771,12 +781,11 @@ __device__ __forceinline__ void tvbx_coupling(
 // the launch of each other and end together.
 __device__ __forceinline__ void tvbx_progress_prio(int k, int n) {
 #if TVBX_PRIO
-  const int q = (4 * k) / n;
-  if (q == 0)
+  if (4 * k < n)
     __builtin_amdgcn_s_setprio(3);
-  else if (q == 1)
+  else if (4 * k < 2 * n)
     __builtin_amdgcn_s_setprio(2);
-  else if (q == 2)
+  else if (4 * k < 3 * n)
     __builtin_amdgcn_s_setprio(1);
   else
     __builtin_amdgcn_s_setprio(0);
@@ -876,26 +885,46 @@ __device__ __forceinline__ void tvbx_coupling_launch(
 }
 #endif
 
-// Coupling of node i at step k of the launch from sums another kernel
-// computed (csum [n_steps][C][N][pitch]), finished as in tvbx_coupling.
-__device__ __forceinline__ void tvbx_coupling_from_sums(
-    const tvbx_step_args &a, int i, int pb, long long n, int k,
-    const tvbx_lane_params (&lp)[TVBX_IPL], float (&c)[TVBX_IPL][TVBX_C]) {
+// accumulators of node i at step k of the launch, computed by another kernel
+// (csum [n_steps][C][N][pitch])
+__device__ __forceinline__ void tvbx_load_sums(const tvbx_step_args &a,
+                                               size_t ip, int k,
+                                               float (&cs)[TVBX_C][TVBX_IPL]) {
   const size_t NP = (size_t)a.n_node * a.pitch;
-  const size_t ip = (size_t)i * a.pitch + pb;
+#pragma unroll
+  for (int kk = 0; kk < TVBX_C; ++kk)
+    tvbx_ldf(a.csum + ((size_t)k * TVBX_C + kk) * NP + ip, cs[kk]);
+}
+
+// coupling at step n from its accumulators, finished as in tvbx_coupling
+__device__ __forceinline__ void tvbx_coupling_from_sums(
+    const tvbx_step_args &a, size_t ip, long long n,
+    const tvbx_lane_params (&lp)[TVBX_IPL],
+    const float (&cs)[TVBX_C][TVBX_IPL], float (&c)[TVBX_IPL][TVBX_C]) {
+  const size_t NP = (size_t)a.n_node * a.pitch;
 #pragma unroll
   for (int kk = 0; kk < TVBX_C; ++kk) {
     float acc[TVBX_IPL];
-    tvbx_ldf(a.csum + ((size_t)k * TVBX_C + kk) * NP + ip, acc);
 #pragma unroll
     for (int q = 0; q < TVBX_IPL; ++q) {
-      acc[q] = acc[q] * tvbx_acc_unscale(a);
+      acc[q] = cs[kk][q] * tvbx_acc_unscale(a);
       c[q][kk] = tvbx_post(kk, acc[q], lp[q], a);
     }
     if (a.rec_sum != nullptr)
       tvbx_stf(a.rec_sum + ((size_t)(n - a.rec_step0) * TVBX_C + kk) * NP + ip,
                acc);
   }
+}
+
+// forced steps: frame x(n) of the lane's instances
+__device__ __forceinline__ void tvbx_load_frame(
+    const tvbx_step_args &a, size_t ip, long long n,
+    float (&xf)[TVBX_S][TVBX_IPL]) {
+  const size_t NP = (size_t)a.n_node * a.pitch;
+#pragma unroll
+  for (int s = 0; s < TVBX_S; ++s)
+    tvbx_ldf(a.force + ((size_t)(n - a.force_step0) * TVBX_S + s) * NP + ip,
+             xf[s]);
 }
 
 // non-finite flags of the lane's instances (bit q: instance pb + q)
@@ -912,11 +941,14 @@ __device__ __forceinline__ void tvbx_flag_nonfinite(
 // dfun (model.py:105-140), Euler / Euler-Maruyama update (scheme.py:82-97),
 // wrap, non-finite flags (every step with `check`) and the ring values of
 // x(n + 1).  x is updated in place; k is the step's index within the launch.
+// Forced steps take x(n + 1) from xf and add their log density to the
+// compensated sum ls + lc.
 __device__ __forceinline__ void tvbx_advance(
     const tvbx_step_args &a, int i, int pb, long long n, int k,
     const tvbx_lane_params (&lp)[TVBX_IPL], float (&x)[TVBX_IPL][TVBX_S],
     const float (&c)[TVBX_IPL][TVBX_C], float (&yo)[TVBX_R][TVBX_IPL],
-    unsigned &bad, bool check) {
+    const float (&xf)[TVBX_S][TVBX_IPL], float (&ls)[TVBX_IPL],
+    float (&lc)[TVBX_IPL], unsigned &bad, bool check) {
   const size_t NP = (size_t)a.n_node * a.pitch;
   const size_t ip = (size_t)i * a.pitch + pb;
 #pragma unroll
@@ -934,24 +966,19 @@ __device__ __forceinline__ void tvbx_advance(
     float xi[TVBX_S];
     if (a.force != nullptr) {
       // forced step: the transition log density of the given x(n + 1)
-      // (scheme.py:42-48, mu = x + dt f, sd = sqrt(dt) g), accumulated in
-      // FP64; the state then takes the given value
-      const float *__restrict__ xn =
-          a.force + (size_t)(n + 1 - a.force_step0) * TVBX_S * NP + ip + q;
+      // (scheme.py:42-48, mu = x + dt f, sd = sqrt(dt) g), accumulated as a
+      // compensated sum; the state then takes the given value
       float lp_step = 0.0f;
 #pragma unroll
       for (int s = 0; s < TVBX_S; ++s) {
         const float mu = x[q][s] + a.dt * f[s];
-        const float xs1 = xn[(size_t)s * NP];
+        const float xs1 = xf[s][q];
         const float r = xs1 - mu;
         const float sd2 = a.dt * g[s] * g[s];
         lp_step -= r * r / (2.0f * sd2);
         x[q][s] = xs1;
       }
-      float ls = a.logp[ip + q], lc = a.logp[NP + ip + q];
-      tvbx_csum_add(ls, lc, lp_step);
-      a.logp[ip + q] = ls;
-      a.logp[NP + ip + q] = lc;
+      tvbx_csum_add(ls[q], lc[q], lp_step);
     } else {
       if (a.noise_mode == 1) {
 #pragma unroll
@@ -1019,17 +1046,17 @@ __device__ __forceinline__ void tvbx_monitor_obs(
   }
 }
 
-// time average over tavg_period steps; at the period's last step the
+// time average over tavg_period steps; at the period's last step (due) the
 // average (optionally through Balloon-Windkessel) goes to sample slot
 // m mod sample_slots and the accumulator restarts
 __device__ __forceinline__ void tvbx_monitor(const tvbx_step_args &a,
-                                             size_t ip, long long n,
+                                             size_t ip, bool due, long long m,
                                              const float (&y_mon)[TVBX_IPL],
                                              float (&acc_t)[TVBX_IPL]) {
   const size_t NP = (size_t)a.n_node * a.pitch;
 #pragma unroll
   for (int q = 0; q < TVBX_IPL; ++q) acc_t[q] = acc_t[q] + y_mon[q];
-  if (((n + 1) % a.tavg_period) == 0) {
+  if (due) {
     float out[TVBX_IPL];
 #pragma unroll
     for (int q = 0; q < TVBX_IPL; ++q) {
@@ -1037,7 +1064,6 @@ __device__ __forceinline__ void tvbx_monitor(const tvbx_step_args &a,
       if (a.bold) out[q] = tvbx_bold_step(a, ip + q, out[q]);
       acc_t[q] = 0.0f;
     }
-    const long long m = (n + 1) / a.tavg_period - 1;
     tvbx_stf(a.samples + (size_t)(m % a.sample_slots) * NP + ip, out);
   }
 }
@@ -1128,6 +1154,8 @@ tvbx_step(const tvbx_step_args a) {
     for (int i0 = i_begin + wave; i0 < i_end; i0 += nwave) {
       const int i = __builtin_amdgcn_readfirstlane(i0);
       const size_t ip = (size_t)i * a.pitch + pb;
+#pragma unroll
+      for (int q = 0; q < TVBX_IPL; ++q) tvbx_load_node(lp[q], a, i, pb + q);
       float x[TVBX_IPL][TVBX_S], c[TVBX_IPL][TVBX_C];
 #pragma unroll
       for (int s = 0; s < TVBX_S; ++s) {
@@ -1144,8 +1172,18 @@ tvbx_step(const tvbx_step_args a) {
       tvbx_load_row(a, cd, wt, i, rw);
       tvbx_coupling(a, cd, wt, rw, ring, st_cur, i, t, pb, n, lp, c);
 
-      float yo[TVBX_R][TVBX_IPL];
-      tvbx_advance(a, i, pb, n, k, lp, x, c, yo, bad, true);
+      float yo[TVBX_R][TVBX_IPL], xf[TVBX_S][TVBX_IPL], ls[TVBX_IPL],
+          lc[TVBX_IPL];
+      if (a.force != nullptr) {
+        tvbx_load_frame(a, ip, n + 1, xf);
+        tvbx_ldf(a.logp + ip, ls);
+        tvbx_ldf(a.logp + NP + ip, lc);
+      }
+      tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad, true);
+      if (a.force != nullptr) {
+        tvbx_stf(a.logp + ip, ls);
+        tvbx_stf(a.logp + NP + ip, lc);
+      }
 #pragma unroll
       for (int s = 0; s < TVBX_S; ++s) {
         float v[TVBX_IPL];
@@ -1173,7 +1211,8 @@ tvbx_step(const tvbx_step_args a) {
       if (a.tavg_period > 0) {
         float acc_t[TVBX_IPL];
         tvbx_ldf(a.tavg + ip, acc_t);
-        tvbx_monitor(a, ip, n, y_mon, acc_t);
+        tvbx_monitor(a, ip, (n + 1) % a.tavg_period == 0,
+                     (n + 1) / a.tavg_period - 1, y_mon, acc_t);
         tvbx_stf(a.tavg + ip, acc_t);
       }
     }
@@ -1246,7 +1285,9 @@ __device__ __forceinline__ void tvbx_pace_end(const tvbx_step_args &a) {
 }
 
 // The blocked launch of one (instance tile bx, node i) pair: n_steps steps
-// of that node with its state in registers.
+// of that node with its state in registers.  SUMS: the launch's coupling
+// accumulators were computed by another kernel (csum).
+template <bool SUMS>
 __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
                                                  int bx, int i,
                                                  int *pace_on = nullptr) {
@@ -1281,12 +1322,30 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   }
   float acc_t[TVBX_IPL];
   if (a.tavg_period > 0) tvbx_ldf(a.tavg + ip, acc_t);
+#pragma unroll
+  for (int q = 0; q < TVBX_IPL; ++q) tvbx_load_node(lp[q], a, i, pb + q);
+  // the monitor's period: steps into it, and the sample it ends with
+  int ph = 0;
+  long long mo = 0;
+  if (a.tavg_period > 0) {
+    mo = n0 / a.tavg_period;
+    ph = (int)(n0 - mo * a.tavg_period);
+  }
+  // given sums and forced frames are loaded one step ahead
+  float cs[TVBX_C][TVBX_IPL], xf[TVBX_S][TVBX_IPL], ls[TVBX_IPL],
+      lc[TVBX_IPL];
+  if (SUMS) tvbx_load_sums(a, ip, 0, cs);
+  if (a.force != nullptr) {
+    tvbx_load_frame(a, ip, n0 + 1, xf);
+    tvbx_ldf(a.logp + ip, ls);
+    tvbx_ldf(a.logp + NP + ip, lc);
+  }
   // the node's row serves every step of the launch
   tvbx_row rw;
-  tvbx_load_row(a, cd, wt, i, rw);
+  if (!SUMS) tvbx_load_row(a, cd, wt, i, rw);
 #if TVBX_EMAJ
   // all the launch's coupling sums first, edges outer and steps inner
-  const bool emaj = a.ring32 && a.csum == nullptr && a.force == nullptr &&
+  const bool emaj = !SUMS && a.ring32 && a.force == nullptr &&
                     a.rec_sum == nullptr && a.n_steps <= TVBX_EMAJ;
   float ce[TVBX_EMAJ][TVBX_IPL][TVBX_C];
   if (emaj) tvbx_coupling_launch(a, cd, wt, rw, ring, t, pb, a.n_steps, lp, ce);
@@ -1315,16 +1374,28 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
         }
     } else
 #endif
-    if (a.csum != nullptr)
-      tvbx_coupling_from_sums(a, i, pb, n, k, lp, c);
-    else
+    if (SUMS) {
+      tvbx_coupling_from_sums(a, ip, n, lp, cs, c);
+      tvbx_load_sums(a, ip, min(k + 1, a.n_steps - 1), cs);
+    } else {
       tvbx_coupling(a, cd, wt, rw, ring, nullptr, i, t, pb, n, lp, c);
+    }
     float yo[TVBX_R][TVBX_IPL];
-    tvbx_advance(a, i, pb, n, k, lp, x, c, yo, bad, a.force != nullptr);
+    tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad,
+                 a.force != nullptr);
+    if (a.force != nullptr)
+      tvbx_load_frame(a, ip, n + (k + 1 < a.n_steps ? 2 : 1), xf);
 #pragma unroll
     for (int r = 0; r < TVBX_R; ++r)
       tvbx_str(ring_w + tvbx_ring_off(t1, r, i, a) + pb, yo[r]);
-    if (a.tavg_period > 0) tvbx_monitor(a, ip, n, y_mon, acc_t);
+    if (a.tavg_period > 0) {
+      const bool due = ++ph == a.tavg_period;
+      tvbx_monitor(a, ip, due, mo, y_mon, acc_t);
+      if (due) {
+        ph = 0;
+        ++mo;
+      }
+    }
     t = t1;
     if (pace_on != nullptr && k + 1 < a.n_steps) tvbx_pace(a, k, pace_on);
   }
@@ -1342,11 +1413,79 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     tvbx_stf(a.state + s * NP + ip, v);
   }
   if (a.tavg_period > 0) tvbx_stf(a.tavg + ip, acc_t);
+  if (a.force != nullptr) {
+    tvbx_stf(a.logp + ip, ls);
+    tvbx_stf(a.logp + NP + ip, lc);
+  }
 #pragma unroll
   for (int q = 0; q < TVBX_IPL; ++q)
     if ((bad >> q) & 1u) a.bad[pb + q] = 1u;
 }
 
+#if !TVBX_USES_POST && !TVBX_EMAJ
+// The sums of a blocked launch ahead of its updates.  Every step of the
+// launch reads slots written before it and pre() does not read post_syn, so
+// the launch's coupling accumulators need none of its updates: this kernel
+// forms them all (one wave per step, node and instance tile) and
+// tvbx_step_sums advances the steps from them.  In one kernel each wave
+// carries its node's whole launch, gathers and updates one after the other;
+// with few (node, tile) pairs that serial chain is the time, and the chip is
+// mostly idle.  Split, the gathers spread over n_steps times the waves and
+// the chain that remains is the update.
+//   grid (8 Bx, n_steps): workgroup ids go to the 8 XCDs round robin, and
+// XCD x takes the x'th eighth of a step's (tile, node) pairs, tile outermost,
+// so that the rows of an instance tile share an L2; a step's workgroups are
+// dispatched together, and with rows sorted by delay the readers of one
+// (source, delay) meet there.
+//   Bound: many gathers with little reuse by HBM (Jansen-Rit N = 998, P =
+// 1024, float32: 5.8 TB/s); with 32 delay bins by the L2 and the issue of the
+// gathers (bfloat16, 256-byte rows: 17.9 us per step, 11.3 TB/s of gathered
+// bytes, against 23 us of the one-kernel launch's 27).
+#define TVBX_SUMS_WAVES 4
+extern "C" __global__ void __launch_bounds__(64 * TVBX_SUMS_WAVES)
+tvbx_sums(const tvbx_step_args a) {
+  const int lane = threadIdx.x & 63;
+  const unsigned N = (unsigned)a.n_node;
+  const unsigned M = (unsigned)(a.pitch / (64 * TVBX_IPL)) * N;
+  const unsigned Mx = (M + 7u) / 8u;
+  const unsigned it = (blockIdx.x >> 3) * TVBX_SUMS_WAVES + (threadIdx.x >> 6);
+  const unsigned id = (blockIdx.x & 7u) * Mx + it;
+  if (it >= Mx || id >= M) return;
+  const int bx = __builtin_amdgcn_readfirstlane((int)(id / N));
+  const int i = __builtin_amdgcn_readfirstlane((int)(id % N));
+  const int k = blockIdx.y;
+  const int pb = (bx * 64 + lane) * TVBX_IPL;
+  const int group = __builtin_amdgcn_readfirstlane(
+      (bx * 64 * TVBX_IPL) / a.group_size);
+  const unsigned *__restrict__ cd = a.coldelay + (size_t)group * a.nnz;
+  const float *__restrict__ wt = tvbx_group_weights(a, group);
+  long long n0;
+  int t;
+  tvbx_start(a, n0, t);
+  t += k;
+  t -= t >= a.horizon ? a.horizon : 0;
+  tvbx_lane_params lp[TVBX_IPL];
+#pragma unroll
+  for (int q = 0; q < TVBX_IPL; ++q) tvbx_load_lane(lp[q], a, pb + q);
+  tvbx_row rw;
+  tvbx_load_row(a, cd, wt, i, rw);
+  float c[TVBX_IPL][TVBX_C];
+  tvbx_coupling<true>(a, cd, wt, rw, (const tvbx_rt *)a.ring, nullptr, i, t,
+                      pb, k, lp, c);
+}
+#endif
+
+// the updates of a blocked launch whose sums are given
+extern "C" __global__ void __launch_bounds__(512)
+tvbx_step_sums(const tvbx_step_args a) {
+  int bx, by;
+  tvbx_block(a, bx, by);
+  const int i = __builtin_amdgcn_readfirstlane(by * a.node_block +
+                                               (int)(threadIdx.x >> 6));
+  if (i < a.n_node) tvbx_blocked_run<true>(a, bx, i);
+}
+
+// the blocked launch in one kernel
 extern "C" __global__ void __launch_bounds__(512, TVBX_MIN_WAVES)
 tvbx_step_blocked(const tvbx_step_args a) {
   int bx, by;
@@ -1355,7 +1494,7 @@ tvbx_step_blocked(const tvbx_step_args a) {
                                                (int)(threadIdx.x >> 6));
   if (a.pace == nullptr) {
     if (i >= a.n_node) return;
-    tvbx_blocked_run(a, bx, i);
+    tvbx_blocked_run<false>(a, bx, i);
     return;
   }
   // paced: every wave of the workgroup takes part in the waits, also one
@@ -1364,7 +1503,7 @@ tvbx_step_blocked(const tvbx_step_args a) {
   if (threadIdx.x == 0) pace_on = 1;
   __syncthreads();
   if (i < a.n_node) {
-    tvbx_blocked_run(a, bx, i, &pace_on);
+    tvbx_blocked_run<false>(a, bx, i, &pace_on);
   } else {
     for (int k = 0; k + 1 < a.n_steps; ++k) tvbx_pace(a, k, &pace_on);
   }
@@ -1388,7 +1527,7 @@ __device__ __forceinline__ void tvbx_batch_item(const tvbx_batch_args &B,
   a.clock = nullptr;
   const int i = node0 + (int)(threadIdx.x >> 6);
   if (i >= a.n_node || i >= node0 + a.node_block) return;
-  tvbx_blocked_run(a, tile, i);
+  tvbx_blocked_run<false>(a, tile, i);
 }
 
 // Without a queue workgroup w takes item w, and the hardware hands
@@ -1561,6 +1700,7 @@ tvbx_history_init(const tvbx_step_args a, int mode) {
   tvbx_rt *ring = (tvbx_rt *)a.ring;
   tvbx_lane_params lp;
   tvbx_load_lane(lp, a, p);
+  tvbx_load_node(lp, a, i, p);
   float x[TVBX_S], y[TVBX_NOBS];
 #pragma unroll
   for (int s = 0; s < TVBX_S; ++s) x[s] = a.state[s * NP + ip];

@@ -120,8 +120,8 @@ typedef struct tvbx_step_args {
    * chunk mfma_pairs holds the 32 packed pairs (delay << 16 | column) and
    * mfma_w the block's 16 x 32 weights as two MFMA A operands (high and low
    * part, 64 lanes x 8 elements each), scaled by 1 / mfma_unscale.
-   * csum [n_steps][C][N][pitch]: coupling sums of the launch's steps, which
-   * the blocked kernel reads instead of gathering when non-null. */
+   * csum [n_steps][C][N][pitch]: coupling accumulators of the launch's steps,
+   * written by tvbx_mfma_sums or tvbx_sums and read by tvbx_step_sums. */
   const int *mfma_blk;
   const unsigned *mfma_pairs;
   const unsigned short *mfma_w;

@@ -153,6 +153,8 @@ struct tvbx_module {
   hipFunction_t hist = nullptr;
   hipFunction_t adj = nullptr;  // present when emitted with the adjoint
   hipFunction_t blocked = nullptr;  // absent in the reference ordering
+  hipFunction_t step_sums = nullptr;  // blocked launch from given sums
+  hipFunction_t sums = nullptr;  // absent also where pre() reads post_syn
   hipFunction_t batch = nullptr;    // absent in the reference ordering
   hipFunction_t logp_grad = nullptr;  // present when emitted with the adjoint
   hipFunction_t mfma = nullptr;  // bfloat16 / float16 rings holding pre(y)
@@ -233,17 +235,54 @@ struct tvbx_sim {
   DevBuf mfma_blk, mfma_pairs, mfma_w, csum;
   float mfma_unscale = 1.0f;
   int mfma_chunks = 0;
+  // blocked launches as two kernels, the sums ahead of the updates
+  bool ahead = false;
 };
 
 // steps per launch of tvbx_mfma_sums (its accumulators: steps x ipl tiles)
 #define TVBX_MFMA_LMAX(ipl) ((ipl) == 4 ? 8 : 16)
 static int mfma_tables(tvbx_sim *s);
 
-// the forward step kernel of the simulation's launch shape
-static hipFunction_t step_fn(const tvbx_sim *s) {
-  const bool blocked =
-      s->d.steps_per_launch > 1 && s->d.node_block < s->d.n_node;
-  return blocked ? s->mod->blocked : s->mod->step;
+static bool is_blocked(const tvbx_sim_desc &d) {
+  return d.steps_per_launch > 1 && d.node_block < d.n_node;
+}
+
+// How often a history value is gathered in a step: edges per distinct
+// (delay, source), of the first delay group (1 when there are too many
+// (delay, source) pairs to count).
+static double gather_reuse(const tvbx_sim_desc &d, const unsigned *cd) {
+  const size_t bits = (size_t)d.horizon * d.n_node;
+  if (d.nnz == 0 || bits > (1ull << 28)) return 1.0;
+  std::vector<bool> seen(bits, false);
+  size_t distinct = 0;
+  for (int e = 0; e < d.nnz; ++e) {
+    const size_t b = (size_t)(cd[e] >> 16) * d.n_node + (cd[e] & 0xffffu);
+    distinct += !seen[b];
+    seen[b] = true;
+  }
+  return (double)d.nnz / (double)distinct;
+}
+
+// Whether a blocked launch runs as two kernels, all its coupling sums ahead
+// of its updates (tvbx_sums, tvbx_step_sums), or as one.  Two kernels win
+// where one would leave the chip idle, and where a history value is gathered
+// several times in a step and the sums' step-by-step order lets the L2 serve
+// the repeats; else the sums' round trip through memory costs more.
+// Measured, us per step, one kernel against two:
+//   few waves: MPR N = 84, P = 64 (84 waves) 2.59 / 1.09, P = 1024 (1344)
+//   5.45 / 2.24, P = 2048 (2688) 3.69 / 3.70, P = 4096 (5376) 7.21 / 7.27;
+//   two-dimensional oscillator, 12 edges a row, 2100 waves 2.04 / 1.78, 4200
+//   waves 2.78 / 3.31; Jansen-Rit N = 379 8-bit, 1137 waves 4.50 / 2.58;
+//   reuse (N = 998, P = 1024): 4.2 edges per value (32 bins) float32 66.4 /
+//   36.3, 16 bits 28.1 / 21.8 (P = 4096: 148 / 87), 8 bits 13.84 / 13.58;
+//   1.4 (128 bins) float32 73.4 / 59.1, 16 bits 35.2 / 32.7, 8 bits 16.6 /
+//   18.8; 1.06 (exact delays) 16 bits 36.4 / 40.0, 8 bits 17.6 / 20.7.
+static bool sums_ahead(const tvbx_sim *s, const unsigned *cd) {
+  const tvbx_sim_desc &d = s->d;
+  if (!is_blocked(d) || !s->mod->sums || !s->mod->step_sums) return false;
+  const long long waves = (long long)(s->pitch / (64 * d.ipl)) * d.n_node;
+  return waves < 2400 ||
+         gather_reuse(d, cd) >= (d.ring_type == 3 ? 2.0 : 1.25);
 }
 
 // advance the device clock by w steps (last node of a captured window)
@@ -382,6 +421,11 @@ static int module_from_image(tvbx_ctx *c, const void *image, size_t size,
   if (hipModuleGetFunction(&m->blocked, m->mod, "tvbx_step_blocked") !=
       hipSuccess)
     m->blocked = nullptr;
+  if (hipModuleGetFunction(&m->step_sums, m->mod, "tvbx_step_sums") !=
+      hipSuccess)
+    m->step_sums = nullptr;
+  if (hipModuleGetFunction(&m->sums, m->mod, "tvbx_sums") != hipSuccess)
+    m->sums = nullptr;
   if (hipModuleGetFunction(&m->batch, m->mod, "tvbx_step_batch") !=
       hipSuccess)
     m->batch = nullptr;
@@ -925,13 +969,13 @@ static void fill_args(tvbx_sim *s, tvbx_step_args &a) {
     a.mfma_pairs = (const unsigned *)s->mfma_pairs.p;
     a.mfma_w = (const unsigned short *)s->mfma_w.p;
     a.mfma_unscale = s->mfma_unscale;
-    a.csum = (float *)s->csum.p;
   }
+  if (s->mfma || (s->ahead && !s->pace)) a.csum = (float *)s->csum.p;
 }
 
 // One forward launch of a.n_steps steps: the step kernel of the launch
-// shape, or with the matrix-core coupling the sums kernel and then the
-// blocked kernel reading its sums.
+// shape, or the kernel that forms the launch's sums (by gathers, or on the
+// matrix cores) and then the blocked updates from them.
 static hipError_t launch_steps(tvbx_sim *s, tvbx_step_args &a,
                                hipStream_t st) {
   const tvbx_sim_desc &d = s->d;
@@ -939,15 +983,19 @@ static hipError_t launch_steps(tvbx_sim *s, tvbx_step_args &a,
   const unsigned gy = (d.n_node + d.node_block - 1) / d.node_block;
   const unsigned bx = 64u * d.waves;
   void *params[] = {&a};
-  if (s->mfma) {
-    hipError_t e = hipModuleLaunchKernel(
-        s->mod->mfma, (d.n_node + 15) / 16, s->pitch / (64 * d.ipl), 1, 256,
-        1, 1, 0, st, params, nullptr);
+  hipFunction_t fn = is_blocked(d) ? s->mod->blocked : s->mod->step;
+  if (a.csum) {
+    const unsigned pairs = gx * (unsigned)d.n_node, per = (pairs + 7) / 8;
+    const hipError_t e =
+        s->mfma ? hipModuleLaunchKernel(s->mod->mfma, (d.n_node + 15) / 16, gx,
+                                        1, 256, 1, 1, 0, st, params, nullptr)
+                : hipModuleLaunchKernel(
+                      s->mod->sums, 8 * ((per + 3) / 4), (unsigned)a.n_steps, 1,
+                      256, 1, 1, 0, st, params, nullptr);
     if (e != hipSuccess) return e;
-    return hipModuleLaunchKernel(s->mod->blocked, gx, gy, 1, bx, 1, 1, 0, st,
-                                 params, nullptr);
+    fn = s->mod->step_sums;
   }
-  return hipModuleLaunchKernel(step_fn(s), gx, gy, 1, bx, 1, 1, 0, st, params,
+  return hipModuleLaunchKernel(fn, gx, gy, 1, bx, 1, 1, 0, st, params,
                                nullptr);
 }
 
@@ -1180,6 +1228,12 @@ extern "C" int tvbx_sim_set_connectome(tvbx_sim *s, const int32_t *row,
   s->h_w.assign(weight, weight + nw);
   s->h_delays.assign(delays, delays + (size_t)d.n_group * d.nnz);
   dfree(s->ccol);
+  const bool ahead = sums_ahead(s, cd.data());
+  if (ahead != s->ahead) drop_graphs(s);
+  // without memory for the sums the launches stay one kernel
+  s->ahead = ahead && dalloc(s->csum, (size_t)d.steps_per_launch *
+                                          d.n_coupled * s->NP * 4) == TVBX_OK;
+  if (ahead && !s->ahead) (void)hipGetLastError();
   if (s->mfma) return mfma_tables(s);
   return TVBX_OK;
 }
@@ -3027,9 +3081,7 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
       a.rec_x = rec_x_of(kw);
       a.rec_sum = rec_sum_of(kw);
       a.rec_step0 = n_lo;
-      void *params[] = {&a};
-      HIPCHK(hipModuleLaunchKernel(step_fn(s), gx, gy, 1, bx, 1, 1, 0, sb,
-                                   params, nullptr));
+      HIPCHK(launch_steps(s, a, sb));
     }
     if (overlap) HIPCHK(hipEventRecord(ev_rep(kw), sb));
     return TVBX_OK;

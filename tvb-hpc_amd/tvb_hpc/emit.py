@@ -216,7 +216,7 @@ class KernelSpec:
         out = []
         for key in sorted(self.kinds) + (['sigma'] if self.sigma_kind else []):
             kind, idx = self.slot(key)
-            if kind in ('inst', 'glob'):
+            if kind != 'const':
                 out.append((key, kind, idx))
         return out
 
@@ -233,9 +233,7 @@ class KernelSpec:
         if not in_node_scope:
             raise ValueError('%s (kind %s) used outside node scope'
                              % (key, kind))
-        if kind == 'node':
-            return 'a.p_node[%d * a.n_node + i]' % idx
-        return 'a.p_ni[((size_t)%d * a.n_node + i) * a.pitch + p]' % idx
+        return 'lp.' + self.cname(key)
 
     # -- emission ----------------------------------------------------------------
 
@@ -286,6 +284,7 @@ class KernelSpec:
             lines.append('#define TVBX_PIPE 1')
         lines.append('#define TVBX_PRIO %d' % int(self.prio))
         lines.append('#define TVBX_EMAJ %d' % self.emaj)
+        lines.append('#define TVBX_ADJOINT %d' % int(self.adjoint))
         # lane parameters
         fields = self._lane_fields()
         lines.append('struct tvbx_lane_params {')
@@ -296,12 +295,20 @@ class KernelSpec:
         lines.append('};')
         lines.append('__device__ __forceinline__ void tvbx_load_lane('
                      'tvbx_lane_params &lp, const tvbx_step_args &a, int p) {')
-        for key, kind, idx in fields:
-            src = ('a.p_inst[(size_t)%d * a.param_pitch + a.inst_off + p]'
-                   % idx if kind == 'inst'
-                   else 'a.p_glob[%d]' % idx)
-            lines.append('  lp.%s = %s;' % (self.cname(key), src))
-        lines.append('}')
+        srcs = {'inst': 'a.p_inst[(size_t)%d * a.param_pitch + a.inst_off + p]',
+                'glob': 'a.p_glob[%d]',
+                'node': 'a.p_node[%d * a.n_node + i]',
+                'ni': 'a.p_ni[((size_t)%d * a.n_node + i) * a.pitch + p]'}
+
+        def loads(kinds):
+            return ['  lp.%s = %s;' % (self.cname(key), srcs[kind] % idx)
+                    for key, kind, idx in fields if kind in kinds]
+
+        lines += loads(('inst', 'glob')) + ['}']
+        lines.append('__device__ __forceinline__ void tvbx_load_node('
+                     'tvbx_lane_params &lp, const tvbx_step_args &a, int i, '
+                     'int p) {')
+        lines += loads(('node', 'ni')) + ['}']
         # coupling: pre / post
         cn = self._cfun_names()
         pre_c, post_c, ringv, pre_nb = [], [], [], []

@@ -106,13 +106,49 @@ def block_lengths(cfg):
     return sorted({min(lmax, b) for b in (8, 16, 32, 64)} - {1})
 
 
+def gather_reuse(csr):
+    "Edges per distinct (delay, source) of the first delay group."
+    if csr.nnz == 0:
+        return 1.0
+    pairs = csr.delays[0].astype(np.int64) * csr.nnode + csr.col
+    return csr.nnz / float(np.unique(pairs).size)
+
+
+def default_ipl(cfg):
+    """Instances per lane of blocked launches with no measured entry.
+
+    Wide lanes need fewer instructions per byte; narrow ones give more waves,
+    and where a history value is gathered several times in a step they keep
+    the rows that an XCD reads at a time small enough for its L2 (256-byte
+    rows won: us per step at N = 998, P = 1024, 32 delay bins, 1 / 2 / 4
+    instances per lane: float32 36.3 / 42.5 / 49.5, bfloat16 28.0 / 21.8 /
+    23.7, 8 bits 27.8 / 16.5 / 13.6).  Without reuse 2 lanes' worth of
+    float32 and 4 of the narrower types suffice.  Below that, the widest with
+    enough waves (float32: MPR N = 84, P = 2048 3.7 at 2,688 waves against
+    4.2 and 5.1 at 1,344 and 672; P = 4096 6.8 at 2,688, 7.2 at 5,376, 8.4
+    at 1,344; 8 bits: N = 379, P = 300 2.56 at 1,137 waves, 2.77 at 1,895
+    narrower ones, N = 150, P = 512 1.61 at 1,200, 1.78 at 600)."""
+    narrow = cfg.ring_dtype != 'f32'
+    if gather_reuse(cfg.csr) >= 1.25:
+        widest = {'f32': 1, 'u8': 4}.get(cfg.ring_dtype, 2)
+    else:
+        widest = 4 if narrow else 2
+    enough = 1100 if narrow else 2400
+    for ipl in sorted(valid_ipls(cfg), reverse=True):
+        waves = cfg.csr.nnode * -(-cfg.n_inst // (64 * ipl))
+        if ipl <= widest and waves >= enough:
+            return ipl
+    return min(valid_ipls(cfg))
+
+
 def default_launch(cfg):
     """Defaults for a configuration with no measured entry, after what won
-    for the built-in ones: the widest ipl the instance count allows; when the
-    smallest delay allows blocks of 8 steps or more, one node per wave in
+    for the built-in ones: when the smallest delay allows blocks of 8 steps
+    or more, ``default_ipl`` instances per lane and one node per wave in
     blocks of up to 32 steps with the 4-waves-per-SIMD register budget (16
     gathers per group from 2 instances per lane, 8 pipelined below), else
-    per-step launches with 4-node workgroups."""
+    per-step launches with 4-node workgroups and the widest ipl the instance
+    count allows."""
     ipls = valid_ipls(cfg)
     ipl = 4 if 4 in ipls and cfg.n_inst >= 1024 else max(
         [i for i in ipls if i <= 2] or [1])
@@ -123,6 +159,7 @@ def default_launch(cfg):
         return dict(ipl=ipl, waves=4, node_block=4,
                     steps_per_launch=min(max(bl or [1]), mfma_steps(ipl)))
     if bl and max(bl) >= 8:
+        ipl = default_ipl(cfg)
         la = dict(ipl=ipl, waves=1, node_block=1,
                   steps_per_launch=min(max(bl), 32), min_waves=4)
         la.update(dict(unroll=16) if ipl >= 2 else dict(unroll=8, pipe=True))

@@ -88,3 +88,39 @@ def test_sums_ahead_where_values_are_reused():
         sim.run(20)
         got.append(sim.get_state())
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize('N,deg,P,groups,ipl,L,window', [
+    (2, 1, 1, 1, 1, 2, 10),
+    (9, 5, 65, 1, 1, 7, 20),
+    (140, 139, 70, 1, 2, 4, 30),
+    (31, 12, 192, 3, 1, 6, 15),
+    (33, 20, 300, 1, 4, 7, 60)])
+def test_reverse_sums_ahead_equal_single_steps(N, deg, P, groups, ipl, L,
+                                               window):
+    """The adjoint of blocked launches (transposed gathers ahead of the
+    recursion) against one reverse step per launch, bit for bit."""
+    csr = _csr(N, deg, groups)
+    m = M.MontbrioPazoRoxin()
+    rng = np.random.default_rng(2)
+    x0 = m.initial_state(N, P, rng)
+    par = {'c:a': rng.uniform(0, 0.1, P).astype(np.float32),
+           'm:eta': -5 + rng.uniform(-.2, .2, (N, P)).astype(np.float32)}
+    ds = rng.standard_normal((12, N, P)).astype(np.float32)
+    gs = None if groups == 1 else P // groups
+    got = []
+    for la in (dict(ipl=ipl, waves=2, node_block=2, steps_per_launch=1),
+               dict(ipl=ipl, waves=1, node_block=1, steps_per_launch=L)):
+        sim = Simulation(m, CF.Linear(m), SC.EulerMaryuyamaStep(0.01, 0.01),
+                         csr, P, params=par,
+                         kinds={'c:a': 'inst', 'm:eta': 'ni'}, horizon=60,
+                         group_size=gs, tavg_period=5, sample_slots=12,
+                         adjoint=True, **la)
+        sim.set_state(x0)
+        sim.init_history('zeros')
+        sim.set_noise(seed=4)
+        sim.checkpoint_run(60, window)
+        got.append(sim.adjoint(ds, 0))
+    for key in ('c:a', 'm:eta'):
+        assert np.isfinite(got[0][key]).all() and np.any(got[0][key])
+        assert np.array_equal(got[0][key], got[1][key])

@@ -49,6 +49,147 @@ __device__ __forceinline__ void tvbx_bloadf(__amdgpu_buffer_rsrc_t r,
 #endif
 }
 
+// The transposed gather: the sum over the edges leaving node j (CSC row crw)
+// of w mu(n + d) of their targets, step n at slot t, in CSC order with the
+// indices read back from the row's registers.
+__device__ __forceinline__ void tvbx_adj_gather(
+    const tvbx_step_args &a, const float *__restrict__ mu_r,
+    const unsigned *__restrict__ crow, const float *__restrict__ cw,
+    const tvbx_row &crw, bool mu32, __amdgpu_buffer_rsrc_t mrs, int t, int pb,
+    float (&accm)[TVBX_IPL]) {
+  const int lane = threadIdx.x & 63;
+  const int N = a.n_node, H = a.horizon;
+  const unsigned lane_off = (unsigned)pb * 4u;
+  const unsigned rowb = (unsigned)a.pitch * 4u;
+#pragma unroll
+  for (int q = 0; q < TVBX_IPL; ++q) accm[q] = 0.0f;
+  const int deg = crw.e1 - crw.e0;
+#define TVBX_ADJ_SRC(C)                                                       \
+  reinterpret_cast<const float *>(                                            \
+  reinterpret_cast<const char *>(                                         \
+      mu_r + ((size_t)(t + (int)((C) >> 16) -                             \
+                       ((t + (int)((C) >> 16)) >= H ? H : 0)) * N +       \
+              ((C) & 0xffffu)) * a.pitch) +                               \
+  tvbx_lane_offset(lane_off))
+// the same with buffer loads at the byte offsets OV (read back per edge)
+#define TVBX_ADJ_BRANGE(NE, OV, WV)                                           \
+  {                                                                           \
+    int u0 = 0;                                                               \
+    for (; u0 + TVBX_ADJ_UNROLL <= (NE); u0 += TVBX_ADJ_UNROLL) {             \
+  unsigned so[TVBX_ADJ_UNROLL];                                           \
+  float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
+      tvbx_lane_u((OV), u0 + u);                                          \
+  __builtin_amdgcn_sched_barrier(0);                                      \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
+      tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
+  __builtin_amdgcn_sched_barrier(0);                                      \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+    const float we = tvbx_lane_f((WV), u0 + u);                           \
+    _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
+        fmaf(we, v[u][q], accm[q]);                                       \
+  }                                                                       \
+    }                                                                         \
+    if (u0 < (NE)) {                                                          \
+  /* the remainder as one group: a slot past the row reads the row's */   \
+  /* last edge again, with the weight 0 its lane holds (adds nothing) */  \
+  unsigned so[TVBX_ADJ_UNROLL];                                           \
+  float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
+      tvbx_lane_u((OV), min(u0 + u, (NE) - 1));                           \
+  __builtin_amdgcn_sched_barrier(0);                                      \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
+      tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
+  __builtin_amdgcn_sched_barrier(0);                                      \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+    const float we = tvbx_lane_f((WV), u0 + u);                           \
+    _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
+        fmaf(we, v[u][q], accm[q]);                                       \
+  }                                                                       \
+    }                                                                         \
+  }
+// TVBX_ADJ_UNROLL gathers in flight, accumulated in CSC order
+#define TVBX_ADJ_RANGE(NE, CV, WV)                                            \
+  {                                                                           \
+    int u0 = 0;                                                               \
+    for (; u0 + TVBX_ADJ_UNROLL <= (NE); u0 += TVBX_ADJ_UNROLL) {             \
+  float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+    const unsigned c = tvbx_lane_u((CV), u0 + u);                         \
+    tvbx_ldf(TVBX_ADJ_SRC(c), v[u]);                                      \
+  }                                                                       \
+  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+    const float we = tvbx_lane_f((WV), u0 + u);                           \
+    _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
+        fmaf(we, v[u][q], accm[q]);                                       \
+  }                                                                       \
+    }                                                                         \
+    for (; u0 < (NE); ++u0) {                                                 \
+  const unsigned c = tvbx_lane_u((CV), u0);                               \
+  float v[TVBX_IPL];                                                      \
+  tvbx_ldf(TVBX_ADJ_SRC(c), v);                                           \
+  const float we = tvbx_lane_f((WV), u0);                                 \
+  _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =          \
+      fmaf(we, v[q], accm[q]);                                            \
+    }                                                                         \
+  }
+  if (mu32) {
+    // byte offsets of mu(n + d) of the row's targets, this step
+    const unsigned o0 = tvbx_mu_row(crw.cd0, t, H, N) * rowb;
+    const unsigned o1 = tvbx_mu_row(crw.cd1, t, H, N) * rowb;
+    const int n0 = min(deg, 64);
+    TVBX_ADJ_BRANGE(n0, o0, crw.w0)
+    const int n1 = min(max(deg - 64, 0), 64);
+    if (n1 > 0) TVBX_ADJ_BRANGE(n1, o1, crw.w1)
+  } else {
+    const int n0 = min(deg, 64);
+    TVBX_ADJ_RANGE(n0, crw.cd0, crw.w0)
+    const int n1 = min(max(deg - 64, 0), 64);
+    if (n1 > 0) TVBX_ADJ_RANGE(n1, crw.cd1, crw.w1)
+  }
+  // rows longer than 128 edges: the rest in chunks of 64 edges, one
+  // edge per lane, gathered in groups like the first 128
+  for (int cb = 128; cb < deg; cb += 64) {
+    const int nc = __builtin_amdgcn_readfirstlane(min(deg - cb, 64));
+    const int ec = crw.e0 + cb + lane;
+    const unsigned cdc = lane < nc ? crow[ec] : 0u;
+    const float wc = lane < nc ? cw[ec] : 0.0f;
+    if (mu32) {
+      const unsigned oc = tvbx_mu_row(cdc, t, H, N) * rowb;
+      TVBX_ADJ_BRANGE(nc, oc, wc)
+    } else {
+      TVBX_ADJ_RANGE(nc, cdc, wc)
+    }
+  }
+#undef TVBX_ADJ_RANGE
+#undef TVBX_ADJ_BRANGE
+#undef TVBX_ADJ_SRC
+}
+
+// One reverse step of (node j, instance p) from x(n), lambda(n + 1), the
+// forward sum, the gathered accm and the forcing fj: lambda(n) into ln, the
+// parameter partials into gc and gm; returns mu(n).
+__device__ __forceinline__ float tvbx_adj_node(
+    const tvbx_step_args &a, int j, int p, const tvbx_lane_params &lp,
+    const float (&x)[TVBX_S], const float (&lam)[TVBX_S], float sum,
+    float accm, float fj, float (&ln)[TVBX_S], float (&gc)[TVBX_NGC],
+    float (&gm)[TVBX_NGM]) {
+  float cc[TVBX_C], jt[TVBX_S], muc[TVBX_C], y[TVBX_NOBS], dhc[TVBX_S],
+      dhm[TVBX_S];
+  cc[0] = tvbx_post(0, sum, lp, a);
+  tvbx_dfun_vjp(x, cc, lam, jt, muc, gm, lp, a, j, p);
+  const float mu = a.dt * muc[0];
+  tvbx_obsrv(x, y, lp, a, j, p);
+  const float aj = tvbx_dpost_dsum(lp, a) * tvbx_dpre(y[0], lp, a) * accm;
+  tvbx_dobsrv(0, x, dhc, lp, a, j, p);
+  tvbx_dobsrv(a.bold_obs, x, dhm, lp, a, j, p);
+#pragma unroll
+  for (int s = 0; s < TVBX_S; ++s)
+    ln[s] = lam[s] + a.dt * jt[s] + aj * dhc[s] + fj * dhm[s];
+  tvbx_dpost_dparam(sum, gc, lp, a);
+  return mu;
+}
+
 // 32 gathers in flight need more than the 128 registers a 1024-thread
 // workgroup leaves each lane: such modules take at most 8 waves per
 // workgroup (the runtime checks the launch against this bound)
@@ -87,12 +228,10 @@ tvbx_adjoint(const tvbx_adj_args A) {
   tvbx_row crw;
   if (one_node && i_begin + wave < i_end)
     tvbx_load_row_of(ccol, crow, cw, i_begin + wave, crw);
-  const unsigned lane_off = (unsigned)pb * 4u;
   // a mu ring under 4 GiB is read through a buffer descriptor with 32-bit
   // byte offsets computed once per step for the row's first 128 edges
   const bool mu32 = (unsigned long long)H * NP * 4ull < 4294967296ull;
   const __amdgpu_buffer_rsrc_t mrs = tvbx_ring_rsrc(mu_r);
-  const unsigned rowb = (unsigned)a.pitch * 4u;
 
   // with one node per wave, lambda and the parameter partials of that node
   // stay in registers for the whole launch (the same additions, in the same
@@ -169,112 +308,8 @@ tvbx_adjoint(const tvbx_adj_args A) {
           for (int q = 0; q < TVBX_IPL; ++q) fo[q] = 0.0f;
         }
       }
-      // mu of the targets of j's outgoing edges at steps n + d: edges in
-      // CSC order, indices read back from the row's registers
       float accm[TVBX_IPL];
-#pragma unroll
-      for (int q = 0; q < TVBX_IPL; ++q) accm[q] = 0.0f;
-      const int deg = crw.e1 - crw.e0;
-#define TVBX_ADJ_SRC(C)                                                       \
-  reinterpret_cast<const float *>(                                            \
-      reinterpret_cast<const char *>(                                         \
-          mu_r + ((size_t)(t + (int)((C) >> 16) -                             \
-                           ((t + (int)((C) >> 16)) >= H ? H : 0)) * N +       \
-                  ((C) & 0xffffu)) * a.pitch) +                               \
-      tvbx_lane_offset(lane_off))
-// the same with buffer loads at the byte offsets OV (read back per edge)
-#define TVBX_ADJ_BRANGE(NE, OV, WV)                                           \
-  {                                                                           \
-    int u0 = 0;                                                               \
-    for (; u0 + TVBX_ADJ_UNROLL <= (NE); u0 += TVBX_ADJ_UNROLL) {             \
-      unsigned so[TVBX_ADJ_UNROLL];                                           \
-      float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
-          tvbx_lane_u((OV), u0 + u);                                          \
-      __builtin_amdgcn_sched_barrier(0);                                      \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
-          tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
-      __builtin_amdgcn_sched_barrier(0);                                      \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-        const float we = tvbx_lane_f((WV), u0 + u);                           \
-        _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
-            fmaf(we, v[u][q], accm[q]);                                       \
-      }                                                                       \
-    }                                                                         \
-    if (u0 < (NE)) {                                                          \
-      /* the remainder as one group: a slot past the row reads the row's */   \
-      /* last edge again, with the weight 0 its lane holds (adds nothing) */  \
-      unsigned so[TVBX_ADJ_UNROLL];                                           \
-      float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
-          tvbx_lane_u((OV), min(u0 + u, (NE) - 1));                           \
-      __builtin_amdgcn_sched_barrier(0);                                      \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
-          tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
-      __builtin_amdgcn_sched_barrier(0);                                      \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-        const float we = tvbx_lane_f((WV), u0 + u);                           \
-        _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
-            fmaf(we, v[u][q], accm[q]);                                       \
-      }                                                                       \
-    }                                                                         \
-  }
-// TVBX_ADJ_UNROLL gathers in flight, accumulated in CSC order
-#define TVBX_ADJ_RANGE(NE, CV, WV)                                            \
-  {                                                                           \
-    int u0 = 0;                                                               \
-    for (; u0 + TVBX_ADJ_UNROLL <= (NE); u0 += TVBX_ADJ_UNROLL) {             \
-      float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-        const unsigned c = tvbx_lane_u((CV), u0 + u);                         \
-        tvbx_ldf(TVBX_ADJ_SRC(c), v[u]);                                      \
-      }                                                                       \
-      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-        const float we = tvbx_lane_f((WV), u0 + u);                           \
-        _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
-            fmaf(we, v[u][q], accm[q]);                                       \
-      }                                                                       \
-    }                                                                         \
-    for (; u0 < (NE); ++u0) {                                                 \
-      const unsigned c = tvbx_lane_u((CV), u0);                               \
-      float v[TVBX_IPL];                                                      \
-      tvbx_ldf(TVBX_ADJ_SRC(c), v);                                           \
-      const float we = tvbx_lane_f((WV), u0);                                 \
-      _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =          \
-          fmaf(we, v[q], accm[q]);                                            \
-    }                                                                         \
-  }
-      if (mu32) {
-        // byte offsets of mu(n + d) of the row's targets, this step
-        const unsigned o0 = tvbx_mu_row(crw.cd0, t, H, N) * rowb;
-        const unsigned o1 = tvbx_mu_row(crw.cd1, t, H, N) * rowb;
-        const int n0 = min(deg, 64);
-        TVBX_ADJ_BRANGE(n0, o0, crw.w0)
-        const int n1 = min(max(deg - 64, 0), 64);
-        if (n1 > 0) TVBX_ADJ_BRANGE(n1, o1, crw.w1)
-      } else {
-        const int n0 = min(deg, 64);
-        TVBX_ADJ_RANGE(n0, crw.cd0, crw.w0)
-        const int n1 = min(max(deg - 64, 0), 64);
-        if (n1 > 0) TVBX_ADJ_RANGE(n1, crw.cd1, crw.w1)
-      }
-      // rows longer than 128 edges: the rest in chunks of 64 edges, one
-      // edge per lane, gathered in groups like the first 128
-      for (int cb = 128; cb < deg; cb += 64) {
-        const int nc = __builtin_amdgcn_readfirstlane(min(deg - cb, 64));
-        const int ec = crw.e0 + cb + lane;
-        const unsigned cdc = lane < nc ? crow[ec] : 0u;
-        const float wc = lane < nc ? cw[ec] : 0.0f;
-        if (mu32) {
-          const unsigned oc = tvbx_mu_row(cdc, t, H, N) * rowb;
-          TVBX_ADJ_BRANGE(nc, oc, wc)
-        } else {
-          TVBX_ADJ_RANGE(nc, cdc, wc)
-        }
-      }
-#undef TVBX_ADJ_RANGE
-#undef TVBX_ADJ_BRANGE
-#undef TVBX_ADJ_SRC
+      tvbx_adj_gather(a, mu_r, crow, cw, crw, mu32, mrs, t, pb, accm);
       if (keep) {
 #pragma unroll
         for (int s = 0; s < TVBX_S; ++s)
@@ -285,28 +320,17 @@ tvbx_adjoint(const tvbx_adj_args A) {
 #pragma unroll
       for (int q = 0; q < TVBX_IPL; ++q) {
         const int p = pb + q;
-        float x[TVBX_S], lam[TVBX_S], cc[TVBX_C], jt[TVBX_S], muc[TVBX_C],
-            gm[TVBX_NGM], gc[TVBX_NGC], y[TVBX_NOBS], dhc[TVBX_S],
-            dhm[TVBX_S];
+        float x[TVBX_S], lam[TVBX_S], ln[TVBX_S], gm[TVBX_NGM], gc[TVBX_NGC];
 #pragma unroll
         for (int s = 0; s < TVBX_S; ++s) {
           x[s] = xs[s][q];
           lam[s] = ls[s][q];
         }
-        cc[0] = tvbx_post(0, sm[q], lp[q], a);
-        tvbx_dfun_vjp(x, cc, lam, jt, muc, gm, lp[q], a, j, p);
-        const float mu = a.dt * muc[0];
-        tvbx_obsrv(x, y, lp[q], a, j, p);
-        const float aj =
-            tvbx_dpost_dsum(lp[q], a) * tvbx_dpre(y[0], lp[q], a) * accm[q];
-        const float fj = fo[q] * rK;
-        tvbx_dobsrv(0, x, dhc, lp[q], a, j, p);
-        tvbx_dobsrv(a.bold_obs, x, dhm, lp[q], a, j, p);
+        const float mu = tvbx_adj_node(a, j, p, lp[q], x, lam, sm[q], accm[q],
+                                       fo[q] * rK, ln, gc, gm);
 #pragma unroll
-        for (int s = 0; s < TVBX_S; ++s)
-          lo[s][q] = lam[s] + a.dt * jt[s] + aj * dhc[s] + fj * dhm[s];
+        for (int s = 0; s < TVBX_S; ++s) lo[s][q] = ln[s];
         mu_o[q] = mu;
-        tvbx_dpost_dparam(sm[q], gc, lp[q], a);
 #if TVBX_HAS_NGC
 #pragma unroll
         for (int g = 0; g < TVBX_NGC; ++g) {
@@ -356,6 +380,155 @@ tvbx_adjoint(const tvbx_adj_args A) {
     for (int g = 0; g < TVBX_NGM; ++g) tvbx_stf(A.g_m + g * NP + jp, gmr[g]);
 #endif
   }
+}
+
+// A blocked reverse launch as two kernels, as the forward ones (tvbx_sums):
+// step n reads mu(n + d), written before a launch of at most d_min steps, so
+// the transposed gathers of all its steps can be formed ahead of the
+// recursion, one wave per step, source node and instance tile, into
+// msum [n_steps][N][pitch] (step index counted down from step0).
+// grid (8 Bx, n_steps): as tvbx_sums.
+extern "C" __global__ void __launch_bounds__(64 * TVBX_SUMS_WAVES)
+tvbx_adj_sums(const tvbx_adj_args A) {
+  const tvbx_step_args &a = A.f;
+  const int lane = threadIdx.x & 63;
+  const unsigned N = (unsigned)a.n_node;
+  const unsigned M = (unsigned)(a.pitch / (64 * TVBX_IPL)) * N;
+  const unsigned Mx = (M + 7u) / 8u;
+  const unsigned it = (blockIdx.x >> 3) * TVBX_SUMS_WAVES + (threadIdx.x >> 6);
+  const unsigned id = (blockIdx.x & 7u) * Mx + it;
+  if (it >= Mx || id >= M) return;
+  const int bx = __builtin_amdgcn_readfirstlane((int)(id / N));
+  const int j = __builtin_amdgcn_readfirstlane((int)(id % N));
+  const int k = blockIdx.y;
+  const int pb = (bx * 64 + lane) * TVBX_IPL;
+  const int group = __builtin_amdgcn_readfirstlane(
+      (bx * 64 * TVBX_IPL) / a.group_size);
+  const unsigned *__restrict__ crow = A.crow + (size_t)group * a.nnz;
+  const float *__restrict__ cw =
+      A.cw + (a.weight_groups ? (size_t)group * a.nnz : 0);
+  const size_t NP = (size_t)N * a.pitch;
+  tvbx_row crw;
+  tvbx_load_row_of(A.ccol, crow, cw, j, crw);
+  const bool mu32 = (unsigned long long)a.horizon * NP * 4ull < 4294967296ull;
+  float accm[TVBX_IPL];
+  tvbx_adj_gather(a, A.mu, crow, cw, crw, mu32, tvbx_ring_rsrc(A.mu),
+                  (int)((a.step0 - k) % a.horizon), pb, accm);
+  tvbx_stf(A.msum + (size_t)k * NP + (size_t)j * a.pitch + pb, accm);
+}
+
+// the recursion of a blocked reverse launch from its gathers: one node per
+// wave, lambda and the partials in registers, the next step's records,
+// gather and forcing loaded while the current one is computed
+extern "C" __global__ void __launch_bounds__(512)
+tvbx_adjoint_sums(const tvbx_adj_args A) {
+  const tvbx_step_args &a = A.f;
+  const int j = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.y * a.node_block + (threadIdx.x >> 6)));
+  if (j >= a.n_node) return;
+  const int pb = (int)(blockIdx.x * 64 + (threadIdx.x & 63)) * TVBX_IPL;
+  const int H = a.horizon;
+  const size_t NP = (size_t)a.n_node * a.pitch;
+  const size_t jp = (size_t)j * a.pitch + pb;
+  const float rK = a.tavg_period > 0 ? 1.0f / (float)a.tavg_period : 0.0f;
+  tvbx_lane_params lp[TVBX_IPL];
+#pragma unroll
+  for (int q = 0; q < TVBX_IPL; ++q) {
+    tvbx_load_lane(lp[q], a, pb + q);
+    tvbx_load_node(lp[q], a, j, pb + q);
+  }
+  float lr[TVBX_S][TVBX_IPL], gcr[TVBX_NGC][TVBX_IPL], gmr[TVBX_NGM][TVBX_IPL];
+#pragma unroll
+  for (int s = 0; s < TVBX_S; ++s) tvbx_ldf(A.lam + s * NP + jp, lr[s]);
+#if TVBX_HAS_NGC
+#pragma unroll
+  for (int g = 0; g < TVBX_NGC; ++g) tvbx_ldf(A.g_c + g * NP + jp, gcr[g]);
+#endif
+#if TVBX_HAS_NGM
+#pragma unroll
+  for (int g = 0; g < TVBX_NGM; ++g) tvbx_ldf(A.g_m + g * NP + jp, gmr[g]);
+#endif
+  int t = (int)(a.step0 % H);
+  // sample of step n (n div T) and the steps into it, counted down
+  long long mq = 0;
+  int mr = 0;
+  if (a.tavg_period > 0) {
+    mq = a.step0 / a.tavg_period;
+    mr = (int)(a.step0 - mq * a.tavg_period);
+  }
+  // the inputs of the launch's step k
+  float xs[TVBX_S][TVBX_IPL], sm[TVBX_IPL], am[TVBX_IPL], fo[TVBX_IPL];
+  auto fetch = [&](int k, long long m) {
+    const size_t w = (size_t)(a.step0 - k - a.rec_step0);
+#pragma unroll
+    for (int s = 0; s < TVBX_S; ++s)
+      tvbx_ldf(A.rec_x + (w * TVBX_S + s) * NP + jp, xs[s]);
+    tvbx_ldf(A.rec_sum + w * TVBX_C * NP + jp, sm);
+    tvbx_ldf(A.msum + (size_t)k * NP + jp, am);
+    m -= A.sample0;
+    if (A.forcing != nullptr && a.tavg_period > 0 && m >= 0 &&
+        m < A.n_forcing) {
+      tvbx_ldf(A.forcing + (size_t)m * NP + jp, fo);
+    } else {
+#pragma unroll
+      for (int q = 0; q < TVBX_IPL; ++q) fo[q] = 0.0f;
+    }
+  };
+  fetch(0, mq);
+  for (int k = 0; k < a.n_steps; ++k) {
+    float xk[TVBX_S][TVBX_IPL], sk[TVBX_IPL], ak[TVBX_IPL], fk[TVBX_IPL];
+#pragma unroll
+    for (int q = 0; q < TVBX_IPL; ++q) {
+#pragma unroll
+      for (int s = 0; s < TVBX_S; ++s) xk[s][q] = xs[s][q];
+      sk[q] = sm[q];
+      ak[q] = am[q];
+      fk[q] = fo[q];
+    }
+    if (a.tavg_period > 0) {
+      if (mr == 0) {
+        mr = a.tavg_period;
+        --mq;
+      }
+      --mr;
+    }
+    if (k + 1 < a.n_steps) fetch(k + 1, mq);
+    float mu_o[TVBX_IPL];
+#pragma unroll
+    for (int q = 0; q < TVBX_IPL; ++q) {
+      float x[TVBX_S], lam[TVBX_S], ln[TVBX_S], gm[TVBX_NGM], gc[TVBX_NGC];
+#pragma unroll
+      for (int s = 0; s < TVBX_S; ++s) {
+        x[s] = xk[s][q];
+        lam[s] = lr[s][q];
+      }
+      const float mu = tvbx_adj_node(a, j, pb + q, lp[q], x, lam, sk[q],
+                                     ak[q], fk[q] * rK, ln, gc, gm);
+#pragma unroll
+      for (int s = 0; s < TVBX_S; ++s) lr[s][q] = ln[s];
+      mu_o[q] = mu;
+#if TVBX_HAS_NGC
+#pragma unroll
+      for (int g = 0; g < TVBX_NGC; ++g) gcr[g][q] = gcr[g][q] + mu * gc[g];
+#endif
+#if TVBX_HAS_NGM
+#pragma unroll
+      for (int g = 0; g < TVBX_NGM; ++g) gmr[g][q] = gmr[g][q] + a.dt * gm[g];
+#endif
+    }
+    tvbx_stf(A.mu + (size_t)t * NP + jp, mu_o);
+    t = t == 0 ? H - 1 : t - 1;
+  }
+#pragma unroll
+  for (int s = 0; s < TVBX_S; ++s) tvbx_stf(A.lam + s * NP + jp, lr[s]);
+#if TVBX_HAS_NGC
+#pragma unroll
+  for (int g = 0; g < TVBX_NGC; ++g) tvbx_stf(A.g_c + g * NP + jp, gcr[g]);
+#endif
+#if TVBX_HAS_NGM
+#pragma unroll
+  for (int g = 0; g < TVBX_NGM; ++g) tvbx_stf(A.g_m + g * NP + jp, gmr[g]);
+#endif
 }
 
 // Parameter gradients of the Euler-Maruyama transition log density of

@@ -1422,6 +1422,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     if ((bad >> q) & 1u) a.bad[pb + q] = 1u;
 }
 
+#define TVBX_SUMS_WAVES 4  // waves per workgroup of the sums kernels
 #if !TVBX_USES_POST && !TVBX_EMAJ
 // The sums of a blocked launch ahead of its updates.  Every step of the
 // launch reads slots written before it and pre() does not read post_syn, so
@@ -1441,7 +1442,6 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
 // 1024, float32: 5.8 TB/s); with 32 delay bins by the L2 and the issue of the
 // gathers (bfloat16, 256-byte rows: 17.9 us per step, 11.3 TB/s of gathered
 // bytes, against 23 us of the one-kernel launch's 27).
-#define TVBX_SUMS_WAVES 4
 extern "C" __global__ void __launch_bounds__(64 * TVBX_SUMS_WAVES)
 tvbx_sums(const tvbx_step_args a) {
   const int lane = threadIdx.x & 63;

@@ -176,6 +176,8 @@ typedef struct tvbx_adj_args {
   long long n_forcing;
   float *g_c;             /* [n_gc][N][pitch] coupling-parameter partials */
   float *g_m;             /* [n_gm][N][pitch] model-parameter partials */
+  float *msum;            /* [n_steps][N][pitch] transposed gathers of the
+                           * launch (tvbx_adj_sums -> tvbx_adjoint_sums) */
 } tvbx_adj_args;
 
 /* Parameter gradients of the Euler-Maruyama log density of forced steps:

@@ -152,6 +152,7 @@ struct tvbx_module {
   hipFunction_t step = nullptr;
   hipFunction_t hist = nullptr;
   hipFunction_t adj = nullptr;  // present when emitted with the adjoint
+  hipFunction_t adj_sums = nullptr, adj_from = nullptr;  // with it too
   hipFunction_t blocked = nullptr;  // absent in the reference ordering
   hipFunction_t step_sums = nullptr;  // blocked launch from given sums
   hipFunction_t sums = nullptr;  // absent also where pre() reads post_syn
@@ -237,6 +238,7 @@ struct tvbx_sim {
   int mfma_chunks = 0;
   // blocked launches as two kernels, the sums ahead of the updates
   bool ahead = false;
+  DevBuf msum;  // the reverse launches' gathers, as csum
 };
 
 // steps per launch of tvbx_mfma_sums (its accumulators: steps x ipl tiles)
@@ -415,6 +417,11 @@ static int module_from_image(tvbx_ctx *c, const void *image, size_t size,
   }
   if (hipModuleGetFunction(&m->adj, m->mod, "tvbx_adjoint") != hipSuccess)
     m->adj = nullptr;
+  if (hipModuleGetFunction(&m->adj_sums, m->mod, "tvbx_adj_sums") !=
+          hipSuccess ||
+      hipModuleGetFunction(&m->adj_from, m->mod, "tvbx_adjoint_sums") !=
+          hipSuccess)
+    m->adj_sums = m->adj_from = nullptr;
   if (hipModuleGetFunction(&m->logp_grad, m->mod, "tvbx_logp_grad") !=
       hipSuccess)
     m->logp_grad = nullptr;
@@ -973,6 +980,14 @@ static void fill_args(tvbx_sim *s, tvbx_step_args &a) {
   if (s->mfma || (s->ahead && !s->pace)) a.csum = (float *)s->csum.p;
 }
 
+// workgroups of 4 waves per step of the sums kernels: an eighth of the
+// (tile, node) pairs on each XCD
+static unsigned sums_grid(const tvbx_sim *s) {
+  const unsigned pairs =
+      (unsigned)(s->pitch / (64 * s->d.ipl)) * (unsigned)s->d.n_node;
+  return 8 * (((pairs + 7) / 8 + 3) / 4);
+}
+
 // One forward launch of a.n_steps steps: the step kernel of the launch
 // shape, or the kernel that forms the launch's sums (by gathers, or on the
 // matrix cores) and then the blocked updates from them.
@@ -985,13 +1000,12 @@ static hipError_t launch_steps(tvbx_sim *s, tvbx_step_args &a,
   void *params[] = {&a};
   hipFunction_t fn = is_blocked(d) ? s->mod->blocked : s->mod->step;
   if (a.csum) {
-    const unsigned pairs = gx * (unsigned)d.n_node, per = (pairs + 7) / 8;
     const hipError_t e =
         s->mfma ? hipModuleLaunchKernel(s->mod->mfma, (d.n_node + 15) / 16, gx,
                                         1, 256, 1, 1, 0, st, params, nullptr)
                 : hipModuleLaunchKernel(
-                      s->mod->sums, 8 * ((per + 3) / 4), (unsigned)a.n_steps, 1,
-                      256, 1, 1, 0, st, params, nullptr);
+                      s->mod->sums, sums_grid(s), (unsigned)a.n_steps, 1, 256,
+                      1, 1, 0, st, params, nullptr);
     if (e != hipSuccess) return e;
     fn = s->mod->step_sums;
   }
@@ -1147,7 +1161,7 @@ extern "C" int tvbx_sim_destroy(tvbx_sim *s) {
     hipStreamDestroy(s->aux);
   }
   for (hipEvent_t e : s->adj_ev) hipEventDestroy(e);
-  DevBuf *mf[] = {&s->mfma_blk, &s->mfma_pairs, &s->mfma_w, &s->csum,
+  DevBuf *mf[] = {&s->msum, &s->mfma_blk, &s->mfma_pairs, &s->mfma_w, &s->csum,
                   &s->pace_buf};
   for (DevBuf *b : mf) dfree(*b);
   for (auto &b : s->ck_state) dfree(b);
@@ -2978,6 +2992,9 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
   AL(g_c, (size_t)ngc * NP * 4);
   AL(g_m, (size_t)ngm * NP * 4);
   AL(g_out, (size_t)ngc * pitch * 4);
+  // reverse launches as two kernels where the forward ones are
+  const bool ahead = s->ahead && s->mod->adj_sums;
+  if (ahead) AL(msum, (size_t)d.steps_per_launch * NP * 4);
   // replaying inside the checkpoints leaves the end-of-run state and ring
   // untouched: nothing to save
   const bool consume = !s->ck_recorded && !s->ck_keep;
@@ -3123,9 +3140,14 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
       A.n_forcing = n_samples;
       A.g_c = (float *)s->g_c.p;
       A.g_m = (float *)s->g_m.p;
+      A.msum = (float *)s->msum.p;
       void *params[] = {&A};
-      HIPCHK(hipModuleLaunchKernel(s->mod->adj, gx, gy, 1, bx, 1, 1, 0, sa,
-                                   params, nullptr));
+      if (ahead)
+        HIPCHK(hipModuleLaunchKernel(s->mod->adj_sums, sums_grid(s),
+                                     (unsigned)A.f.n_steps, 1, 256, 1, 1, 0,
+                                     sa, params, nullptr));
+      HIPCHK(hipModuleLaunchKernel(ahead ? s->mod->adj_from : s->mod->adj, gx,
+                                   gy, 1, bx, 1, 1, 0, sa, params, nullptr));
     }
     if (overlap) HIPCHK(hipEventRecord(ev_rev(kw), sa));
   }

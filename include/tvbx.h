@@ -351,6 +351,16 @@ int tvbx_stream_rates(tvbx_ctx *ctx, size_t bytes, double *read_gbs,
 int tvbx_fc_loss(tvbx_ctx *ctx, const float *samples, long long n, int N,
                  int P, const float *target, int target_per_instance,
                  float *loss, float *s, float *mean);
+
+/* The gradient of sum_p gout[p] loss[p] with respect to the samples, from
+ * tvbx_fc_loss's s and mean:
+ *   dsamples[m][k][p] = gout[p] sum_j s[k][j][p] (samples[m][j][p] -
+ *                       mean[j][p]),
+ * float32 device arrays, samples and dsamples [n][N][P], gout [P].  Queued
+ * on the context's stream; no workspace. */
+int tvbx_fc_loss_grad(tvbx_ctx *ctx, const float *samples, long long n, int N,
+                      int P, const float *s, const float *mean,
+                      const float *gout, float *dsamples);
 /* out[c][r] = in[r][c] - sub[r % sub_rows][c] (sub may be null): device
  * arrays, in [rows][cols] -> out [cols][rows].  No counterpart in the
  * reference: it moves the FC-loss gradient's operands between the

@@ -2410,6 +2410,84 @@ k_fl_loss(const double *__restrict__ m2, int N, int pitch, int P,
   }
 }
 
+// The loss's gradient, dx[m][k][p] = gout[p] sum_j s[k][j][p] (x[m][j][p] -
+// mean[j][p]): per instance a matrix product, with the instances innermost
+// in every operand, so lanes are instances and a wave keeps a FG_M x FG_K
+// tile of (sample, node) sums per lane: per j it loads FG_M + FG_K values
+// (coalesced) for FG_M FG_K fused multiply-adds, with no transposed copies.
+// The next j's values are loaded while the current ones are used.
+//   The FG_W waves of a workgroup share the samples of one m tile.  Each XCD
+// (which takes workgroup ids round robin) works through a contiguous range
+// of (instance tile, m tile, node group); the node groups of an m tile run
+// together (its samples are fetched once) while an instance tile's s fits
+// the L2, else the m tiles of a node group (its rows of s are).
+// grid 8 ceil(items / 8), block 64 FG_W.
+#define FG_M 16
+#define FG_K 8
+#define FG_W 4
+__global__ void __launch_bounds__(64 * FG_W, 2)
+k_fl_grad(const float *__restrict__ x, int M, int N, int P,
+          const float *__restrict__ s, const float *__restrict__ mean,
+          const float *__restrict__ gout, int mt, int kg, int k_outer,
+          unsigned items, float *__restrict__ dx) {
+  const unsigned per = gridDim.x / 8;
+  const unsigned id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (id >= items) return;
+  const unsigned B = (unsigned)mt * (unsigned)kg;
+  const unsigned b = id % B;
+  const int m0 = (int)(k_outer ? b % mt : b / kg) * FG_M;
+  const int k0 = __builtin_amdgcn_readfirstlane(
+      (int)(((k_outer ? b / mt : b % kg) * FG_W + (threadIdx.x >> 6)) * FG_K));
+  if (k0 >= N) return;
+  const int p = (int)(id / B) * 64 + (threadIdx.x & 63);
+  const unsigned pp = min(p, P - 1);  // lanes past P store nothing
+  const size_t NP = (size_t)N * P;
+  // rows past the last sample or node repeat it
+  const float *xr[FG_M], *sr[FG_K];
+#pragma unroll
+  for (int r = 0; r < FG_M; ++r) xr[r] = x + (size_t)min(m0 + r, M - 1) * NP;
+#pragma unroll
+  for (int c = 0; c < FG_K; ++c) sr[c] = s + (size_t)min(k0 + c, N - 1) * NP;
+  float acc[FG_M][FG_K];
+#pragma unroll
+  for (int r = 0; r < FG_M; ++r)
+#pragma unroll
+    for (int c = 0; c < FG_K; ++c) acc[r][c] = 0.0f;
+  float xv[FG_M], sv[FG_K], mv;
+  auto fetch = [&](int j) {
+    const size_t o = (size_t)j * P;
+#pragma unroll
+    for (int r = 0; r < FG_M; ++r) xv[r] = xr[r][o + pp];
+#pragma unroll
+    for (int c = 0; c < FG_K; ++c) sv[c] = sr[c][o + pp];
+    mv = mean[o + pp];
+  };
+  fetch(0);
+  for (int j = 0; j < N; ++j) {
+    float xc[FG_M], sc[FG_K];
+#pragma unroll
+    for (int r = 0; r < FG_M; ++r) xc[r] = xv[r] - mv;
+#pragma unroll
+    for (int c = 0; c < FG_K; ++c) sc[c] = sv[c];
+    fetch(min(j + 1, N - 1));
+#pragma unroll
+    for (int r = 0; r < FG_M; ++r)
+#pragma unroll
+      for (int c = 0; c < FG_K; ++c)
+        acc[r][c] = fmaf(sc[c], xc[r], acc[r][c]);
+  }
+  const float g = gout[pp];
+  if (p >= P) return;
+#pragma unroll
+  for (int r = 0; r < FG_M; ++r) {
+    if (m0 + r >= M) break;
+#pragma unroll
+    for (int c = 0; c < FG_K; ++c)
+      if (k0 + c < N)
+        dx[(size_t)(m0 + r) * NP + (size_t)(k0 + c) * P + p] = g * acc[r][c];
+  }
+}
+
 // out[c][r] = in[r][c] - sub[r % sub_rows][c] (sub null: no subtraction),
 // in [rows][cols] -> out [cols][rows], through 64 x 64 tiles in LDS.
 // grid (ceil(cols / 64), ceil(rows / 64)) (the y extent split over z when
@@ -2519,6 +2597,27 @@ extern "C" int tvbx_fc_loss(tvbx_ctx *c, const float *samples, long long n,
                      N, pitch, P, target, target_per_instance, rs, loss, s);
   hipLaunchKernelGGL(k_f64_to_f32_rows, dim3(grid1d((size_t)N * P, 256)),
                      dim3(256), 0, st, dmean, (size_t)N, pitch, P, mean);
+  HIPCHK(hipGetLastError());
+  return TVBX_OK;
+}
+
+extern "C" int tvbx_fc_loss_grad(tvbx_ctx *c, const float *samples,
+                                 long long n, int N, int P, const float *s,
+                                 const float *mean, const float *gout,
+                                 float *dsamples) {
+  CHECK(c && samples && s && mean && gout && dsamples, "null argument");
+  CHECK(n >= 1 && N >= 1 && P >= 1, "empty problem");
+  CHECK(n <= (1ll << 30), "too many samples");
+  HIPCHK(hipSetDevice(c->device));
+  const long long mt = (n + FG_M - 1) / FG_M;
+  const int kg = (N + FG_K * FG_W - 1) / (FG_K * FG_W);
+  const long long items = (long long)((P + 63) / 64) * mt * kg;
+  CHECK(items < (1ll << 31) - 8, "FC loss gradient too large for one launch");
+  const int k_outer = (size_t)N * N * 256 > (3u << 20);
+  hipLaunchKernelGGL(k_fl_grad, dim3(8 * (unsigned)((items + 7) / 8)),
+                     dim3(64 * FG_W), 0, c->stream, samples, (int)n, N, P, s,
+                     mean, gout, (int)mt, kg, k_outer, (unsigned)items,
+                     dsamples);
   HIPCHK(hipGetLastError());
   return TVBX_OK;
 }

@@ -147,9 +147,9 @@ def fc_loss(samples, fc_target):
 class _FcLossDevice(torch.autograd.Function):
     """fc_loss of device samples on the HIP kernels: the FP64 co-moments
     and the loss with its derivative in libtvbx (tvbx_fc_loss), the samples'
-    gradient as one batched float32 product per instance,
-    dL_p/dx_p = gout_p (x_p - mean_p) S_p, between two transposes
-    (tvbx_transpose) that take the instance axis outermost and back."""
+    gradient as one float32 product per instance, dL_p/dx_p = gout_p (x_p -
+    mean_p) S_p, with the instances innermost throughout
+    (tvbx_fc_loss_grad)."""
 
     @staticmethod
     def forward(ctx, samples, fc_target, hctx):
@@ -179,17 +179,11 @@ class _FcLossDevice(torch.autograd.Function):
         M, N, P = x.shape
         hctx = ctx.hctx
         dev = x.device
-        xt = torch.empty((P, M * N), dtype=torch.float32, device=dev)
-        sp = (s.permute(2, 0, 1) *
-              gout.detach().float()[:, None, None]).contiguous()
-        torch.cuda.current_stream(dev).synchronize()
-        hctx.transpose(x.data_ptr(), M * N, P, xt.data_ptr(),
-                       mean.data_ptr(), N)
-        hctx.sync()
-        y = torch.bmm(xt.view(P, M, N), sp)
+        g = gout.detach().float().contiguous()
         dx = torch.empty((M, N, P), dtype=torch.float32, device=dev)
         torch.cuda.current_stream(dev).synchronize()
-        hctx.transpose(y.data_ptr(), P, M * N, dx.data_ptr())
+        hctx.fc_loss_grad(x.data_ptr(), M, N, P, s.data_ptr(),
+                          mean.data_ptr(), g.data_ptr(), dx.data_ptr())
         hctx.sync()
         return dx.to(ctx.dtype), None, None
 

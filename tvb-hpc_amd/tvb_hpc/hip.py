@@ -118,6 +118,7 @@ _SIGS = {
     'tvbx_corr': [_P, _P, _LL, _I, _I, _P],
     'tvbx_corr_noalloc': [_P, _P, _LL, _I, _I, _P],
     'tvbx_fc_loss': [_P, _P, _LL, _I, _I, _P, _I, _P, _P, _P],
+    'tvbx_fc_loss_grad': [_P, _P, _LL, _I, _I, _P, _P, _P, _P],
     'tvbx_transpose': [_P, _P, _LL, _LL, _P, _I, _P],
     'tvbx_stream_rates': [_P, _SZ, _P, _P],
     'tvbx_rmap_create': [_P, _P, _I, _I, _P],
@@ -296,6 +297,18 @@ class Context:
                                  ctypes.c_void_p(loss_ptr),
                                  ctypes.c_void_p(s_ptr),
                                  ctypes.c_void_p(mean_ptr)))
+
+    def fc_loss_grad(self, samples_ptr, n, N, P, s_ptr, mean_ptr, gout_ptr,
+                     dsamples_ptr):
+        """tvbx_fc_loss_grad on device memory: the samples' gradient (n, N, P)
+        of sum(gout * loss) from fc_loss's s and mean, gout (P,); queued on
+        this context's stream."""
+        check(lib().tvbx_fc_loss_grad(self.h, ctypes.c_void_p(samples_ptr),
+                                      int(n), int(N), int(P),
+                                      ctypes.c_void_p(s_ptr),
+                                      ctypes.c_void_p(mean_ptr),
+                                      ctypes.c_void_p(gout_ptr),
+                                      ctypes.c_void_p(dsamples_ptr)))
 
     def stream_rates(self, mib=1024):
         """(read GB/s, copy GB/s): the best of a grid-stride read and a

@@ -528,18 +528,6 @@ __global__ void k_fill_f64(double *p, size_t n, double v) {
   for (; i < n; i += stride) p[i] = v;
 }
 
-// out[r][p] = in[r][p] (pitch-strided FP64 rows -> compact float32 rows)
-__global__ void k_f64_to_f32_rows(const double *__restrict__ in, size_t rows,
-                                  int pitch, int P, float *__restrict__ out) {
-  size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; k < rows * (size_t)P; k += stride) {
-    const size_t r = k / P;
-    const int p = (int)(k - r * P);
-    out[k] = (float)in[r * pitch + p];
-  }
-}
-
 __global__ void k_fill_u32(unsigned *p, size_t n, unsigned v) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -2315,11 +2303,15 @@ extern "C" int tvbx_corr_noalloc(tvbx_ctx *c, const float *samples,
 // Since M2_ij = sum_m xc_mi xc_mj (xc = x - mean, sum_m xc_m = 0), the
 // samples' gradient is dL/dx_mk = sum_j S_kj xc_mj with S symmetric,
 // S_kj = dL/dM2_kj (k != j) and S_kk = 2 dL/dM2_kk = -rs_k^2 D_k.
-//   One lane per instance; the waves of a workgroup share its 64 instances
-// and take the rows k = w, w + NW, ...; their partial sums meet in LDS.  A
+//   Lanes are instances; a workgroup is FL_NW rows of a 64-instance tile, one
+// a wave, so that rows and tiles together fill the chip (one workgroup per
+// tile, its waves looping over the rows of all three passes, left 16 of 256
+// CUs busy at P = 1024: 552 us for 84 nodes, against 85 us in these four
+// kernels).  The sums over pairs go through one partial per row group; every
+// pass re-reads the co-moments, from the caches up to some hundred MB.  A
 // pair's a_ij and G_ij are computed from (min, max) in one order, so the two
-// waves that need a pair get the same values and S comes out symmetric.
-#define FL_NW 16
+// rows that need a pair get the same values and S comes out symmetric.
+#define FL_NW 8
 __device__ __forceinline__ double fl_a(const double *__restrict__ m2,
                                        const double *__restrict__ rs, int i,
                                        int j, int N, int pitch, int p) {
@@ -2336,78 +2328,123 @@ __device__ __forceinline__ double fl_b(const float *__restrict__ target,
                   : (double)target[(size_t)lo * N + hi];
 }
 
-// sum over the workgroup's waves of v (one value per lane), for every wave
-__device__ __forceinline__ double fl_wg_sum(double v, double *red) {
+// per (node, instance): 1 / sqrt(M2_ii) and the mean (u: the mean of the
+// block, merged into nothing) as float32 [N][P].  grid (pitch / 64, N),
+// block 64.
+__global__ void k_fl_node(const double *__restrict__ m2, int N, int pitch,
+                          int P, const double *__restrict__ u,
+                          double *__restrict__ rs, float *__restrict__ mean) {
+  const int p = blockIdx.x * 64 + threadIdx.x;
+  const int i = blockIdx.y;
+  rs[(size_t)i * pitch + p] = 1.0 / sqrt(m2[tri_index(i, i, N) * pitch + p]);
+  if (p < P) mean[(size_t)i * P + p] = (float)u[(size_t)i * pitch + p];
+}
+
+// the workgroup's sum of v over its waves into part[g][p] (wave 0)
+__device__ __forceinline__ void fl_group_sum(double v, double *red,
+                                             double *__restrict__ part,
+                                             int pitch) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __syncthreads();  // red is free
   red[w * 64 + lane] = v;
   __syncthreads();
+  if (w == 0) {
+    double t = red[lane];
+#pragma unroll
+    for (int k = 1; k < FL_NW; ++k) t += red[k * 64 + lane];
+    part[(size_t)blockIdx.y * pitch + blockIdx.x * 64 + lane] = t;
+  }
+}
+
+// the sum of plane q of part [planes][G][pitch] over the row groups
+__device__ __forceinline__ double fl_total(const double *__restrict__ part,
+                                           int q, int G, int pitch, int p) {
   double t = 0.0;
-  for (int k = 0; k < FL_NW; ++k) t += red[k * 64 + lane];
-  __syncthreads();
+#pragma unroll 8
+  for (int g = 0; g < G; ++g) t += part[((size_t)q * G + g) * pitch + p];
   return t;
 }
 
-// grid ceil(P / 64), block 64 * FL_NW.  m2 [N(N+1)/2][pitch], target
-// [N][N] (shared) or [N][N][P] (per instance); rs [N][pitch] workspace;
-// loss [P]; s [N][N][P].
+// pass 1: sums of the two triangles (planes 0, 1 of part [5][G][pitch]).
+// grid (pitch / 64, G = ceil(N / FL_NW)), block 64 FL_NW.
 __global__ void __launch_bounds__(64 * FL_NW)
-k_fl_loss(const double *__restrict__ m2, int N, int pitch, int P,
-          const float *__restrict__ target, int per_inst,
-          double *__restrict__ rs, float *__restrict__ loss,
-          float *__restrict__ s) {
+k_fl_sum(const double *__restrict__ m2, int N, int pitch, int P,
+         const float *__restrict__ target, int per_inst,
+         const double *__restrict__ rs, double *__restrict__ part) {
   __shared__ double red[64 * FL_NW];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int p = blockIdx.x * 64 + lane;
-  const bool on = p < P;
-  // lanes past P compute on the workgroup's first instance (always < P, and
-  // its rs column is written by this workgroup) and store nothing
-  const int pp = on ? p : blockIdx.x * 64;
-  for (int i = w; i < N; i += FL_NW)
-    rs[(size_t)i * pitch + p] =
-        1.0 / sqrt(m2[tri_index(i, i, N) * pitch + pp]);
-  __syncthreads();
-  const double *rsp = rs;
-  // pass 1: means of the two triangles
+  const int p = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int pt = min(p, P - 1);  // the target has no padding
+  const int i = blockIdx.y * FL_NW + (threadIdx.x >> 6);
   double sa = 0.0, sb = 0.0;
-  for (int i = w; i < N; i += FL_NW)
-    for (int j = i + 1; j < N; ++j) {
-      sa += fl_a(m2, rsp, i, j, N, pitch, pp);
-      sb += fl_b(target, per_inst, i, j, N, P, pp);
-    }
-  const double K = 0.5 * (double)N * (double)(N - 1);
-  const double ma = fl_wg_sum(sa, red) / K, mb = fl_wg_sum(sb, red) / K;
-  // pass 2: norms and the dot product of the centred triangles
-  double saa = 0.0, sbb = 0.0, sab = 0.0;
-  for (int i = w; i < N; i += FL_NW)
-    for (int j = i + 1; j < N; ++j) {
-      const double a = fl_a(m2, rsp, i, j, N, pitch, pp) - ma;
-      const double b = fl_b(target, per_inst, i, j, N, P, pp) - mb;
-      saa = fma(a, a, saa);
-      sbb = fma(b, b, sbb);
-      sab = fma(a, b, sab);
-    }
-  saa = fl_wg_sum(saa, red);
-  sbb = fl_wg_sum(sbb, red);
-  sab = fl_wg_sum(sab, red);
-  const double nab = sqrt(saa * sbb);
-  const double r = sab / nab;
-  if (on && w == 0) loss[p] = (float)(1.0 - r);
-  // pass 3: S, row k by its wave
-  for (int k = w; k < N; k += FL_NW) {
-    const double rk = rsp[(size_t)k * pitch + pp];
-    double D = 0.0;
-    for (int j = 0; j < N; ++j) {
-      if (j == k) continue;
-      const double a = fl_a(m2, rsp, k, j, N, pitch, pp);
-      const double b = fl_b(target, per_inst, k, j, N, P, pp);
-      const double G = -((b - mb) / nab - r * (a - ma) / saa);
-      D = fma(G, a, D);
-      if (on)
-        s[((size_t)k * N + j) * P + p] =
-            (float)(G * rk * rsp[(size_t)j * pitch + pp]);
-    }
-    if (on) s[((size_t)k * N + k) * P + p] = (float)(-rk * rk * D);
+#pragma unroll 8
+  for (int j = i + 1; j < N; ++j) {
+    sa += fl_a(m2, rs, i, j, N, pitch, p);
+    sb += fl_b(target, per_inst, i, j, N, P, pt);
   }
+  const size_t plane = (size_t)gridDim.y * pitch;
+  fl_group_sum(sa, red, part, pitch);
+  fl_group_sum(sb, red, part + plane, pitch);
+}
+
+// pass 2: norms and the dot product of the centred triangles (planes 2 .. 4)
+__global__ void __launch_bounds__(64 * FL_NW)
+k_fl_norm(const double *__restrict__ m2, int N, int pitch, int P,
+          const float *__restrict__ target, int per_inst,
+          const double *__restrict__ rs, double *__restrict__ part) {
+  __shared__ double red[64 * FL_NW];
+  const int p = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int pt = min(p, P - 1);
+  const int i = blockIdx.y * FL_NW + (threadIdx.x >> 6);
+  const int G = gridDim.y;
+  const double K = 0.5 * (double)N * (double)(N - 1);
+  const double ma = fl_total(part, 0, G, pitch, p) / K;
+  const double mb = fl_total(part, 1, G, pitch, p) / K;
+  double saa = 0.0, sbb = 0.0, sab = 0.0;
+#pragma unroll 8
+  for (int j = i + 1; j < N; ++j) {
+    const double a = fl_a(m2, rs, i, j, N, pitch, p) - ma;
+    const double b = fl_b(target, per_inst, i, j, N, P, pt) - mb;
+    saa = fma(a, a, saa);
+    sbb = fma(b, b, sbb);
+    sab = fma(a, b, sab);
+  }
+  const size_t plane = (size_t)G * pitch;
+  fl_group_sum(saa, red, part + 2 * plane, pitch);
+  fl_group_sum(sbb, red, part + 3 * plane, pitch);
+  fl_group_sum(sab, red, part + 4 * plane, pitch);
+}
+
+// pass 3: the loss [P] and S [N][N][P], row k by its wave
+__global__ void __launch_bounds__(64 * FL_NW)
+k_fl_s(const double *__restrict__ m2, int N, int pitch, int P,
+       const float *__restrict__ target, int per_inst,
+       const double *__restrict__ rs, const double *__restrict__ part,
+       float *__restrict__ loss, float *__restrict__ s) {
+  const int p = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int k = blockIdx.y * FL_NW + (threadIdx.x >> 6);
+  if (k >= N || p >= P) return;
+  const int G = gridDim.y;
+  const double K = 0.5 * (double)N * (double)(N - 1);
+  const double ma = fl_total(part, 0, G, pitch, p) / K;
+  const double mb = fl_total(part, 1, G, pitch, p) / K;
+  const double saa = fl_total(part, 2, G, pitch, p);
+  const double nab = sqrt(saa * fl_total(part, 3, G, pitch, p));
+  const double r = fl_total(part, 4, G, pitch, p) / nab;
+  if (k == 0) loss[p] = (float)(1.0 - r);
+  const double rk = rs[(size_t)k * pitch + p];
+  const double inab = 1.0 / nab, rsaa = r / saa;
+  double D = 0.0;
+#pragma unroll 4
+  for (int j = 0; j < N; ++j) {
+    if (j == k) continue;
+    const double a = fl_a(m2, rs, k, j, N, pitch, p);
+    const double b = fl_b(target, per_inst, k, j, N, P, p);
+    const double gkj = -((b - mb) * inab - (a - ma) * rsaa);
+    D = fma(gkj, a, D);
+    s[((size_t)k * N + j) * P + p] =
+        (float)(gkj * rk * rs[(size_t)j * pitch + p]);
+  }
+  s[((size_t)k * N + k) * P + p] = (float)(-rk * rk * D);
 }
 
 // The loss's gradient, dx[m][k][p] = gout[p] sum_j s[k][j][p] (x[m][j][p] -
@@ -2555,6 +2592,7 @@ extern "C" int tvbx_fc_loss(tvbx_ctx *c, const float *samples, long long n,
   const size_t o_m2 = take(tri * pitch * 8), o_mean = take(NP * 8),
                o_s1 = take(NP * 8), o_u = take(NP * 8),
                o_shift = take(NP * 4), o_rs = take(NP * 8),
+               o_part = take((size_t)((N + FL_NW - 1) / FL_NW) * pitch * 40),
                o_tiles = take((size_t)n_tiles * 8),
                o_smp = stage ? take((size_t)n * NP * 4) : 0;
   int rc = ctx_work(c, used);
@@ -2591,12 +2629,16 @@ extern "C" int tvbx_fc_loss(tvbx_ctx *c, const float *samples, long long n,
   hipLaunchKernelGGL(k_fc_update, dim3((unsigned)nwg), dim3(64 * FC_NW), 0,
                      st, smp, (int)n, 0ll, (int)n, N, pitch, 0.0, tiles,
                      n_tiles, n_fblk, shift, s1, u, m2);
-  hipLaunchKernelGGL(k_fc_mean, dim3(pitch / 64, N), dim3(64), 0, st, N,
-                     pitch, (int)n, 0.0, u, dmean);
-  hipLaunchKernelGGL(k_fl_loss, dim3(pitch / 64), dim3(64 * FL_NW), 0, st, m2,
-                     N, pitch, P, target, target_per_instance, rs, loss, s);
-  hipLaunchKernelGGL(k_f64_to_f32_rows, dim3(grid1d((size_t)N * P, 256)),
-                     dim3(256), 0, st, dmean, (size_t)N, pitch, P, mean);
+  double *part = reinterpret_cast<double *>(base + o_part);
+  const dim3 rows(pitch / 64, (N + FL_NW - 1) / FL_NW);
+  hipLaunchKernelGGL(k_fl_node, dim3(pitch / 64, N), dim3(64), 0, st, m2, N,
+                     pitch, P, u, rs, mean);
+  hipLaunchKernelGGL(k_fl_sum, rows, dim3(64 * FL_NW), 0, st, m2, N, pitch, P,
+                     target, target_per_instance, rs, part);
+  hipLaunchKernelGGL(k_fl_norm, rows, dim3(64 * FL_NW), 0, st, m2, N, pitch,
+                     P, target, target_per_instance, rs, part);
+  hipLaunchKernelGGL(k_fl_s, rows, dim3(64 * FL_NW), 0, st, m2, N, pitch, P,
+                     target, target_per_instance, rs, part, loss, s);
   HIPCHK(hipGetLastError());
   return TVBX_OK;
 }

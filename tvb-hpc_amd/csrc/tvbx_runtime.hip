@@ -183,6 +183,7 @@ struct tvbx_sim {
   DevBuf out_input, out_drift, out_diffs, tavg, bold_state, samples, bad,
       noise, fc_mean, fc_m2, corr, stale;
   DevBuf fc_tiles, fc_shift, fc_s1, fc_u;  // FC merge work buffers
+  int smp_ld = 0;  // row length of the samples (0: pitch)
   // forced steps (tvbx_sim_logp): trajectory window and log-density sums
   DevBuf force, logp, logp_sum, lg_c, lg_m;
   long long force_step0 = 0;
@@ -522,12 +523,6 @@ __global__ void k_fill_f32(float *p, size_t n, float v) {
   for (; i < n; i += stride) p[i] = v;
 }
 
-__global__ void k_fill_f64(double *p, size_t n, double v) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; i < n; i += stride) p[i] = v;
-}
-
 __global__ void k_fill_u32(unsigned *p, size_t n, unsigned v) {
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -539,8 +534,6 @@ __host__ __device__ inline size_t tri_index(int i, int j, int N) {
   return (size_t)i * N - (size_t)i * (i - 1) / 2 + (size_t)(j - i);
 }
 
-#define FC_ST 8   // tiles per super-tile edge (rows kept in one XCD's L2)
-
 // Merge of a block of m = `count` monitor samples (slots first, first + 1,
 // ... modulo slots) into FP64 co-moments M2 and means ma of the n_a samples
 // merged before (Chan, Golub & LeVeque's pairwise update):
@@ -549,94 +542,128 @@ __host__ __device__ inline size_t tri_index(int i, int j, int N) {
 // With d_k = x_k - shift for any per-(node, instance) shift,
 //   sum_k (x_ki - mb_i)(x_kj - mb_j) = sum_k d_ki d_kj - S1_i S1_j / m,
 //   S1 = sum_k d_k,
-// so the block is read once.  The shift is the running mean rounded to
+// so no second pass over the block needs its mean.  The shift is the running mean rounded to
 // float (the block's first sample before the first merge), which keeps d
 // small and makes x - shift exact in double.
 
-// per (node, instance): shift, S1 and u of the block
-__global__ void k_fc_prep(const float *__restrict__ samples, int slots,
-                          long long first, int count, int N, int pitch,
-                          double n_prev, const double *__restrict__ mean,
-                          float *__restrict__ shift, double *__restrict__ s1,
-                          double *__restrict__ u) {
-  const int p = blockIdx.x * 64 + threadIdx.x;
+// per (node, instance): shift, S1 and u of the block; rows of ld >= the
+// instances in use.  The 4 waves of a workgroup take a quarter of the samples
+// each, 16 loads in flight a wave: bound by the reads (500 x 84 x 1024 in 29
+// us, 6.0 TB/s; one wave per (node, 64 instances) with one load at a time
+// took 251 us).
+// grid (pitch / 64, N), block 256.
+#define FC_PREP_U 16
+__global__ void __launch_bounds__(256)
+k_fc_prep(const float *__restrict__ samples, int ld, int slots,
+          long long first, int count, int N, int pitch, double n_prev,
+          const double *__restrict__ mean, float *__restrict__ shift,
+          double *__restrict__ s1, double *__restrict__ u) {
+  __shared__ double part[4 * 64];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p = blockIdx.x * 64 + lane;
   const int i = blockIdx.y;
-  const size_t NP = (size_t)N * pitch;
+  const size_t SN = (size_t)N * ld;
+  // padding instances read the last one's values
+  const float *row = samples + (size_t)i * ld + min(p, ld - 1);
   const size_t ip = (size_t)i * pitch + p;
-  const double ma = mean[ip];
-  const float sh = n_prev > 0.0 ? (float)ma
-                                : samples[(size_t)(first % slots) * NP + ip];
+  const int slot0 = (int)(first % slots);
+  const double ma = n_prev > 0.0 ? mean[ip] : 0.0;
+  const float sh = n_prev > 0.0 ? (float)ma : row[(size_t)slot0 * SN];
+  const int k0 = (int)((long long)count * w / 4);
+  const int k1 = (int)((long long)count * (w + 1) / 4);
+  int slot = slot0 + k0;
+  slot -= slot >= slots ? slots : 0;
   double s = 0.0;
-  for (int k = 0; k < count; ++k)
-    s += (double)samples[(size_t)((first + k) % slots) * NP + ip] - (double)sh;
+  for (int k = k0; k < k1; k += FC_PREP_U) {
+    float v[FC_PREP_U];
+#pragma unroll
+    for (int t = 0; t < FC_PREP_U; ++t) {
+      // a sample past the share repeats the last and is not added
+      v[t] = row[(size_t)slot * SN];
+      if (k + t + 1 < k1) slot = slot + 1 == slots ? 0 : slot + 1;
+    }
+#pragma unroll
+    for (int t = 0; t < FC_PREP_U; ++t)
+      if (k + t < k1) s += (double)v[t] - (double)sh;
+  }
+  part[w * 64 + lane] = s;
+  __syncthreads();
+  if (w) return;
+  s = part[lane] + part[64 + lane] + part[128 + lane] + part[192 + lane];
   shift[ip] = sh;
   s1[ip] = s;
   u[ip] = ((double)sh + s / (double)count) - ma;
 }
 
-// co-moments of one 16 x 16 tile of node pairs (tile I <= tile J) for the
-// 64 instances of one lane block.  Workgroups are numbered so that each of
+// co-moments of one 16 x 16 tile of node pairs (tile I <= tile J) for a block
+// of PB instances.  Workgroups are numbered so that each of
 // the 8 XCDs (which take workgroup ids round robin) works through a
 // contiguous range of (instance block, tile), tiles in super-tile order.
 #define FC_TILE 16
 #define FC_KC 4     // samples per MFMA (K of v_mfma_f64_16x16x4f64)
 #define FC_XS ((FC_KC + 1) * 48 + 1)  // LDS dwords per instance (see below)
+#define FC_NW 8     // waves per workgroup (8 measured faster than 4 or 16)
 typedef double fc_d4 __attribute__((ext_vector_type(4)));
 
 // The block's co-moments C_ij = sum_k d_ki d_kj of one 16 x 16 tile of node
-// pairs for a block of 32 instances, on the FP64 matrix cores: per instance,
+// pairs for a block of PB instances, on the FP64 matrix cores: per instance,
 // C += A B with A (16 x 4) the d of the tile's row nodes over 4 samples and
 // B (4 x 16) those of its column nodes; v_mfma_f64_16x16x4f64 takes A[i][k]
 // from lane 16 k + i, B[k][j] from lane 16 k + j, and leaves C[4 r + l / 16]
-// [l % 16] in element r of lane l.  Each of the 8 waves keeps 4 instances'
-// tiles (4 doubles per lane each) for the whole block.
+// [l % 16] in element r of lane l.  Each of the 8 waves keeps PB / 8
+// instances' tiles (4 doubles per lane each) for the whole block.
 //   Samples are staged 4 at a time through LDS transposed, instance-major:
 // x[pl][k * 48 + r] (r < 16: row node I0 + r, else column node J0 + r - 16;
 // 16 dwords of padding per sample and one per instance; "sample" 4 holds the
 // 32 nodes' shifts, written once), so the operand reads (lanes = (k, node))
-// fall in distinct banks; each half-wave stages 8 node rows of one sample,
-// and the next 4 samples' global loads are in flight while the current ones
+// fall in distinct banks; a wave stages half of one sample's node rows, and the next 4 samples' global loads are in flight while the current ones
 // are multiplied.  d = x - shift is formed in FP64 at the operand (exact, as
-// the shift is the float running mean).  A small LDS footprint (31 KB) and
-// few registers per wave let 3 workgroups of 8 waves share a CU.
+// the shift is the float running mean).  With PB = 32 (128-byte loads,
+// 31 KB of LDS) 3 workgroups of 8 waves share a CU; PB = 16 gives twice the
+// workgroups, 4 to a CU, for problems that would not fill the chip (the rule
+// is at fc_shape_of).
+//   Bound: the FP64 matrix cores are busy half of the time at best (N = 998,
+// P = 1024, 255 samples: 7.2 ms, 36 TFLOP/s, SQ_VALU_MFMA_BUSY_CYCLES 52 %),
+// with the operands' FP64 conversions and the staging between the products.
+// Tiles of 32 x 32 nodes, which halve both per product, took 7.0 ms there and
+// were slower on small problems.
 //   The merge into M2 (lanes = instances, coalesced) goes through LDS in 4
-// passes of 64 pairs: in pass m, element m of lane l is pair 64 m + l.
-#define FC_PB 32  // instances per workgroup
-#define FC_NW 8   // waves per workgroup (8 measured faster than 4 or 16)
-#define FC_IW (FC_PB / FC_NW)     // instances per wave
-#define FC_RG (64 / FC_NW)        // node rows staged per half-wave
-#define FC_GS (FC_NW / 2)         // half-waves per staged sample
-__global__ void __launch_bounds__(64 * FC_NW, 6)
+// passes of 64 pairs: in pass m, element m of lane l is pair 64 m + l.  The
+// first merge (n_prev == 0) writes M2 without reading it.
+template <int PB>
+__global__ void __launch_bounds__(64 * FC_NW, PB == 16 ? 8 : 6)
 k_fc_update(const float *__restrict__ samples, int slots, long long first,
-            int count, int N, int pitch, double n_prev,
+            int count, int N, int pitch, double n_prev, int ld,
             const int2 *__restrict__ tiles, int n_tiles, int n_pblk,
             const float *__restrict__ shift, const double *__restrict__ s1,
             const double *__restrict__ u, double *__restrict__ m2) {
-  __shared__ __attribute__((aligned(16))) float xs[FC_PB * FC_XS];
+  constexpr int IW = PB / FC_NW;     // instances per wave
+  constexpr int G = 64 / PB;         // row groups of a wave's lanes
+  constexpr int RG = 16 / G;         // node rows staged per lane
+  __shared__ __attribute__((aligned(16))) float xs[PB * FC_XS];
   const unsigned per = gridDim.x / 8;  // grid is a multiple of 8
   const unsigned L = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (L >= (unsigned)n_tiles * (unsigned)n_pblk) return;  // whole workgroup
   const int pblk = L / n_tiles;
   const int2 tj = tiles[L % n_tiles];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int I0 = tj.x * FC_TILE, J0 = tj.y * FC_TILE;
-  const size_t NP = (size_t)N * pitch;
-  const int p0 = pblk * FC_PB;
+  const size_t SN = (size_t)N * ld;  // one sample, rows of ld values
+  const int p0 = pblk * PB;
   // operand roles of this lane: sample k of the 4, row / column node l % 16
   const int ok = lane >> 4, on = lane & 15;
-  // staging roles: instance sl of the block; half-wave g = 2 w + sh stages
-  // FC_RG node rows of sample g / FC_GS
-  const int sl = lane & 31, sh = lane >> 5;
-  const int sg = 2 * wave + sh;
-  // the sample a wave stages is the same for its two halves (FC_GS is
-  // even): sk = wave / 2
-  const int sk = __builtin_amdgcn_readfirstlane(sg / FC_GS);
-  const int sr0 = (sg % FC_GS) * FC_RG;
+  // staging roles: instance sl of the block; wave w stages, of sample w / 2,
+  // node rows 16 (w % 2) .. + 15 of the tile's 32, RG to a lane group
+  const int sl = lane % PB, sg = lane / PB;
+  const int sk = wave / 2;
+  const int sr0 = 16 * (wave & 1) + sg * RG;
   const int snode0 = sr0 < FC_TILE ? I0 + sr0 : J0 + sr0 - FC_TILE;
   // the shifts of the tile's 32 nodes, staged once
 #pragma unroll
-  for (int t = 0; t < 16 / FC_NW; ++t) {
-    const int r = sg * (16 / FC_NW) + t;
+  for (int t = 0; t < 32 * PB / (64 * FC_NW); ++t) {
+    const int r = (threadIdx.x + 64 * FC_NW * t) / PB;
     const int node = r < FC_TILE ? I0 + r : J0 + r - FC_TILE;
     xs[sl * FC_XS + FC_KC * 48 + r] =
         node < N ? shift[(size_t)node * pitch + p0 + sl] : 0.0f;
@@ -644,35 +671,37 @@ k_fc_update(const float *__restrict__ samples, int slots, long long first,
   __syncthreads();  // the staged shifts are read next
   // the shifts of the operand nodes (row node on of the A operand, column
   // node on of the B operand) of each of the wave's instances, in FP64
-  double sa[FC_IW], sb[FC_IW];
+  double sa[IW], sb[IW];
 #pragma unroll
-  for (int q = 0; q < FC_IW; ++q) {
-    const float *sq = xs + (FC_IW * wave + q) * FC_XS + FC_KC * 48 + on;
+  for (int q = 0; q < IW; ++q) {
+    const float *sq = xs + (IW * wave + q) * FC_XS + FC_KC * 48 + on;
     sa[q] = (double)sq[0];
     sb[q] = (double)sq[16];
   }
-  fc_d4 acc[FC_IW];
+  fc_d4 acc[IW];
 #pragma unroll
-  for (int q = 0; q < FC_IW; ++q) acc[q] = fc_d4{0.0, 0.0, 0.0, 0.0};
+  for (int q = 0; q < IW; ++q) acc[q] = fc_d4{0.0, 0.0, 0.0, 0.0};
   const int slot0 = (int)(first % slots);
   // this lane's element of node row snode0 + t of a sample: 32-bit byte
   // offsets from the sample's base (the host checks N pitch 4 < 4 GiB)
   // through a buffer descriptor whose range is one sample, so that the
-  // padding rows past N read as 0 (a buffer load past the range returns 0)
+  // padding rows past N read as 0 (a buffer load past the range returns 0).
+  // Lanes past the last instance of rows of ld < pitch read the next row's
+  // values: such instances are M2's padding.
   const unsigned eo0 =
-      ((unsigned)snode0 * (unsigned)pitch + (unsigned)(p0 + sl)) * 4u;
-  const unsigned rowb = (unsigned)pitch * 4u;
-  const int nrec = (int)((unsigned)N * (unsigned)pitch * 4u);
-  float pre[FC_RG];
+      ((unsigned)snode0 * (unsigned)ld + (unsigned)(p0 + sl)) * 4u;
+  const unsigned rowb = (unsigned)ld * 4u;
+  const int nrec = (int)((unsigned)N * (unsigned)ld * 4u);
+  float pre[RG];
   auto fetch = [&](int k0) {
     if (k0 + sk < count) {  // uniform: one sample per wave
       int slot = slot0 + k0 + sk;
       slot -= slot >= slots ? slots : 0;
       const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<float *>(samples + (size_t)slot * NP), (short)0, nrec,
+          const_cast<float *>(samples + (size_t)slot * SN), (short)0, nrec,
           0x00020000);
 #pragma unroll
-      for (int t = 0; t < FC_RG; ++t)
+      for (int t = 0; t < RG; ++t)
         pre[t] = __builtin_bit_cast(
             float,
             __builtin_amdgcn_raw_buffer_load_b32(r, eo0 + t * rowb, 0, 0));
@@ -681,7 +710,7 @@ k_fc_update(const float *__restrict__ samples, int slots, long long first,
       // d is exactly 0 (as for the padding nodes past N, whose values and
       // shifts are both staged as 0)
 #pragma unroll
-      for (int t = 0; t < FC_RG; ++t)
+      for (int t = 0; t < RG; ++t)
         pre[t] = xs[sl * FC_XS + FC_KC * 48 + sr0 + t];
     }
   };
@@ -689,20 +718,20 @@ k_fc_update(const float *__restrict__ samples, int slots, long long first,
   for (int k0 = 0; k0 < count; k0 += FC_KC) {
     __syncthreads();  // the previous samples are consumed
 #pragma unroll
-    for (int t = 0; t < FC_RG; ++t)
+    for (int t = 0; t < RG; ++t)
       xs[sl * FC_XS + sk * 48 + sr0 + t] = pre[t];
     __syncthreads();
     if (k0 + FC_KC < count) fetch(k0 + FC_KC);  // in flight meanwhile
     // all the wave's operand reads first, then the products
-    float xa[FC_IW], xb[FC_IW];
+    float xa[IW], xb[IW];
 #pragma unroll
-    for (int q = 0; q < FC_IW; ++q) {
-      const float *xq = xs + (FC_IW * wave + q) * FC_XS + ok * 48 + on;
+    for (int q = 0; q < IW; ++q) {
+      const float *xq = xs + (IW * wave + q) * FC_XS + ok * 48 + on;
       xa[q] = xq[0];
       xb[q] = xq[16];
     }
 #pragma unroll
-    for (int q = 0; q < FC_IW; ++q) {
+    for (int q = 0; q < IW; ++q) {
       const double a = (double)xa[q] - sa[q];
       const double b = (double)xb[q] - sb[q];
       acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[q], 0, 0, 0);
@@ -711,30 +740,35 @@ k_fc_update(const float *__restrict__ samples, int slots, long long first,
   // merge: M2_ij += C_ij - S1_i S1_j / m + u_i u_j n_a m / (n_a + m)
   const double m = (double)count;
   const double wgt = n_prev * m / (n_prev + m);
-  double *tb = reinterpret_cast<double *>(xs);  // [64 pairs][33] doubles
+  double *tb = reinterpret_cast<double *>(xs);  // [64 pairs][PB + 1]
   const bool diag = tj.x == tj.y;
+  const bool first_merge = __builtin_amdgcn_readfirstlane(n_prev == 0.0);
   const int p = p0 + sl;
 #pragma unroll
   for (int pass = 0; pass < 4; ++pass) {
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < FC_IW; ++q)
-      tb[lane * 33 + FC_IW * wave + q] = acc[q][pass];
+    for (int q = 0; q < IW; ++q)
+      tb[lane * (PB + 1) + IW * wave + q] = acc[q][pass];
     __syncthreads();
-    // half-wave g: pairs of the pass 32 g / FC_NW .., lanes = instances
+    // lanes = instances
 #pragma unroll
-    for (int e = 0; e < 32 / FC_NW; ++e) {
-      const int pl = (32 / FC_NW) * sg + e;
+    for (int e = 0; e < PB / FC_NW; ++e) {
+      const int pl = (threadIdx.x + 64 * FC_NW * e) / PB;
       const int pi = 64 * pass + pl;
       const int i = I0 + (pi >> 4), j = J0 + (pi & 15);
       if (i >= N || j >= N || (diag && j < i)) continue;
-      const double c = tb[pl * 33 + sl];
+      const double c = tb[pl * (PB + 1) + sl];
       const double s1i = s1[(size_t)i * pitch + p];
       const double s1j = s1[(size_t)j * pitch + p];
       const double ui = u[(size_t)i * pitch + p];
       const double uj = u[(size_t)j * pitch + p];
+      const double v = c - s1i * s1j / m + ui * uj * wgt;
       double *dst = m2 + tri_index(i, j, N) * pitch + p;
-      *dst = *dst + (c - s1i * s1j / m + ui * uj * wgt);
+      if (first_merge)
+        *dst = v;
+      else
+        *dst = *dst + v;
     }
   }
 }
@@ -746,7 +780,82 @@ __global__ void k_fc_mean(int N, int pitch, int count, double n_prev,
   const int p = blockIdx.x * 64 + threadIdx.x;
   const size_t ip = (size_t)blockIdx.y * pitch + p;
   const double m = (double)count;
-  mean[ip] = mean[ip] + u[ip] * (m / (n_prev + m));
+  const double ma = n_prev > 0.0 ? mean[ip] : 0.0;
+  mean[ip] = ma + u[ip] * (m / (n_prev + m));
+}
+
+// Tiles (I, J), I <= J, of the upper triangle in super-tile order: thread k
+// finds its tile by skipping whole super-tiles.
+#define FC_ST 8   // tiles per super-tile edge (rows kept in one XCD's L2)
+__global__ void k_fc_tile_table(int T, int n_tiles, int2 *__restrict__ t) {
+  int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n_tiles) return;
+  int2 *dst = t + k;
+  const int TS = (T + FC_ST - 1) / FC_ST;
+  for (int si = 0; si < TS; ++si) {
+    const int ni = min(T - si * FC_ST, FC_ST);
+    for (int sj = si; sj < TS; ++sj) {
+      const int nj = min(T - sj * FC_ST, FC_ST);
+      const int here = si == sj ? ni * (ni + 1) / 2 : ni * nj;
+      if (k >= here) {
+        k -= here;
+        continue;
+      }
+      int i = 0;
+      if (si == sj)
+        for (; k >= ni - i; ++i) k -= ni - i;
+      else
+        i = k / nj, k -= i * nj;
+      *dst = make_int2(si * FC_ST + i,
+                       si == sj ? si * FC_ST + i + k : sj * FC_ST + k);
+      return;
+    }
+  }
+}
+
+// The tiles and the instances per workgroup of a merge of N nodes.  Measured,
+// us for 32 / 16 instances: 21 tiles x 2 blocks of 32 (84 nodes, P = 64, 500
+// samples) 81 / 59, 91 x 4 35 / 27, 28 x 22 97 / 83, 21 x 32 166 / 160, 190 x
+// 16 168 / 163, 21 x 128 (P = 4096, 2000 samples) 2133 / 3344, 2016 x 32 (N =
+// 998, 255 samples) 7255 / 8931.
+struct fc_shape {
+  int pb, T, n_tiles;
+};
+static fc_shape fc_shape_of(int N, int pitch) {
+  fc_shape f;
+  f.T = (N + FC_TILE - 1) / FC_TILE;
+  f.n_tiles = f.T * (f.T + 1) / 2;
+  f.pb = (long long)f.n_tiles * (pitch / 32) < 1024 ? 16 : 32;
+  return f;
+}
+
+static void fc_tile_table(hipStream_t st, const fc_shape &f, int2 *tiles) {
+  hipLaunchKernelGGL(k_fc_tile_table, dim3((f.n_tiles + 255) / 256), dim3(256),
+                     0, st, f.T, f.n_tiles, tiles);
+}
+
+// whether the merge's grid fits a launch
+static bool fc_fits(const fc_shape &f, int pitch) {
+  return (unsigned long long)f.n_tiles * (pitch / f.pb) < (1ull << 31) - 8;
+}
+
+// merge a block of samples, rows of ld >= the instances in use, into m2
+// (shift, s1: work buffers of f32 and f64 [N][pitch]; u is left for
+// k_fc_mean)
+static void fc_merge(hipStream_t st, const fc_shape &f, const float *samples,
+                     int ld, int slots, long long first, int count, int N,
+                     int pitch, double n_prev, const int2 *tiles,
+                     const double *mean, float *shift, double *s1, double *u,
+                     double *m2) {
+  const unsigned nb = pitch / f.pb;
+  const unsigned nwg = (unsigned)((f.n_tiles * nb + 7) / 8 * 8);
+  hipLaunchKernelGGL(k_fc_prep, dim3(pitch / 64, N), dim3(256), 0, st, samples,
+                     ld, slots, first, count, N, pitch, n_prev, mean, shift,
+                     s1, u);
+  auto update = f.pb == 16 ? k_fc_update<16> : k_fc_update<32>;
+  hipLaunchKernelGGL(update, dim3(nwg), dim3(64 * FC_NW), 0, st, samples,
+                     slots, first, count, N, pitch, n_prev, ld, tiles,
+                     f.n_tiles, (int)nb, shift, s1, u, m2);
 }
 
 // corr_ij = M2_ij / sqrt(M2_ii M2_jj) (metric.py:111-139; the 1/n of the
@@ -844,15 +953,6 @@ static int fill_f32(tvbx_sim *s, DevBuf &b, float v) {
   if (!n) return TVBX_OK;
   hipLaunchKernelGGL(k_fill_f32, dim3(grid1d(n, 256)), dim3(256), 0,
                      s->ctx->stream, (float *)b.p, n, v);
-  HIPCHK(hipGetLastError());
-  return TVBX_OK;
-}
-
-static int fill_f64(tvbx_sim *s, DevBuf &b, double v) {
-  size_t n = b.bytes / 8;
-  if (!n) return TVBX_OK;
-  hipLaunchKernelGGL(k_fill_f64, dim3(grid1d(n, 256)), dim3(256), 0,
-                     s->ctx->stream, (double *)b.p, n, v);
   HIPCHK(hipGetLastError());
   return TVBX_OK;
 }
@@ -1110,10 +1210,6 @@ extern "C" int tvbx_sim_create(tvbx_ctx *c, tvbx_module *m,
       DevBuf head{s->bold_state.p, NP * 4};
       rc = fill_f32(s, head, 0.0f);
     }
-  }
-  if (rc == TVBX_OK && d.fc) {
-    rc = fill_f64(s, s->fc_mean, 0.0);
-    if (rc == TVBX_OK) rc = fill_f64(s, s->fc_m2, 0.0);
   }
   if (rc == TVBX_OK) {
     hipError_t e = hipStreamSynchronize(c->stream);
@@ -1556,66 +1652,33 @@ extern "C" int tvbx_sim_set_noise(tvbx_sim *s, int mode,
   return TVBX_OK;
 }
 
-// tiles (I, J), I <= J, of the upper triangle in super-tile order
-static std::vector<int> fc_tile_order(int T) {
-  std::vector<int> t;
-  const int TS = (T + FC_ST - 1) / FC_ST;
-  for (int si = 0; si < TS; ++si)
-    for (int sj = si; sj < TS; ++sj)
-      for (int I = si * FC_ST; I < std::min(T, si * FC_ST + FC_ST); ++I)
-        for (int J = std::max(I, sj * FC_ST);
-             J < std::min(T, sj * FC_ST + FC_ST); ++J) {
-          t.push_back(I);
-          t.push_back(J);
-        }
-  return t;
-}
-
 static int fc_flush(tvbx_sim *s) {
   const tvbx_sim_desc &d = s->d;
   long long pending = s->samples_made - s->samples_used;
   if (!d.fc || pending <= 0) return TVBX_OK;
   const int N = d.n_node;
-  const int T = (N + FC_TILE - 1) / FC_TILE;
-  const int n_tiles = T * (T + 1) / 2;
-  int rc = TVBX_OK;
-  if (!s->fc_tiles.p) {
-    std::vector<int> t = fc_tile_order(T);
-    rc = dalloc(s->fc_tiles, t.size() * 4);
-    if (rc != TVBX_OK) return rc;
-    HIPCHK(hipMemcpyAsync(s->fc_tiles.p, t.data(), t.size() * 4,
-                          hipMemcpyHostToDevice, s->ctx->stream));
-    HIPCHK(hipStreamSynchronize(s->ctx->stream));
-  }
-  rc = dalloc(s->fc_shift, s->NP * 4);
-  if (rc == TVBX_OK) rc = dalloc(s->fc_s1, s->NP * 8);
-  if (rc == TVBX_OK) rc = dalloc(s->fc_u, s->NP * 8);
-  if (rc != TVBX_OK) return rc;
-  const long long first = (s->sample_base + s->samples_used) % d.sample_slots;
-  const double n_prev = (double)s->samples_used;
-  const int n_pblk = s->pitch / 64;
-  const int n_fblk = s->pitch / FC_PB;  // instance blocks of the merge
-  hipLaunchKernelGGL(k_fc_prep, dim3(n_pblk, N), dim3(64), 0, s->ctx->stream,
-                     (const float *)s->samples.p, d.sample_slots, first,
-                     (int)pending, N, s->pitch, n_prev,
-                     (const double *)s->fc_mean.p, (float *)s->fc_shift.p,
-                     (double *)s->fc_s1.p, (double *)s->fc_u.p);
-  HIPCHK(hipGetLastError());
-  const unsigned long long nwg =
-      ((unsigned long long)n_tiles * n_fblk + 7) / 8 * 8;
-  CHECK(nwg < (1ull << 31), "FC problem too large for one launch");
+  const fc_shape f = fc_shape_of(N, s->pitch);
+  hipStream_t st = s->ctx->stream;
+  CHECK(fc_fits(f, s->pitch), "FC problem too large for one launch");
   CHECK((unsigned long long)N * s->pitch * 4ull < (1ull << 32),
         "one monitor sample must stay under 4 GiB for the FC merge");
-  hipLaunchKernelGGL(k_fc_update, dim3((unsigned)nwg), dim3(64 * FC_NW), 0,
-                     s->ctx->stream, (const float *)s->samples.p,
-                     d.sample_slots, first, (int)pending, N, s->pitch, n_prev,
-                     (const int2 *)s->fc_tiles.p, n_tiles, n_fblk,
-                     (const float *)s->fc_shift.p, (const double *)s->fc_s1.p,
-                     (const double *)s->fc_u.p, (double *)s->fc_m2.p);
-  HIPCHK(hipGetLastError());
-  hipLaunchKernelGGL(k_fc_mean, dim3(n_pblk, N), dim3(64), 0, s->ctx->stream,
-                     N, s->pitch, (int)pending, n_prev,
-                     (const double *)s->fc_u.p, (double *)s->fc_mean.p);
+  if (!s->fc_tiles.p) {
+    int rc = dalloc(s->fc_tiles, (size_t)f.n_tiles * 8);
+    if (rc == TVBX_OK) rc = dalloc(s->fc_shift, s->NP * 4);
+    if (rc == TVBX_OK) rc = dalloc(s->fc_s1, s->NP * 8);
+    if (rc == TVBX_OK) rc = dalloc(s->fc_u, s->NP * 8);
+    if (rc != TVBX_OK) return rc;
+    fc_tile_table(st, f, (int2 *)s->fc_tiles.p);
+  }
+  const long long first = (s->sample_base + s->samples_used) % d.sample_slots;
+  const double n_prev = (double)s->samples_used;
+  fc_merge(st, f, (const float *)s->samples.p,
+           s->smp_ld ? s->smp_ld : s->pitch, d.sample_slots, first, (int)pending, N, s->pitch, n_prev, (const int2 *)s->fc_tiles.p,
+           (const double *)s->fc_mean.p, (float *)s->fc_shift.p,
+           (double *)s->fc_s1.p, (double *)s->fc_u.p, (double *)s->fc_m2.p);
+  hipLaunchKernelGGL(k_fc_mean, dim3(s->pitch / 64, N), dim3(64), 0, st, N,
+                     s->pitch, (int)pending, n_prev, (const double *)s->fc_u.p,
+                     (double *)s->fc_mean.p);
   HIPCHK(hipGetLastError());
   s->samples_used = s->samples_made;
   return TVBX_OK;
@@ -2095,15 +2158,12 @@ extern "C" int tvbx_sim_logp(tvbx_sim *s, const float *traj,
 
 extern "C" int tvbx_sim_fc_reset(tvbx_sim *s) {
   CHECK(s && s->d.fc, "sim created without fc");
-  HIPCHK(hipSetDevice(s->ctx->device));
-  int rc = fill_f64(s, s->fc_mean, 0.0);
-  if (rc == TVBX_OK) rc = fill_f64(s, s->fc_m2, 0.0);
-  s->samples_used = s->samples_made;
-  // samples folded from now on start a fresh accumulation
+  // samples folded from now on start a fresh accumulation: the next merge,
+  // its first, writes the co-moments and means without reading them
   s->sample_base += s->samples_made;
   s->samples_made = 0;
   s->samples_used = 0;
-  return rc;
+  return TVBX_OK;
 }
 
 extern "C" int tvbx_sim_get_flags(tvbx_sim *s, uint32_t *flags) {
@@ -2171,13 +2231,16 @@ extern "C" int tvbx_corr(tvbx_ctx *c, const float *samples, long long n,
   s.pitch = (P + 63) / 64 * 64;
   s.NP = (size_t)N * s.pitch;
   const size_t tri = (size_t)N * (N + 1) / 2;
-  int rc = dalloc(s.samples, (size_t)n * s.NP * 4);
+  const size_t smp = (size_t)n * N * P * 4;
+  s.smp_ld = P;  // the rows as they are
+  int rc = dalloc(s.samples, smp);
   if (rc == TVBX_OK) rc = dalloc(s.fc_mean, s.NP * 8);
   if (rc == TVBX_OK) rc = dalloc(s.fc_m2, tri * s.pitch * 8);
-  if (rc == TVBX_OK) rc = fill_f32(&s, s.samples, 0.0f);
-  if (rc == TVBX_OK) rc = fill_f64(&s, s.fc_mean, 0.0);
-  if (rc == TVBX_OK) rc = fill_f64(&s, s.fc_m2, 0.0);
-  if (rc == TVBX_OK) rc = up2d(&s, s.samples.p, samples, (size_t)n * N);
+  hipError_t e = hipSuccess;
+  if (rc == TVBX_OK)
+    e = hipMemcpyAsync(s.samples.p, samples, smp, hipMemcpyDefault, c->stream);
+  if (rc == TVBX_OK && e != hipSuccess)
+    rc = fail(TVBX_E_HIP, "tvbx_corr: %s", hipGetErrorString(e));
   if (rc == TVBX_OK) {
     s.samples_made = n;
     rc = tvbx_sim_fc(&s, 0, P, corr, nullptr);
@@ -2190,32 +2253,6 @@ extern "C" int tvbx_corr(tvbx_ctx *c, const float *samples, long long n,
 }
 
 // ------------------------------------------------- allocation-free FC
-// The tile table of k_fc_update in super-tile order (fc_tile_order), built
-// on the device by one thread.
-__global__ void k_fc_tile_table(int T, int2 *__restrict__ t) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  int k = 0;
-  const int TS = (T + FC_ST - 1) / FC_ST;
-  for (int si = 0; si < TS; ++si)
-    for (int sj = si; sj < TS; ++sj)
-      for (int I = si * FC_ST; I < min(T, si * FC_ST + FC_ST); ++I)
-        for (int J = max(I, sj * FC_ST); J < min(T, sj * FC_ST + FC_ST); ++J)
-          t[k++] = make_int2(I, J);
-}
-
-// rows [n * N][P] -> [n * N][pitch], the padding lanes zero
-__global__ void k_pitch_rows(const float *__restrict__ in, size_t rows, int P,
-                             int pitch, float *__restrict__ out) {
-  const size_t total = rows * (size_t)pitch;
-  size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; k < total; k += stride) {
-    const size_t r = k / pitch;
-    const int p = (int)(k - r * pitch);
-    out[k] = p < P ? in[r * P + p] : 0.0f;
-  }
-}
-
 // tvbx_corr on device memory with every intermediate in the device's
 // scratch array: no allocation, no host copy, no synchronisation.
 extern "C" int tvbx_corr_noalloc(tvbx_ctx *c, const float *samples,
@@ -2229,10 +2266,7 @@ extern "C" int tvbx_corr_noalloc(tvbx_ctx *c, const float *samples,
   const int pitch = (P + 63) / 64 * 64;
   const size_t NP = (size_t)N * pitch;
   const size_t tri = (size_t)N * (N + 1) / 2;
-  const int T = (N + FC_TILE - 1) / FC_TILE;
-  const int n_tiles = T * (T + 1) / 2;
-  const int n_fblk = pitch / FC_PB;
-  const bool stage = pitch != P;  // the FC kernels read [n][N][pitch]
+  const fc_shape f = fc_shape_of(N, pitch);
   // the scratch's pieces, each 256-byte aligned
   size_t used = 0;
   auto take = [&used](size_t bytes) {
@@ -2242,15 +2276,18 @@ extern "C" int tvbx_corr_noalloc(tvbx_ctx *c, const float *samples,
   };
   const size_t o_m2 = take(tri * pitch * 8), o_mean = take(NP * 8),
                o_s1 = take(NP * 8), o_u = take(NP * 8),
-               o_shift = take(NP * 4), o_tiles = take((size_t)n_tiles * 8),
-               o_smp = stage ? take((size_t)n * NP * 4) : 0;
+               o_shift = take(NP * 4),
+               o_tiles = take((size_t)f.n_tiles * 8);
+  // the limit on the sizes counts a padded copy of ragged samples too,
+  // which the merge does without
+  if (pitch != P) take((size_t)n * NP * 4);
   CHECK(used <= TVBX_SCRATCH_BYTES,
         "tvbx_corr_noalloc: n=%lld, N=%d, P=%d need %zu bytes of device "
         "scratch; the limit is %zu bytes",
         n, N, P, used, (size_t)TVBX_SCRATCH_BYTES);
-  const unsigned long long nwg =
-      ((unsigned long long)n_tiles * n_fblk + 7) / 8 * 8;
-  CHECK(nwg < (1ull << 31), "FC problem too large for one launch");
+  CHECK(fc_fits(f, pitch), "FC problem too large for one launch");
+  CHECK((unsigned long long)N * pitch * 4ull < (1ull << 32),
+        "one sample must stay under 4 GiB for the FC merge");
   HIPCHK(hipSetDevice(c->device));
   char *base = static_cast<char *>(g_scratch_ptr[c->device]);
   double *m2 = reinterpret_cast<double *>(base + o_m2);
@@ -2259,31 +2296,12 @@ extern "C" int tvbx_corr_noalloc(tvbx_ctx *c, const float *samples,
   double *u = reinterpret_cast<double *>(base + o_u);
   float *shift = reinterpret_cast<float *>(base + o_shift);
   int2 *tiles = reinterpret_cast<int2 *>(base + o_tiles);
-  const float *smp = samples;
   hipStream_t st = c->stream;
-  // the scratch keeps the previous call's contents: the co-moments and
-  // means start from zero (fill kernels, so the call can be captured)
-  hipLaunchKernelGGL(k_fill_f64, dim3(grid1d(tri * pitch, 256)), dim3(256),
-                     0, st, m2, tri * pitch, 0.0);
-  hipLaunchKernelGGL(k_fill_f64, dim3(grid1d(NP, 256)), dim3(256), 0, st,
-                     mean, NP, 0.0);
-  hipLaunchKernelGGL(k_fc_tile_table, dim3(1), dim3(64), 0, st, T, tiles);
-  if (stage) {
-    float *sp = reinterpret_cast<float *>(base + o_smp);
-    hipLaunchKernelGGL(k_pitch_rows, dim3(grid1d((size_t)n * NP, 256)),
-                       dim3(256), 0, st, samples, (size_t)n * N, P, pitch,
-                       sp);
-    smp = sp;
-  }
-  hipLaunchKernelGGL(k_fc_prep, dim3(pitch / 64, N), dim3(64), 0, st, smp,
-                     (int)n, 0ll, (int)n, N, pitch, 0.0, mean, shift, s1, u);
-  CHECK((unsigned long long)N * pitch * 4ull < (1ull << 32),
-        "one sample must stay under 4 GiB for the FC merge");
-  hipLaunchKernelGGL(k_fc_update, dim3((unsigned)nwg), dim3(64 * FC_NW), 0,
-                     st, smp, (int)n, 0ll, (int)n, N, pitch, 0.0, tiles,
-                     n_tiles, n_fblk, shift, s1, u, m2);
-  hipLaunchKernelGGL(k_fc_mean, dim3(pitch / 64, N), dim3(64), 0, st, N,
-                     pitch, (int)n, 0.0, u, mean);
+  // the scratch keeps the previous call's contents; a first merge reads
+  // neither the co-moments nor the means
+  fc_tile_table(st, f, tiles);
+  fc_merge(st, f, samples, P, (int)n, 0ll, (int)n, N, pitch, 0.0, tiles, mean,
+           shift, s1, u, m2);
   hipLaunchKernelGGL(k_fc_corr_full, dim3((P + 63) / 64, N), dim3(64), 0, st,
                      m2, N, pitch, 0, P, corr);
   HIPCHK(hipGetLastError());
@@ -2579,56 +2597,33 @@ extern "C" int tvbx_fc_loss(tvbx_ctx *c, const float *samples, long long n,
   const int pitch = (P + 63) / 64 * 64;
   const size_t NP = (size_t)N * pitch;
   const size_t tri = (size_t)N * (N + 1) / 2;
-  const int T = (N + FC_TILE - 1) / FC_TILE;
-  const int n_tiles = T * (T + 1) / 2;
-  const int n_fblk = pitch / FC_PB;
-  const bool stage = pitch != P;  // the FC kernels read [n][N][pitch]
+  const fc_shape f = fc_shape_of(N, pitch);
   size_t used = 0;
   auto take = [&used](size_t bytes) {
     const size_t o = used;
     used += (bytes + 255) / 256 * 256;
     return o;
   };
-  const size_t o_m2 = take(tri * pitch * 8), o_mean = take(NP * 8),
-               o_s1 = take(NP * 8), o_u = take(NP * 8),
-               o_shift = take(NP * 4), o_rs = take(NP * 8),
+  const size_t o_m2 = take(tri * pitch * 8), o_s1 = take(NP * 8),
+               o_u = take(NP * 8), o_shift = take(NP * 4), o_rs = take(NP * 8),
                o_part = take((size_t)((N + FL_NW - 1) / FL_NW) * pitch * 40),
-               o_tiles = take((size_t)n_tiles * 8),
-               o_smp = stage ? take((size_t)n * NP * 4) : 0;
+               o_tiles = take((size_t)f.n_tiles * 8);
+  CHECK(fc_fits(f, pitch), "FC problem too large for one launch");
+  CHECK((unsigned long long)N * pitch * 4ull < (1ull << 32),
+        "one sample must stay under 4 GiB for the FC merge");
   int rc = ctx_work(c, used);
   if (rc != TVBX_OK) return rc;
   char *base = static_cast<char *>(c->work);
   double *m2 = reinterpret_cast<double *>(base + o_m2);
-  double *dmean = reinterpret_cast<double *>(base + o_mean);
   double *s1 = reinterpret_cast<double *>(base + o_s1);
   double *u = reinterpret_cast<double *>(base + o_u);
   float *shift = reinterpret_cast<float *>(base + o_shift);
   double *rs = reinterpret_cast<double *>(base + o_rs);
   int2 *tiles = reinterpret_cast<int2 *>(base + o_tiles);
-  const unsigned long long nwg =
-      ((unsigned long long)n_tiles * n_fblk + 7) / 8 * 8;
-  CHECK(nwg < (1ull << 31), "FC problem too large for one launch");
   hipStream_t st = c->stream;
-  const float *smp = samples;
-  hipLaunchKernelGGL(k_fill_f64, dim3(grid1d(tri * pitch, 256)), dim3(256),
-                     0, st, m2, tri * pitch, 0.0);
-  hipLaunchKernelGGL(k_fill_f64, dim3(grid1d(NP, 256)), dim3(256), 0, st,
-                     dmean, NP, 0.0);
-  hipLaunchKernelGGL(k_fc_tile_table, dim3(1), dim3(64), 0, st, T, tiles);
-  if (stage) {
-    float *sp = reinterpret_cast<float *>(base + o_smp);
-    hipLaunchKernelGGL(k_pitch_rows, dim3(grid1d((size_t)n * NP, 256)),
-                       dim3(256), 0, st, samples, (size_t)n * N, P, pitch,
-                       sp);
-    smp = sp;
-  }
-  hipLaunchKernelGGL(k_fc_prep, dim3(pitch / 64, N), dim3(64), 0, st, smp,
-                     (int)n, 0ll, (int)n, N, pitch, 0.0, dmean, shift, s1, u);
-  CHECK((unsigned long long)N * pitch * 4ull < (1ull << 32),
-        "one sample must stay under 4 GiB for the FC merge");
-  hipLaunchKernelGGL(k_fc_update, dim3((unsigned)nwg), dim3(64 * FC_NW), 0,
-                     st, smp, (int)n, 0ll, (int)n, N, pitch, 0.0, tiles,
-                     n_tiles, n_fblk, shift, s1, u, m2);
+  fc_tile_table(st, f, tiles);
+  fc_merge(st, f, samples, P, (int)n, 0ll, (int)n, N, pitch, 0.0, tiles,
+           nullptr, shift, s1, u, m2);
   double *part = reinterpret_cast<double *>(base + o_part);
   const dim3 rows(pitch / 64, (N + FL_NW - 1) / FL_NW);
   hipLaunchKernelGGL(k_fl_node, dim3(pitch / 64, N), dim3(64), 0, st, m2, N,

@@ -140,8 +140,8 @@ struct tvbx_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipDeviceProp_t prop{};
-  // device workspace of the context-level calls (tvbx_fc_loss), grown on
-  // demand and kept until tvbx_ctx_destroy
+  // device workspace of the calls that leave nothing in it (tvbx_fc_loss,
+  // tvbx_sim_fc_sc_error), grown on demand and kept until tvbx_ctx_destroy
   void *work = nullptr;
   size_t work_bytes = 0;
 };
@@ -860,52 +860,95 @@ static void fc_merge(hipStream_t st, const fc_shape &f, const float *samples,
 
 // corr_ij = M2_ij / sqrt(M2_ii M2_jj) (metric.py:111-139; the 1/n of the
 // covariance cancels) for instances p0 .. p0 + np - 1, both triangles, into
-// corr [np][N][N].  grid (ceil(np / 64), N), block 64.
-__global__ void k_fc_corr_full(const double *__restrict__ m2, int N,
-                               int pitch, int p0, int np,
-                               float *__restrict__ corr) {
-  const int q = blockIdx.x * 64 + threadIdx.x;
-  const int i = blockIdx.y;
-  if (q >= np) return;
-  const int p = p0 + q;
-  const double mii = m2[tri_index(i, i, N) * pitch + p];
-  float *cq = corr + (size_t)q * N * N;
-  for (int j = i; j < N; ++j) {
-    const double mjj = m2[tri_index(j, j, N) * pitch + p];
-    const float v =
-        (float)(m2[tri_index(i, j, N) * pitch + p] / sqrt(mii * mjj));
-    cq[(size_t)i * N + j] = v;
-    cq[(size_t)j * N + i] = v;
+// corr [np][N][N].  M2 is instance-innermost and corr instance-outermost: a
+// workgroup forms a 16 x 16 tile of pairs (I <= J) for FK_PB instances with
+// lanes = instances, and writes the tile and its mirror through LDS in runs
+// of 16 values (one lane per instance storing value by value along N^2 took
+// 110 us for 700 instances of 116 nodes, 46 MB read and 38 MB written; 30
+// us this way).  grid (ceil(np / FK_PB), T, T), block 256.
+#define FK_PB 32
+__global__ void __launch_bounds__(256)
+k_fc_corr_full(const double *__restrict__ m2, int N, int pitch, int p0,
+               int np, float *__restrict__ corr) {
+  __shared__ float tile[FK_PB][16 * 16 + 1];
+  const int I0 = blockIdx.z * 16, J0 = blockIdx.y * 16;
+  if (J0 < I0) return;  // whole workgroup
+  const int q0 = blockIdx.x * FK_PB;
+  const int ql = threadIdx.x % FK_PB, g = threadIdx.x / FK_PB;
+  const int p = p0 + min(q0 + ql, np - 1);
+  const int nj = min(16, N - J0);
+  for (int i = I0 + g; i < min(I0 + 16, N); i += 256 / FK_PB) {
+    const double mii = m2[tri_index(i, i, N) * pitch + p];
+    const int jb = I0 == J0 ? i - I0 : 0;
+#pragma unroll 4
+    for (int jl = jb; jl < nj; ++jl) {
+      const int j = J0 + jl;
+      const double mjj = m2[tri_index(j, j, N) * pitch + p];
+      const float v =
+          (float)(m2[tri_index(i, j, N) * pitch + p] / sqrt(mii * mjj));
+      tile[ql][(i - I0) * 16 + jl] = v;
+      if (I0 == J0) tile[ql][jl * 16 + i - I0] = v;
+    }
   }
+  __syncthreads();
+  const int nq = min(FK_PB, np - q0);
+  const int c = threadIdx.x & 15;
+  for (int e = threadIdx.x >> 4; e < nq * 16; e += 16) {
+    const int q = e >> 4, r = e & 15;
+    float *cq = corr + (size_t)(q0 + q) * N * N;
+    if (I0 + r < N && J0 + c < N)
+      cq[(size_t)(I0 + r) * N + J0 + c] = tile[q][r * 16 + c];
+    if (I0 != J0 && J0 + r < N && I0 + c < N)
+      cq[(size_t)(J0 + r) * N + I0 + c] = tile[q][c * 16 + r];
+  }
+}
+
+static void fc_corr(hipStream_t st, const double *m2, int N, int pitch, int p0,
+                    int np, float *corr) {
+  const unsigned T = (N + 15) / 16;
+  hipLaunchKernelGGL(k_fc_corr_full, dim3((np + FK_PB - 1) / FK_PB, T, T),
+                     dim3(256), 0, st, m2, N, pitch, p0, np, corr);
 }
 
 // FC-SC error of row i: part[i][p] = sum over j > i of (corr_ij - sc_ij)^2,
 // corr in FP64 from the co-moments (hackathon.py:74-80 compares
 // numpy.corrcoef, FP64, with the weights over triu_indices(N, 1)).
-// sc_row[j] holds sc_ij of this row as FP64.  grid (pitch / 64, N), block 64.
+// sc [N][N] as the caller gave it.  grid (pitch / 64, N), block 64.
 __global__ void k_fc_sc_row(const double *__restrict__ m2, int N, int pitch,
-                            const double *__restrict__ sc,
+                            const float *__restrict__ sc,
                             double *__restrict__ part) {
   const int p = blockIdx.x * 64 + threadIdx.x;
   const int i = blockIdx.y;
   const double mii = m2[tri_index(i, i, N) * pitch + p];
-  const double *__restrict__ sci = sc + (size_t)i * N;
+  const float *__restrict__ sci = sc + (size_t)i * N;
   double acc = 0.0;
+#pragma unroll 8
   for (int j = i + 1; j < N; ++j) {
     const double mjj = m2[tri_index(j, j, N) * pitch + p];
     const double c = m2[tri_index(i, j, N) * pitch + p] / sqrt(mii * mjj);
-    const double d = c - sci[j];
+    const double d = c - (double)sci[j];
     acc = fma(d, d, acc);
   }
   part[(size_t)i * pitch + p] = acc;
 }
 
-// err[p] = sum over rows i (ascending) of part[i][p].  grid pitch / 64.
-__global__ void k_fc_sc_sum(const double *__restrict__ part, int N, int pitch,
-                            double *__restrict__ err) {
-  const int p = blockIdx.x * 64 + threadIdx.x;
+// err[p] = sum over rows i of part[i][p]: the 16 waves of a workgroup add a
+// sixteenth of the rows each, ascending, then their sums in order (one wave
+// for all rows took 330 us at N = 998).  grid pitch / 64, block 1024.
+__global__ void __launch_bounds__(1024)
+k_fc_sc_sum(const double *__restrict__ part, int N, int pitch,
+            double *__restrict__ err) {
+  __shared__ double red[16 * 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane;
   double acc = 0.0;
-  for (int i = 0; i < N; ++i) acc += part[(size_t)i * pitch + p];
+#pragma unroll 8
+  for (int i = w * N / 16; i < (w + 1) * N / 16; ++i)
+    acc += part[(size_t)i * pitch + p];
+  red[w * 64 + lane] = acc;
+  __syncthreads();
+  if (w) return;
+  for (int k = 1; k < 16; ++k) acc += red[k * 64 + lane];
   err[p] = acc;
 }
 
@@ -941,6 +984,21 @@ static void dfree(DevBuf &b) {
   if (b.p) hipFree(b.p);
   b.p = nullptr;
   b.bytes = 0;
+}
+
+// the context's workspace, at least `bytes` (grown on demand; its contents
+// are a call's own)
+static int ctx_work(tvbx_ctx *c, size_t bytes) {
+  if (c->work && c->work_bytes >= bytes) return TVBX_OK;
+  if (c->work) {
+    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipFree(c->work));
+  }
+  c->work = nullptr;
+  c->work_bytes = 0;
+  HIPCHK(hipMalloc(&c->work, bytes));
+  c->work_bytes = bytes;
+  return TVBX_OK;
 }
 
 static unsigned grid1d(size_t n, int block) {
@@ -1956,9 +2014,8 @@ extern "C" int tvbx_sim_fc(tvbx_sim *s, int p0, int np, float *corr,
   const size_t nn = (size_t)N * N;
   rc = dalloc(s->corr, (size_t)np * nn * 4);
   if (rc != TVBX_OK) return rc;
-  hipLaunchKernelGGL(k_fc_corr_full, dim3((np + 63) / 64, N), dim3(64), 0,
-                     s->ctx->stream, (const double *)s->fc_m2.p, N, s->pitch,
-                     p0, np, (float *)s->corr.p);
+  fc_corr(s->ctx->stream, (const double *)s->fc_m2.p, N, s->pitch, p0, np,
+          (float *)s->corr.p);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(corr, s->corr.p, (size_t)np * nn * 4,
                         hipMemcpyDeviceToHost, s->ctx->stream));
@@ -1979,34 +2036,29 @@ extern "C" int tvbx_sim_fc_sc_error(tvbx_sim *s, const float *sc, int p0,
   if (np == 0) return TVBX_OK;
   CHECK(s->samples_used >= 2, "FC needs at least two samples");
   const int N = d.n_node;
-  std::vector<double> sc64((size_t)N * N);
-  for (size_t k = 0; k < sc64.size(); ++k) sc64[k] = (double)sc[k];
-  DevBuf dsc, part, derr;
-  rc = dalloc(dsc, sc64.size() * 8);
-  if (rc == TVBX_OK) rc = dalloc(part, (size_t)N * s->pitch * 8);
-  if (rc == TVBX_OK) rc = dalloc(derr, (size_t)s->pitch * 8);
-  hipError_t e = hipSuccess;
-  if (rc == TVBX_OK)
-    e = hipMemcpyAsync(dsc.p, sc64.data(), sc64.size() * 8,
-                       hipMemcpyHostToDevice, s->ctx->stream);
-  if (rc == TVBX_OK && e == hipSuccess) {
+  // the context's workspace: sc, one partial per (row, instance), the sums
+  const size_t nn = ((size_t)N * N * 4 + 255) / 256 * 256;
+  rc = ctx_work(s->ctx, nn + ((size_t)N + 1) * s->pitch * 8);
+  if (rc != TVBX_OK) return rc;
+  float *dsc = (float *)s->ctx->work;
+  double *part = (double *)((char *)s->ctx->work + nn);
+  double *derr = part + (size_t)N * s->pitch;
+  hipError_t e = hipMemcpyAsync(dsc, sc, (size_t)N * N * 4,
+                                hipMemcpyHostToDevice, s->ctx->stream);
+  if (e == hipSuccess) {
     hipLaunchKernelGGL(k_fc_sc_row, dim3(s->pitch / 64, N), dim3(64), 0,
                        s->ctx->stream, (const double *)s->fc_m2.p, N, s->pitch,
-                       (const double *)dsc.p, (double *)part.p);
-    hipLaunchKernelGGL(k_fc_sc_sum, dim3(s->pitch / 64), dim3(64), 0,
-                       s->ctx->stream, (const double *)part.p, N, s->pitch,
-                       (double *)derr.p);
+                       dsc, part);
+    hipLaunchKernelGGL(k_fc_sc_sum, dim3(s->pitch / 64), dim3(1024), 0,
+                       s->ctx->stream, part, N, s->pitch, derr);
     e = hipGetLastError();
   }
-  if (rc == TVBX_OK && e == hipSuccess)
-    e = hipMemcpyAsync(err, (const double *)derr.p + p0, (size_t)np * 8,
-                       hipMemcpyDeviceToHost, s->ctx->stream);
-  if (rc == TVBX_OK && e == hipSuccess) e = hipStreamSynchronize(s->ctx->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(err, derr + p0, (size_t)np * 8, hipMemcpyDeviceToHost,
+                       s->ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(s->ctx->stream);
   if (rc == TVBX_OK && e != hipSuccess)
     rc = fail(TVBX_E_HIP, "tvbx_sim_fc_sc_error: %s", hipGetErrorString(e));
-  dfree(dsc);
-  dfree(part);
-  dfree(derr);
   return rc;
 }
 
@@ -2302,8 +2354,7 @@ extern "C" int tvbx_corr_noalloc(tvbx_ctx *c, const float *samples,
   fc_tile_table(st, f, tiles);
   fc_merge(st, f, samples, P, (int)n, 0ll, (int)n, N, pitch, 0.0, tiles, mean,
            shift, s1, u, m2);
-  hipLaunchKernelGGL(k_fc_corr_full, dim3((P + 63) / 64, N), dim3(64), 0, st,
-                     m2, N, pitch, 0, P, corr);
+  fc_corr(st, m2, N, pitch, 0, P, corr);
   HIPCHK(hipGetLastError());
   return TVBX_OK;
 }
@@ -2570,19 +2621,6 @@ k_transpose(const float *__restrict__ in, long long rows, long long cols,
     const long long c = c0 + k, r = r0 + tx;
     if (c < cols && r < rows) out[c * rows + r] = tile[tx][k];
   }
-}
-
-static int ctx_work(tvbx_ctx *c, size_t bytes) {
-  if (c->work && c->work_bytes >= bytes) return TVBX_OK;
-  if (c->work) {
-    HIPCHK(hipStreamSynchronize(c->stream));
-    HIPCHK(hipFree(c->work));
-  }
-  c->work = nullptr;
-  c->work_bytes = 0;
-  HIPCHK(hipMalloc(&c->work, bytes));
-  c->work_bytes = bytes;
-  return TVBX_OK;
 }
 
 extern "C" int tvbx_fc_loss(tvbx_ctx *c, const float *samples, long long n,

@@ -2867,56 +2867,142 @@ struct tvbx_rmap {
   DevBuf members;  // [nnode] vertices by region, ascending within a region
 };
 
-// roi[r][j][p] = sum of node[k][j][p] over the vertices k of region r, added
-// in ascending k from 0 (the reference kernel's order: one pass over k
-// adding into roi[rmap[k]]), so float32 results equal its sequential ones.
-// The loads of RMAP_UNROLL vertices are in flight together and added in
-// order.  grid (nroi * nvar, ceil(n_inst / 64)), block 64.
-#define RMAP_UNROLL 32
-__global__ void __launch_bounds__(64)
+// roi[r][c] = sum of node[k][c] over the vertices k of region r, c one of the
+// row's C = nvar n_inst columns, added in ascending k from 0 (the reference
+// kernel's order: one pass over k adding into roi[rmap[k]]), so float32
+// results equal its sequential ones.
+//   The additions of a column are one serial chain; what can be hidden is the
+// loads' latency.  A workgroup takes a region and up to 64 columns (CP the
+// next power of two).  Wave 0's lanes, one a column, add up a tile of V
+// vertices from LDS (column-major, 4 vertices to a read, the next reads
+// issued ahead of the additions); RM_D groups of RM_G waves take the tiles in
+// turn, so that each has RM_D tiles' time for its loads (RM_V values a
+// thread, the vertex indices of its next tile loaded beside them).  A tile
+// is handed over through one of two LDS buffers at each barrier.  A partial
+// tile is padded with zeros: adding +0 changes no sum that began at +0.
+//   Bound by the chain, 3.1 ns an addition, where the largest region decides
+// (against a wave per region, row and 64 instances with 16 loads in flight):
+// 20,484 vertices in 148 regions, 2 columns, the largest region 1265: 6.1 us
+// (36.4); 173,449 in 57, the largest 19,212: 60 us (518); 515,056 in 400, the
+// largest 9130, 128 columns: 150 us (476), and in even regions, where the
+// reads bind, 67 us, 4.0 TB/s (78).  One group of loads beside the sums
+// instead of RM_D by turns: 7.9, 93 and 287 us.
+// grid (nroi, y, z) with y z >= ceil(C / 64), block RM_T.
+#define RM_D 3
+#define RM_G 4
+#define RM_V 16
+#define RM_T (64 * (1 + RM_D * RM_G))
+template <int CP>
+__global__ void __launch_bounds__(RM_T)
 k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
-              int nvar, int n_inst, const float *__restrict__ node,
+              long long C, const float *__restrict__ node,
               float *__restrict__ roi) {
-  const int rj = blockIdx.x;
-  const int r = rj / nvar, j = rj - r * nvar;
-  const int p = blockIdx.y * 64 + threadIdx.x;
-  const bool on = p < n_inst;
+  constexpr int RV = 64 * RM_G / CP;   // vertices per round of loads
+  constexpr int V = RV * RM_V;         // and per tile
+  constexpr int LD = V + 4;            // LDS row of a column (16-byte aligned)
+  constexpr int B = 8;                 // LDS reads ahead of the additions
+  __shared__ __attribute__((aligned(16))) float tile[2][CP * LD];
+  const int r = blockIdx.x;
+  const long long cb = (long long)blockIdx.z * gridDim.y + blockIdx.y;
+  if (cb * 64 >= C) return;  // whole workgroup
   const int m0 = rptr[r], m1 = rptr[r + 1];
-  const size_t row = (size_t)nvar * n_inst;
-  const float *__restrict__ src = node + (size_t)j * n_inst + (on ? p : 0);
-  float acc = 0.0f;
-  int m = m0;
-  for (; m + RMAP_UNROLL <= m1; m += RMAP_UNROLL) {
-    float v[RMAP_UNROLL];
+  const int nt = (m1 - m0 + V - 1) / V;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wave == 0) {
+    // the sums; lanes past CP or C repeat a column and store nothing
+    const int c = threadIdx.x % CP;
+    float acc = 0.0f;
+    for (int t = 0; t < nt; ++t) {
+      __syncthreads();  // tile t is in buffer t & 1
+      const float4 *__restrict__ t4 =
+          reinterpret_cast<const float4 *>(tile[t & 1] + c * LD);
+      const int n4 = (min(V, m1 - m0 - t * V) + 3) / 4;
+      // two batches of B reads by turns, whole batches (V is a multiple of
+      // 8 B): what lies past the region in the tile is zeros
+      float4 q[2][B];
 #pragma unroll
-    for (int u = 0; u < RMAP_UNROLL; ++u)
-      v[u] = src[(size_t)members[m + u] * row];
+      for (int u = 0; u < B; ++u) q[0][u] = t4[u];
+      for (int x = 0; x < n4; x += 2 * B) {
 #pragma unroll
-    for (int u = 0; u < RMAP_UNROLL; ++u) acc += v[u];
+        for (int h = 0; h < 2; ++h) {
+          const int nx = min(x + (h + 1) * B, V / 4 - B);
+#pragma unroll
+          for (int u = 0; u < B; ++u) q[1 - h][u] = t4[nx + u];
+          __builtin_amdgcn_sched_barrier(0);  // or the reads sink below
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            acc += q[h][u].x;
+            acc += q[h][u].y;
+            acc += q[h][u].z;
+            acc += q[h][u].w;
+          }
+        }
+      }
+    }
+    const long long col = cb * 64 + c;
+    if (threadIdx.x < CP && col < C) roi[(size_t)r * C + col] = acc;
+    return;
   }
-  for (; m < m1; ++m) acc += src[(size_t)members[m] * row];
-  if (on) roi[(size_t)rj * n_inst + p] = acc;
+  // the loads: group g takes tiles g, g + RM_D, ...
+  const int g = (wave - 1) / RM_G;
+  const int e = (int)threadIdx.x - 64 - g * 64 * RM_G;
+  const int c = e % CP, row = e / CP;
+  const float *__restrict__ src = node + min(cb * 64 + c, C - 1);
+  int k[RM_V];
+  float v[RM_V];
+  // rows past the region repeat its last vertex; no branch, behind which each
+  // load would wait for the one before
+  auto index = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < RM_V; ++u)
+      k[u] = members[min(m0 + t * V + u * RV + row, m1 - 1)];
+  };
+  auto fetch = [&]() {
+#pragma unroll
+    for (int u = 0; u < RM_V; ++u) v[u] = src[(size_t)k[u] * C];
+  };
+  if (g < nt) {
+    index(g);
+    fetch();
+    index(g + RM_D);
+  }
+  for (int t = 0; t < nt; ++t) {
+    if (t % RM_D == g) {
+#pragma unroll
+      for (int u = 0; u < RM_V; ++u) {
+        const int x = u * RV + row;
+        tile[t & 1][c * LD + x] = m0 + t * V + x < m1 ? v[u] : 0.0f;
+      }
+      if (t + RM_D < nt) {
+        fetch();
+        index(t + 2 * RM_D);
+      }
+    }
+    // buffer t & 1 is written; wave 0 has finished tile t - 1 here, so that
+    // the next round may write the other one
+    __syncthreads();
+  }
 }
 
-// node[k][j][p] = roi[rmap[k]][j][p]: one wave per vertex k at a time
-// (all nvar rows), vertices strided over the grid.  grid (<= 16384,
-// ceil(n_inst / 64)), block 256.
+// node[k][c] = roi[rmap[k]][c], a thread per W consecutive columns of a row
+// (W = 4 where the rows are multiples of 16 bytes), I the type that counts
+// the output's words: every lane busy whatever the row's length (a wave per
+// vertex and 64 instances took 57.6 us for 515,056 x 128 where this takes
+// 41, 6.5 TB/s, and 4.1 us for 20,484 x 2 where this takes 2.2).
+template <int W, typename I>
 __global__ void __launch_bounds__(256)
-k_rmap_from_avg(const int *__restrict__ rmap, int nvar, int n_inst,
-                long long nnode, const float *__restrict__ roi,
-                float *__restrict__ node) {
-  const int p = blockIdx.y * 64 + (threadIdx.x & 63);
-  const long long w0 = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const long long ws = (long long)gridDim.x * 4;
-  if (p >= n_inst) return;
-  const size_t row = (size_t)nvar * n_inst;
-  for (long long k = w0; k < nnode; k += ws) {
-    const float *__restrict__ src = roi + (size_t)rmap[k] * row + p;
-    float *__restrict__ dst = node + (size_t)k * row + p;
-    for (int j = 0; j < nvar; ++j) dst[(size_t)j * n_inst] = src[(size_t)j * n_inst];
+k_rmap_from_avg(const int *__restrict__ rmap, I row, I total,
+                const float *__restrict__ roi, float *__restrict__ node) {
+  typedef float wv __attribute__((ext_vector_type(W)));
+  const wv *__restrict__ src = reinterpret_cast<const wv *>(roi);
+  wv *__restrict__ dst = reinterpret_cast<wv *>(node);
+  const I stride = (I)gridDim.x * 256;
+  for (I e = (I)blockIdx.x * 256 + threadIdx.x; e < total; e += stride) {
+    const I k = e / row;
+    dst[e] = src[(I)rmap[k] * row + (e - k * row)];
+    if (total - e <= stride) break;  // e + stride would wrap
   }
 }
-
 
 extern "C" int tvbx_rmap_create(tvbx_ctx *c, const int *rmap, int nnode,
                                 int nroi, tvbx_rmap **out) {
@@ -2999,19 +3085,39 @@ static int rmap_run(tvbx_rmap *r, bool to_avg, int nvar, int n_inst,
   if (rc == TVBX_OK && !dsrc)
     e = hipMemcpyAsync(tin.p, src, bin, hipMemcpyHostToDevice, st);
   if (rc == TVBX_OK && e == hipSuccess) {
-    const unsigned tiles = (unsigned)((n_inst + 63) / 64);
-    const long long rows = (long long)rows_out * nvar;
-    if (to_avg)
-      hipLaunchKernelGGL(k_rmap_to_avg, dim3((unsigned)rows, tiles), dim3(64),
-                         0, st, (const int *)r->rptr.p,
-                         (const int *)r->members.p, nvar, n_inst, s, d);
-    else
-      hipLaunchKernelGGL(k_rmap_from_avg,
-                         dim3((unsigned)std::min<long long>(
-                                  ((long long)r->nnode + 3) / 4, 16384),
-                              tiles),
-                         dim3(256), 0, st, (const int *)r->rmap.p, nvar,
-                         n_inst, (long long)r->nnode, s, d);
+    const long long C = (long long)nvar * n_inst;
+    if (to_avg) {
+      auto fn = C > 32  ? k_rmap_to_avg<64>
+                : C > 16 ? k_rmap_to_avg<32>
+                : C > 8  ? k_rmap_to_avg<16>
+                : C > 4  ? k_rmap_to_avg<8>
+                : C > 2  ? k_rmap_to_avg<4>
+                : C > 1  ? k_rmap_to_avg<2>
+                         : k_rmap_to_avg<1>;
+      const long long nb = (C + 63) / 64, gy = std::min<long long>(nb, 65535);
+      hipLaunchKernelGGL(fn, dim3((unsigned)r->nroi, (unsigned)gy,
+                                  (unsigned)((nb + gy - 1) / gy)),
+                         dim3(RM_T), 0, st, (const int *)r->rptr.p,
+                         (const int *)r->members.p, C, s, d);
+    } else {
+      const bool wide =
+          C % 4 == 0 && ((uintptr_t)s | (uintptr_t)d) % 16 == 0;
+      const long long row = wide ? C / 4 : C, total = row * r->nnode;
+      const unsigned grid = grid1d((size_t)total, 256);
+      const int *map = (const int *)r->rmap.p;
+      if (total < (1ll << 32)) {
+        auto fn = wide ? k_rmap_from_avg<4, unsigned>
+                       : k_rmap_from_avg<1, unsigned>;
+        hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, st, map,
+                           (unsigned)row, (unsigned)total, s, d);
+      } else {
+        auto fn = wide ? k_rmap_from_avg<4, unsigned long long>
+                       : k_rmap_from_avg<1, unsigned long long>;
+        hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, st, map,
+                           (unsigned long long)row, (unsigned long long)total,
+                           s, d);
+      }
+    }
     e = hipGetLastError();
   }
   if (rc == TVBX_OK && e == hipSuccess && !ddst)

@@ -173,8 +173,9 @@ int tvbx_sim_init_history(tvbx_sim *sim, int mode);
 int tvbx_sim_set_noise(tvbx_sim *sim, int mode, unsigned long long seed);
 /* execution mode of tvbx_sim_run: use_graph != 0 replays hipGraph-captured
  * windows of graph_window steps (the step counter lives on the device, so
- * one capture serves every window; runs with injected noise and remainders
- * are launched directly); profile != 0 brackets every step launch (or graph
+ * one capture serves every window; runs with injected noise, remainders and
+ * launches of 8 steps or more that split the nodes over workgroups are
+ * launched directly); profile != 0 brackets every step launch (or graph
  * window) with events for tvbx_sim_timing.  Default: graphs of 100 steps,
  * no profiling.  (The reference's driver launches one kernel per window of
  * n_inner_steps from the host, cuda_run.py:124-142.) */

@@ -1813,10 +1813,17 @@ static long long gcd_ll(long long a, long long b) {
   return a;
 }
 
-// length of a graph window: graph_window rounded to a multiple of the steps
-// per launch and of the monitor period; 0 when graphs are off
+// Length of a graph window: graph_window rounded to a multiple of the steps
+// per launch and of the monitor period; 0 when graphs are off, and for
+// blocked launches of 8 steps or more: enqueueing one (about 4 us a kernel)
+// takes less than running it, while a window costs its clock's upload and
+// tick and the gaps around them (Jansen-Rit N = 379, P = 300, 300 steps 770
+// us in windows, 743 without; a new simulation's first 300 steps 850 and
+// 783; Kuramoto N = 76, P = 64, 200 steps, first 770 and 722).  Launches of
+// a step are the ones that the host cannot keep up with.
 static long long graph_len(tvbx_sim *s) {
-  if (!s->use_graph) return 0;
+  if (!s->use_graph || (is_blocked(s->d) && s->d.steps_per_launch >= 8))
+    return 0;
   long long L = s->d.steps_per_launch;
   if (s->d.tavg_period > 0)
     L = L / gcd_ll(L, s->d.tavg_period) * s->d.tavg_period;

@@ -671,8 +671,9 @@ class Simulation:
             check(lib().tvbx_sim_set_noise(self.h, 1, int(seed)))
 
     def set_exec(self, graph=True, window=100, profile=False):
-        """graph: replay hipGraph windows of `window` steps; profile: time
-        every launch (or window) with events for ``timing()``."""
+        """graph: replay hipGraph windows of `window` steps (launches of 8
+        steps or more that split the nodes go directly); profile: time every
+        launch (or window) with events for ``timing()``."""
         check(lib().tvbx_sim_set_exec(self.h, int(bool(graph)), int(window),
                                       int(bool(profile))))
 

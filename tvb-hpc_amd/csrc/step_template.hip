@@ -1284,25 +1284,175 @@ __device__ __forceinline__ void tvbx_pace_end(const tvbx_step_args &a) {
   }
 }
 
+// Waits for a value's load here (an empty asm statement that takes it, no
+// instruction).  Values that a step loop carries are settled before it and
+// at the end of each pass, where exactly the pass's own later loads and
+// stores are in flight behind them; left to the loop's head, the wait would
+// be for the least common count of its entries, that is for everything, the
+// ring's store of the pass before included.
+template <int A>
+__device__ __forceinline__ void tvbx_settle(float (&v)[A]) {
+#pragma unroll
+  for (int q = 0; q < A; ++q) asm volatile("" : "+v"(v[q]));
+}
+template <int A, int B>
+__device__ __forceinline__ void tvbx_settle(float (&v)[A][B]) {
+#pragma unroll
+  for (int q = 0; q < A; ++q) tvbx_settle(v[q]);
+}
+
+#if TVBX_USES_POST && TVBX_RING_T == 0 && TVBX_IPL == 1 && !TVBX_ORDER_REF && \
+    !TVBX_EMAJ
+#define TVBX_SPLIT 1
+// Blocked launch with a workgroup per (node, 64 / G instances), for a pre()
+// that reads post_syn, so that the sums cannot be formed ahead of the
+// updates.  In one wave a node's step is a serial chain of its row's pre()
+// (sines), with few nodes and instances on a nearly idle chip; here the row
+// is spread over the lanes and waves, and what stays serial is the sum.
+// Kuramoto, N = 76, 22 edges a row, us per step: P = 64 (76 waves' worth)
+// 3.35 in one wave, 1.38 with G = 4, K = 2 (4 instead of 2 waves 1.23, but
+// 2.19 at P = 128; whole waves of instances, G = 1, with 4 waves 2.01, 8
+// 1.66); P = 128 3.36 / 1.48.  Bound by the issue of the pre() and of the
+// sums that every wave repeats.
+//   K waves gather: lane (g, q) = (lane / (64 / G), lane % (64 / G))
+// of wave w takes edges (u K + w) G + g of a block of 64 for instance q,
+// and puts their pre() into LDS.  Edges past the row's end are the last one
+// again, with weight 0, which leaves the sum unchanged (as in the gathers by
+// groups).
+template <int G, int K>
+struct tvbx_split {
+  static constexpr int BLK = 64;          // edges of a block
+  static constexpr int E = BLK / (K * G); // of them a lane's
+  static constexpr int Q = 64 / G;        // instances
+  struct lds {
+    float term[2][BLK][Q];
+    __attribute__((aligned(16))) float w[2][BLK];
+  };
+
+  // the lane's edges of block c: delay, and byte offset of the column's row
+  // in a slot; the block's weights to LDS
+  static __device__ __forceinline__ void row(
+      const tvbx_step_args &a, const unsigned *__restrict__ cd,
+      const float *__restrict__ wt, int e0, int cnt, int c, unsigned lane_off,
+      int (&d)[E], unsigned (&col)[E], float *__restrict__ w) {
+    const int wave = threadIdx.x >> 6, g = (threadIdx.x & 63) / Q;
+    unsigned x[E];
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      x[u] = cd[e0 + min(c * BLK + (u * K + wave) * G + g, cnt - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      d[u] = (int)(x[u] >> 16);
+      col[u] = (x[u] & 0xffffu) * (unsigned)(a.pitch * sizeof(tvbx_rt)) +
+               lane_off;
+      asm volatile("" : "+v"(d[u]), "+v"(col[u]));
+    }
+    for (int l = threadIdx.x; l < BLK; l += 64 * (K + 1))
+      w[l] = c * BLK + l < cnt ? wt[e0 + c * BLK + l] : 0.0f;
+  }
+
+  static __device__ __forceinline__ void fetch(
+      const tvbx_step_args &a, int t, int kk, const int (&d)[E],
+      const unsigned (&col)[E], tvbx_raw (&v)[E]) {
+    const __amdgpu_buffer_rsrc_t rs = tvbx_ring_rsrc(a.ring);
+    const unsigned obs =
+        (unsigned)a.n_node * (unsigned)(a.pitch * sizeof(tvbx_rt));
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      int slot = t - d[u];
+      slot += slot < 0 ? a.horizon : 0;
+      v[u] = tvbx_bload(rs, (unsigned)slot * (TVBX_R * obs) + col[u],
+                        (unsigned)kk * obs);
+    }
+  }
+
+  // n8: the block's edges, rounded up to 8
+  static __device__ __forceinline__ void pre(
+      const tvbx_step_args &a, const tvbx_lane_params &lp, int kk, int n8,
+      float post, const tvbx_raw (&v)[E], float (*__restrict__ term)[Q]) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      if (u * K * G < n8) {
+#if TVBX_PRE_NB
+        // NaN outside the branch-free form's range, or for a non-finite value
+        float p = tvbx_pre_nb(kk, v[u], post, lp, a);
+        if (__builtin_isnan(p)) p = tvbx_pre(kk, v[u], post, lp, a);
+#else
+        const float p = tvbx_pre(kk, v[u], post, lp, a);
+#endif
+        term[(u * K + wave) * G + lane / Q][lane % Q] = p;
+      }
+    }
+  }
+
+  // acc += w[e] term[e] for the block's edges, in order
+  static __device__ __forceinline__ float sum(
+      const float (*__restrict__ term)[Q], const float *__restrict__ w, int n8,
+      float acc) {
+    const int q = threadIdx.x % Q;
+    float v[2][8];
+    float4 ww[2][2];
+    auto load = [&](int h, int b) {
+      const float4 *w4 = reinterpret_cast<const float4 *>(w + b);
+      ww[h][0] = w4[0];
+      ww[h][1] = w4[1];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[h][u] = term[b + u][q];
+    };
+    load(0, 0);
+    for (int e = 0; e < n8; e += 16) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int b = e + 8 * h;
+        if (b >= n8) break;
+        load(1 - h, min(b + 8, BLK - 8));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+          acc = fmaf(ww[h][x].x, v[h][4 * x], acc);
+          acc = fmaf(ww[h][x].y, v[h][4 * x + 1], acc);
+          acc = fmaf(ww[h][x].z, v[h][4 * x + 2], acc);
+          acc = fmaf(ww[h][x].w, v[h][4 * x + 3], acc);
+        }
+      }
+    }
+    return acc;
+  }
+};
+#endif
+
 // The blocked launch of one (instance tile bx, node i) pair: n_steps steps
-// of that node with its state in registers.  SUMS: the launch's coupling
-// accumulators were computed by another kernel (csum).
-template <bool SUMS>
+// of that node with its state in registers.  MODE 0: gathers and updates by
+// the wave; 1: the launch's coupling accumulators were computed by another
+// kernel (csum); 2: the gathers and pre() by K waves (tvbx_split<G, K>); all
+// of them add the terms up and advance the node, so that none waits for
+// another's state, and one more wave, which gathers nothing and so has no
+// loads behind its stores to wait for, stores the results.
+template <int MODE, int G = 1, int K = 1>
 __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
                                                  int bx, int i,
-                                                 int *pace_on = nullptr) {
+                                                 int *pace_on = nullptr,
+                                                 void *shared = nullptr) {
   const int lane = threadIdx.x & 63;
-  const int pb = (bx * 64 + lane) * TVBX_IPL;
+  // MODE 2: bx counts the groups of 64 / G instances
+  const int pb = MODE == 2 ? bx * (64 / G) + lane % (64 / G)
+                           : (bx * 64 + lane) * TVBX_IPL;
   const int N = a.n_node;
   const int H = a.horizon;
   const size_t NP = (size_t)N * a.pitch;
   const int group = __builtin_amdgcn_readfirstlane(
-      (bx * 64 * TVBX_IPL) / a.group_size);
+      (bx * (64 / G) * TVBX_IPL) / a.group_size);
   const unsigned *__restrict__ cd = a.coldelay + (size_t)group * a.nnz;
   const float *__restrict__ wt = tvbx_group_weights(a, group);
   const tvbx_rt *__restrict__ ring = (const tvbx_rt *)a.ring;
   tvbx_rt *ring_w = (tvbx_rt *)a.ring;
   const size_t ip = (size_t)i * a.pitch + pb;
+  constexpr bool SUMS = MODE == 1;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const bool gathers = MODE != 2 || wave < K;
+  const bool lead = MODE != 2 || (wave == K && lane < 64 / G);
 
   tvbx_lane_params lp[TVBX_IPL];
 #pragma unroll
@@ -1340,9 +1490,47 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     tvbx_ldf(a.logp + ip, ls);
     tvbx_ldf(a.logp + NP + ip, lc);
   }
+  if (MODE != 0) {
+    tvbx_settle(x);
+    if (a.tavg_period > 0) tvbx_settle(acc_t);
+    if (SUMS) tvbx_settle(cs);
+    if (a.force != nullptr) {
+      tvbx_settle(xf);
+      tvbx_settle(ls);
+      tvbx_settle(lc);
+    }
+  }
   // the node's row serves every step of the launch
   tvbx_row rw;
-  if (!SUMS) tvbx_load_row(a, cd, wt, i, rw);
+  if (MODE == 0) tvbx_load_row(a, cd, wt, i, rw);
+#if TVBX_SPLIT
+  // MODE 2: an exchange through LDS is a (step, coupled observable, block of
+  // the row); the next one's gathers are in flight meanwhile
+  typedef tvbx_split<G, K> split;
+  typename split::lds &sh = *static_cast<typename split::lds *>(shared);
+  const unsigned lane_off = (unsigned)pb * (unsigned)sizeof(tvbx_rt);
+  int e0 = 0, cnt = 0, nc = 0, bf = 0;
+  int sd[split::E];
+  unsigned sc[split::E];
+  float post[TVBX_C];
+  tvbx_raw gv[split::E];
+  if (MODE == 2) {
+    e0 = a.row[i];
+    cnt = a.row[i + 1] - e0;
+    nc = (cnt + split::BLK - 1) / split::BLK;
+#pragma unroll
+    for (int kk = 0; kk < TVBX_C; ++kk)
+      post[kk] = ring[tvbx_ring_off(t, kk, i, a) + pb];
+    tvbx_settle(post);
+    if (nc > 0) {
+      split::row(a, cd, wt, e0, cnt, 0, lane_off, sd, sc, sh.w[0]);
+      // a row of one block keeps its weights in both buffers
+      for (int l = threadIdx.x; nc == 1 && l < split::BLK; l += 64 * (K + 1))
+        sh.w[1][l] = l < cnt ? wt[e0 + l] : 0.0f;
+      if (gathers) split::fetch(a, t, 0, sd, sc, gv);
+    }
+  }
+#endif
 #if TVBX_EMAJ
   // all the launch's coupling sums first, edges outer and steps inner
   const bool emaj = !SUMS && a.ring32 && a.force == nullptr &&
@@ -1355,10 +1543,45 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     tvbx_progress_prio(k, a.n_steps);
     const long long n = n0 + k;
     const int t1 = (t + 1 == H) ? 0 : t + 1;
-    if (a.rec_x != nullptr) tvbx_record_state(a, ip, n, x);
+    float cn[TVBX_C][TVBX_IPL], xn[TVBX_S][TVBX_IPL];
+    if (SUMS) tvbx_load_sums(a, ip, min(k + 1, a.n_steps - 1), cn);
+    if (SUMS && a.force != nullptr)
+      tvbx_load_frame(a, ip, n + (k + 1 < a.n_steps ? 2 : 1), xn);
+    if (lead && a.rec_x != nullptr) tvbx_record_state(a, ip, n, x);
     float y_mon[TVBX_IPL];
     if (a.tavg_period > 0) tvbx_monitor_obs(a, i, pb, lp, x, y_mon);
     float c[TVBX_IPL][TVBX_C];
+#if TVBX_SPLIT
+    if (MODE == 2) {
+#pragma unroll
+      for (int kk = 0; kk < TVBX_C; ++kk) {
+        float acc = 0.0f;
+        for (int cc = 0; cc < nc; ++cc) {
+          const int n8 = (min(split::BLK, cnt - split::BLK * cc) + 7) & ~7;
+          if (gathers)
+            split::pre(a, lp[0], kk, n8, post[kk], gv, sh.term[bf]);
+          const bool more = cc + 1 < nc, last = kk + 1 == TVBX_C;
+          if (nc > 1)
+            split::row(a, cd, wt, e0, cnt, more ? cc + 1 : 0, lane_off, sd, sc,
+                       sh.w[1 - bf]);
+          // (after the launch's last exchange: a slot that the launch writes,
+          // read and not used)
+          if (gathers)
+            split::fetch(a, more || !last ? t : t1,
+                         more ? kk : (last ? 0 : kk + 1), sd, sc, gv);
+          __syncthreads();
+          acc = split::sum(sh.term[bf], sh.w[bf], n8, acc);
+          // no barrier after the reads: the block's terms are written again
+          // two exchanges on, past the next one's barrier
+          bf ^= 1;
+        }
+        acc = acc * tvbx_acc_unscale(a);
+        if (lead && a.rec_sum != nullptr)
+          a.rec_sum[((size_t)(n - a.rec_step0) * TVBX_C + kk) * NP + ip] = acc;
+        c[0][kk] = tvbx_post(kk, acc, lp[0], a);
+      }
+    } else
+#endif
 #if TVBX_EMAJ
     if (emaj) {
       // ce[k] without dynamic register indexing
@@ -1376,19 +1599,26 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
 #endif
     if (SUMS) {
       tvbx_coupling_from_sums(a, ip, n, lp, cs, c);
-      tvbx_load_sums(a, ip, min(k + 1, a.n_steps - 1), cs);
-    } else {
+    } else if (MODE == 0) {
       tvbx_coupling(a, cd, wt, rw, ring, nullptr, i, t, pb, n, lp, c);
     }
     float yo[TVBX_R][TVBX_IPL];
     tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad,
                  a.force != nullptr);
-    if (a.force != nullptr)
+    if (!SUMS && a.force != nullptr)
       tvbx_load_frame(a, ip, n + (k + 1 < a.n_steps ? 2 : 1), xf);
+#if TVBX_SPLIT
+    if (MODE == 2) {
 #pragma unroll
-    for (int r = 0; r < TVBX_R; ++r)
-      tvbx_str(ring_w + tvbx_ring_off(t1, r, i, a) + pb, yo[r]);
-    if (a.tavg_period > 0) {
+      for (int kk = 0; kk < TVBX_C; ++kk) post[kk] = yo[kk][0];
+    }
+#endif
+    if (lead) {
+#pragma unroll
+      for (int r = 0; r < TVBX_R; ++r)
+        tvbx_str(ring_w + tvbx_ring_off(t1, r, i, a) + pb, yo[r]);
+    }
+    if (lead && a.tavg_period > 0) {
       const bool due = ++ph == a.tavg_period;
       tvbx_monitor(a, ip, due, mo, y_mon, acc_t);
       if (due) {
@@ -1397,6 +1627,20 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
       }
     }
     t = t1;
+    if (SUMS) {
+      tvbx_settle(cn);
+#pragma unroll
+      for (int kk = 0; kk < TVBX_C; ++kk)
+#pragma unroll
+        for (int q = 0; q < TVBX_IPL; ++q) cs[kk][q] = cn[kk][q];
+    }
+    if (SUMS && a.force != nullptr) {
+      tvbx_settle(xn);
+#pragma unroll
+      for (int s = 0; s < TVBX_S; ++s)
+#pragma unroll
+        for (int q = 0; q < TVBX_IPL; ++q) xf[s][q] = xn[s][q];
+    }
     if (pace_on != nullptr && k + 1 < a.n_steps) tvbx_pace(a, k, pace_on);
   }
   // An unforced update keeps a non-finite state non-finite (x itself is a
@@ -1404,6 +1648,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   // so the state at the end of the launch flags every instance that went
   // non-finite during it; forced steps, which replace the state, were
   // checked at every step.
+  if (!lead) return;
   if (a.force == nullptr) tvbx_flag_nonfinite(a, pb, x, bad);
 #pragma unroll
   for (int s = 0; s < TVBX_S; ++s) {
@@ -1482,8 +1727,18 @@ tvbx_step_sums(const tvbx_step_args a) {
   tvbx_block(a, bx, by);
   const int i = __builtin_amdgcn_readfirstlane(by * a.node_block +
                                                (int)(threadIdx.x >> 6));
-  if (i < a.n_node) tvbx_blocked_run<true>(a, bx, i);
+  if (i < a.n_node) tvbx_blocked_run<1>(a, bx, i);
 }
+
+#if TVBX_SPLIT
+// the blocked launch with a workgroup per node and 16 instances; grid
+// (pitch / 16, nodes)
+extern "C" __global__ void __launch_bounds__(192, 4)
+tvbx_step_split(const tvbx_step_args a) {
+  __shared__ tvbx_split<4, 2>::lds sh;
+  tvbx_blocked_run<2, 4, 2>(a, blockIdx.x, blockIdx.y, nullptr, &sh);
+}
+#endif
 
 // the blocked launch in one kernel
 extern "C" __global__ void __launch_bounds__(512, TVBX_MIN_WAVES)
@@ -1494,7 +1749,7 @@ tvbx_step_blocked(const tvbx_step_args a) {
                                                (int)(threadIdx.x >> 6));
   if (a.pace == nullptr) {
     if (i >= a.n_node) return;
-    tvbx_blocked_run<false>(a, bx, i);
+    tvbx_blocked_run<0>(a, bx, i);
     return;
   }
   // paced: every wave of the workgroup takes part in the waits, also one
@@ -1503,7 +1758,7 @@ tvbx_step_blocked(const tvbx_step_args a) {
   if (threadIdx.x == 0) pace_on = 1;
   __syncthreads();
   if (i < a.n_node) {
-    tvbx_blocked_run<false>(a, bx, i, &pace_on);
+    tvbx_blocked_run<0>(a, bx, i, &pace_on);
   } else {
     for (int k = 0; k + 1 < a.n_steps; ++k) tvbx_pace(a, k, &pace_on);
   }
@@ -1527,7 +1782,7 @@ __device__ __forceinline__ void tvbx_batch_item(const tvbx_batch_args &B,
   a.clock = nullptr;
   const int i = node0 + (int)(threadIdx.x >> 6);
   if (i >= a.n_node || i >= node0 + a.node_block) return;
-  tvbx_blocked_run<false>(a, tile, i);
+  tvbx_blocked_run<0>(a, tile, i);
 }
 
 // Without a queue workgroup w takes item w, and the hardware hands

@@ -155,6 +155,8 @@ struct tvbx_module {
   hipFunction_t adj_sums = nullptr, adj_from = nullptr;  // with it too
   hipFunction_t blocked = nullptr;  // absent in the reference ordering
   hipFunction_t step_sums = nullptr;  // blocked launch from given sums
+  hipFunction_t split = nullptr;  // blocked launch, a workgroup per node and
+                                  // 16 instances
   hipFunction_t sums = nullptr;  // absent also where pre() reads post_syn
   hipFunction_t batch = nullptr;    // absent in the reference ordering
   hipFunction_t logp_grad = nullptr;  // present when emitted with the adjoint
@@ -432,6 +434,8 @@ static int module_from_image(tvbx_ctx *c, const void *image, size_t size,
   if (hipModuleGetFunction(&m->step_sums, m->mod, "tvbx_step_sums") !=
       hipSuccess)
     m->step_sums = nullptr;
+  if (hipModuleGetFunction(&m->split, m->mod, "tvbx_step_split") != hipSuccess)
+    m->split = nullptr;
   if (hipModuleGetFunction(&m->sums, m->mod, "tvbx_sums") != hipSuccess)
     m->sums = nullptr;
   if (hipModuleGetFunction(&m->batch, m->mod, "tvbx_step_batch") !=
@@ -1175,6 +1179,17 @@ static unsigned sums_grid(const tvbx_sim *s) {
   return 8 * (((pairs + 7) / 8 + 3) / 4);
 }
 
+// Whether a blocked launch gives each node and 16 instances a workgroup of 3
+// waves (tvbx_step_split) instead of each node and 64 instances a wave: while
+// that leaves the chip idle (Kuramoto N = 76, us per step, a wave against a
+// workgroup: 76 waves 3.35 / 1.38, 152 3.36 / 1.48, 304 3.42 / 2.58, 608
+// 3.50 / 3.95).
+static bool split_launch(const tvbx_sim *s, const tvbx_step_args &a) {
+  const tvbx_sim_desc &d = s->d;
+  return is_blocked(d) && s->mod->split && !a.csum && !a.pace && a.ring32 &&
+         (long long)(s->pitch / 64) * d.n_node <= 384;
+}
+
 // One forward launch of a.n_steps steps: the step kernel of the launch
 // shape, or the kernel that forms the launch's sums (by gathers, or on the
 // matrix cores) and then the blocked updates from them.
@@ -1186,6 +1201,10 @@ static hipError_t launch_steps(tvbx_sim *s, tvbx_step_args &a,
   const unsigned bx = 64u * d.waves;
   void *params[] = {&a};
   hipFunction_t fn = is_blocked(d) ? s->mod->blocked : s->mod->step;
+  if (split_launch(s, a))
+    return hipModuleLaunchKernel(s->mod->split, (unsigned)(s->pitch / 16),
+                                 (unsigned)d.n_node, 1, 192, 1, 1, 0, st,
+                                 params, nullptr);
   if (a.csum) {
     const hipError_t e =
         s->mfma ? hipModuleLaunchKernel(s->mod->mfma, (d.n_node + 15) / 16, gx,

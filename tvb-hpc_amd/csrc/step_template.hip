@@ -613,6 +613,61 @@ __device__ __forceinline__ bool tvbx_group_redo(const float (&acc0)[TVBX_IPL],
 #endif
 #endif
 
+#if !TVBX_ORDER_REF && !TVBX_USES_POST
+// The same for the kernel that forms a launch's sums (tvbx_sums), whose many
+// waves hide each other's latency, so that instructions per edge decide: the
+// weights of whole groups come through the scalar cache (WK, 16 to a load)
+// instead of a v_readlane an edge, the lanes of a row's edges are immediates,
+// and a row's last edges go in a group of 4, 8 or 16 (weights by WR).  32
+// steps of Jansen-Rit N = 379, P = 300, 8 bits: 41.4 us with the groups of
+// the one-kernel launch, 38.0; N = 998, P = 1024, bfloat16, 32 bins, where
+// the memory side binds: 585, 570.
+#define TVBX_SUMS_GROUP (TVBX_RING_T == 0 && TVBX_IPL == 4 ? 8 : 16)
+template <int CNT, typename IX, typename LD, typename WK>
+__device__ __forceinline__ void tvbx_sums_group(
+    const tvbx_step_args &a, const tvbx_lane_params (&lp)[TVBX_IPL], int kk,
+    IX ix, LD ld, WK w, float (&acc)[TVBX_IPL]) {
+  const float post[TVBX_IPL] = {};
+  unsigned sx[CNT];
+  tvbx_raw v[CNT];
+#pragma unroll
+  for (int u = 0; u < CNT; ++u) sx[u] = ix(u);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < CNT; ++u) v[u] = ld(sx[u]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < CNT; ++u)
+    tvbx_accum(acc, w(u), v[u], post, lp, a, kk);
+}
+
+template <typename IX, typename LD, typename WK, typename WR>
+__device__ __forceinline__ void tvbx_sums_range(
+    const tvbx_step_args &a, const tvbx_lane_params (&lp)[TVBX_IPL], int kk,
+    int ne, IX ix, LD ld, WK wk, WR wr, float (&acc)[TVBX_IPL]) {
+  constexpr int B = TVBX_SUMS_GROUP;
+  // (unrolled: the edges' lanes are then immediates)
+#pragma unroll
+  for (int g = 0; g < 64; g += B)
+    if (g + B <= ne)
+      tvbx_sums_group<B>(
+          a, lp, kk, [&](int u) { return ix(g + u); }, ld,
+          [&](int u) { return wk(g + u); }, acc);
+  const int b = ne & -B;
+  const int r = ne - b;
+  if (r <= 0) return;
+  // past the row's end its last edge again, with weight 0
+  const auto ixl = [&](int u) { return ix(min(b + u, ne - 1)); };
+  const auto wl = [&](int u) { return u < r ? wr(min(b + u, ne - 1)) : 0.0f; };
+  if (r <= 4)
+    tvbx_sums_group<4>(a, lp, kk, ixl, ld, wl, acc);
+  else if (B == 8 || r <= 8)
+    tvbx_sums_group<8>(a, lp, kk, ixl, ld, wl, acc);
+  else
+    tvbx_sums_group<16>(a, lp, kk, ixl, ld, wl, acc);
+}
+#endif
+
 // Coupling sums c[q][kk] of node i at step n (ring slot t): the CSR row
 // reduction of network.py:115-136 over the edges in row order, with rec_sum
 // recording for the adjoint.  RAW: the accumulators go to csum instead, n
@@ -650,11 +705,9 @@ __device__ __forceinline__ void tvbx_coupling(
   // ring).  With fewer instances per lane there is too little arithmetic
   // per edge to hide the scalar load, and the weights come from the row's
   // registers as the offsets do.
-#if TVBX_IPL == 4
   typedef __attribute__((address_space(4))) const float tvbx_cwt;
   const tvbx_cwt *wk =
       (const tvbx_cwt *)(wt + __builtin_amdgcn_readfirstlane(row.e0));
-#endif
 #endif
 #pragma unroll
   for (int kk = 0; kk < TVBX_C; ++kk) {
@@ -695,8 +748,24 @@ __device__ __forceinline__ void tvbx_coupling(
 #define TVBX_WK1(x) TVBX_W1(x)
 #endif
 #define TVBX_LB(o) tvbx_bload(rs, voff, (o))
-      TVBX_GATHER_LD(n0, TVBX_X0, TVBX_LB, TVBX_WK0)
-      if (n1 > 0) TVBX_GATHER_LD(n1, TVBX_X1, TVBX_LB, TVBX_WK1)
+#if !TVBX_USES_POST
+      if (RAW) {
+        const auto ld = [&](unsigned o) { return TVBX_LB(o); };
+        tvbx_sums_range(
+            a, lp, kk, n0, [&](int x) { return TVBX_X0(x); }, ld,
+            [&](int x) { return wk[x]; }, [&](int x) { return TVBX_W0(x); },
+            acc);
+        if (n1 > 0)
+          tvbx_sums_range(
+              a, lp, kk, n1, [&](int x) { return TVBX_X1(x); }, ld,
+              [&](int x) { return wk[64 + x]; },
+              [&](int x) { return TVBX_W1(x); }, acc);
+      } else
+#endif
+      {
+        TVBX_GATHER_LD(n0, TVBX_X0, TVBX_LB, TVBX_WK0)
+        if (n1 > 0) TVBX_GATHER_LD(n1, TVBX_X1, TVBX_LB, TVBX_WK1)
+      }
 #undef TVBX_LB
     } else {
       const char *rk = reinterpret_cast<const char *>(ring) +
@@ -738,7 +807,16 @@ __device__ __forceinline__ void tvbx_coupling(
         const unsigned voff =
             lane_off + (unsigned)(kk * a.n_node) * (unsigned)rowb;
 #define TVBX_LB(o) tvbx_bload(rs, voff, (o))
-        TVBX_GATHER_LD(nc, TVBX_XC, TVBX_LB, TVBX_WC)
+#if !TVBX_USES_POST
+        if (RAW)
+          tvbx_sums_range(
+              a, lp, kk, nc, [&](int x) { return TVBX_XC(x); },
+              [&](unsigned o) { return TVBX_LB(o); },
+              [&](int x) { return wk[cb + x]; },
+              [&](int x) { return TVBX_WC(x); }, acc);
+        else
+#endif
+          TVBX_GATHER_LD(nc, TVBX_XC, TVBX_LB, TVBX_WC)
 #undef TVBX_LB
       } else {
         const char *rk = reinterpret_cast<const char *>(ring) +

@@ -1016,6 +1016,24 @@ __device__ __forceinline__ void tvbx_flag_nonfinite(
       bad |= (unsigned)(!isfinite(x[q][s]) && pb + q < a.n_inst) << q;
 }
 
+// Waits for a value's load here (an empty asm statement that takes it, no
+// instruction).  Values that a step loop carries are settled before it and
+// at the end of each pass, where exactly the pass's own later loads and
+// stores are in flight behind them; left to the loop's head, the wait would
+// be for the least common count of its entries, that is for everything, the
+// ring's store of the pass before included.  The same where a branch loads
+// what the code after it uses.
+template <int A>
+__device__ __forceinline__ void tvbx_settle(float (&v)[A]) {
+#pragma unroll
+  for (int q = 0; q < A; ++q) asm volatile("" : "+v"(v[q]));
+}
+template <int A, int B>
+__device__ __forceinline__ void tvbx_settle(float (&v)[A][B]) {
+#pragma unroll
+  for (int q = 0; q < A; ++q) tvbx_settle(v[q]);
+}
+
 // dfun (model.py:105-140), Euler / Euler-Maruyama update (scheme.py:82-97),
 // wrap, non-finite flags (every step with `check`) and the ring values of
 // x(n + 1).  x is updated in place; k is the step's index within the launch.
@@ -1071,6 +1089,7 @@ __device__ __forceinline__ void tvbx_advance(
         const float *nz = a.noise + (size_t)k * a.noise_tstride;
 #pragma unroll
         for (int s = 0; s < TVBX_S; ++s) xi[s] = nz[s * NP + ip + q];
+        tvbx_settle(xi);
       } else {
 #pragma unroll
         for (int s = 0; s < TVBX_S; ++s) xi[s] = 0.0f;
@@ -1360,23 +1379,6 @@ __device__ __forceinline__ void tvbx_pace_end(const tvbx_step_args &a) {
       atomicExch(a.pace + 128, 0u);
     }
   }
-}
-
-// Waits for a value's load here (an empty asm statement that takes it, no
-// instruction).  Values that a step loop carries are settled before it and
-// at the end of each pass, where exactly the pass's own later loads and
-// stores are in flight behind them; left to the loop's head, the wait would
-// be for the least common count of its entries, that is for everything, the
-// ring's store of the pass before included.
-template <int A>
-__device__ __forceinline__ void tvbx_settle(float (&v)[A]) {
-#pragma unroll
-  for (int q = 0; q < A; ++q) asm volatile("" : "+v"(v[q]));
-}
-template <int A, int B>
-__device__ __forceinline__ void tvbx_settle(float (&v)[A][B]) {
-#pragma unroll
-  for (int q = 0; q < A; ++q) tvbx_settle(v[q]);
 }
 
 #if TVBX_USES_POST && TVBX_RING_T == 0 && TVBX_IPL == 1 && !TVBX_ORDER_REF && \

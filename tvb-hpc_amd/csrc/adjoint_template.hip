@@ -475,6 +475,17 @@ tvbx_adjoint_sums(const tvbx_adj_args A) {
     }
   };
   fetch(0, mq);
+  // (the step's carried values: as in the forward updates)
+  auto settle = [&]() {
+    tvbx_settle(xs);
+    tvbx_settle(sm);
+    tvbx_settle(am);
+    tvbx_settle(fo);
+  };
+  tvbx_settle(lr);
+  tvbx_settle(gcr);
+  tvbx_settle(gmr);
+  settle();
   for (int k = 0; k < a.n_steps; ++k) {
     float xk[TVBX_S][TVBX_IPL], sk[TVBX_IPL], ak[TVBX_IPL], fk[TVBX_IPL];
 #pragma unroll
@@ -518,6 +529,7 @@ tvbx_adjoint_sums(const tvbx_adj_args A) {
     }
     tvbx_stf(A.mu + (size_t)t * NP + jp, mu_o);
     t = t == 0 ? H - 1 : t - 1;
+    settle();
   }
 #pragma unroll
   for (int s = 0; s < TVBX_S; ++s) tvbx_stf(A.lam + s * NP + jp, lr[s]);
@@ -540,7 +552,13 @@ tvbx_adjoint_sums(const tvbx_adj_args A) {
 // with the emitted vector-Jacobian products; c(n) = post(sum(n)) from the
 // sums the forced steps recorded.  Compensated float32 sums over the window,
 // added into the compensated sums of the earlier windows.
+//   Few waves, each a serial chain: with a step's loads in the step itself
+// their latency was most of it.  The frames and sums of the next TVBX_LPG
+// steps are loaded while a block of as many is worked off, and a frame is
+// loaded once, x(n + 1) of one step being x(n) of the next (MPR N = 84, P =
+// 512, 150 steps: 122 us with the loads in the step, 50).
 // grid (pitch / (64 ipl), N), block 64.
+#define TVBX_LPG (4 / TVBX_IPL)
 extern "C" __global__ void __launch_bounds__(64)
 tvbx_logp_grad(const tvbx_logp_args L) {
   const tvbx_step_args &a = L.f;
@@ -563,34 +581,79 @@ tvbx_logp_grad(const tvbx_logp_args L) {
 #pragma unroll
     for (int g = 0; g < TVBX_NGC; ++g) gc_acc[q][g] = gc_err[q][g] = 0.0f;
   }
-  for (int k = 0; k < a.n_steps; ++k) {
-    tvbx_progress_prio(k, a.n_steps);
-    const float *__restrict__ x0 = a.force + (size_t)k * TVBX_S * NP + ip;
-    const float *__restrict__ x1 = x0 + (size_t)TVBX_S * NP;
-    const float *__restrict__ sm = L.rec_sum + (size_t)k * TVBX_C * NP + ip;
+  // x(n) and the frames and sums of a block: xb[u] = x(n + 1 + u)
+  float x0[TVBX_S][TVBX_IPL], xb[TVBX_LPG][TVBX_S][TVBX_IPL],
+      sb[TVBX_LPG][TVBX_IPL];
+  const int T = a.n_steps;
+  auto frame = [&](int k, float (&o)[TVBX_S][TVBX_IPL]) {
+#pragma unroll
+    for (int s = 0; s < TVBX_S; ++s)
+      tvbx_ldf(a.force + ((size_t)k * TVBX_S + s) * NP + ip, o[s]);
+  };
+  auto block = [&](int k, float (&o)[TVBX_LPG][TVBX_S][TVBX_IPL],
+                   float (&sm)[TVBX_LPG][TVBX_IPL]) {
+#pragma unroll
+    for (int u = 0; u < TVBX_LPG; ++u) {
+      const int m = min(k + u, T - 1);
+      frame(m + 1, o[u]);
+      tvbx_ldf(L.rec_sum + (size_t)m * TVBX_C * NP + ip, sm[u]);
+    }
+  };
+  if (T > 0) {
+    frame(0, x0);
+    block(0, xb, sb);
+    tvbx_settle(x0);
+    tvbx_settle(sb);
+#pragma unroll
+    for (int u = 0; u < TVBX_LPG; ++u) tvbx_settle(xb[u]);
+  }
+  for (int k = 0; k < T; k += TVBX_LPG) {
+    tvbx_progress_prio(k, T);
+    float xn[TVBX_LPG][TVBX_S][TVBX_IPL], sn[TVBX_LPG][TVBX_IPL];
+    block(k + TVBX_LPG, xn, sn);
+#pragma unroll
+    for (int u = 0; u < TVBX_LPG; ++u) {
+      if (k + u < T) {
+#pragma unroll
+        for (int q = 0; q < TVBX_IPL; ++q) {
+          const int p = pb + q;
+          float x[TVBX_S], f[TVBX_S], g[TVBX_S], lam[TVBX_S], jt[TVBX_S],
+              c[TVBX_C], muc[TVBX_C], gm[TVBX_NGM], gc[TVBX_NGC];
+#pragma unroll
+          for (int s = 0; s < TVBX_S; ++s)
+            x[s] = u == 0 ? x0[s][q] : xb[u > 0 ? u - 1 : 0][s][q];
+          const float sum = sb[u][q];
+          c[0] = tvbx_post(0, sum, lp[q], a);
+          tvbx_dfun(x, c, f, g, lp[q], a, i, p);
+#pragma unroll
+          for (int s = 0; s < TVBX_S; ++s) {
+            const float mu = x[s] + a.dt * f[s];
+            lam[s] = (xb[u][s][q] - mu) / (g[s] * g[s]);
+          }
+          tvbx_dfun_vjp(x, c, lam, jt, muc, gm, lp[q], a, i, p);
+          tvbx_dpost_dparam(sum, gc, lp[q], a);
+#pragma unroll
+          for (int r = 0; r < TVBX_NGM; ++r)
+            tvbx_csum_add(gm_acc[q][r], gm_err[q][r], gm[r]);
+#pragma unroll
+          for (int r = 0; r < TVBX_NGC; ++r)
+            tvbx_csum_add(gc_acc[q][r], gc_err[q][r], muc[0] * gc[r]);
+        }
+      }
+    }
+    tvbx_settle(sn);
+#pragma unroll
+    for (int u = 0; u < TVBX_LPG; ++u) tvbx_settle(xn[u]);
 #pragma unroll
     for (int q = 0; q < TVBX_IPL; ++q) {
-      const int p = pb + q;
-      float x[TVBX_S], f[TVBX_S], g[TVBX_S], lam[TVBX_S], jt[TVBX_S],
-          c[TVBX_C], muc[TVBX_C], gm[TVBX_NGM], gc[TVBX_NGC];
 #pragma unroll
-      for (int s = 0; s < TVBX_S; ++s) x[s] = x0[(size_t)s * NP + q];
-      const float sum = sm[q];
-      c[0] = tvbx_post(0, sum, lp[q], a);
-      tvbx_dfun(x, c, f, g, lp[q], a, i, p);
+      for (int s = 0; s < TVBX_S; ++s) x0[s][q] = xb[TVBX_LPG - 1][s][q];
 #pragma unroll
-      for (int s = 0; s < TVBX_S; ++s) {
-        const float mu = x[s] + a.dt * f[s];
-        lam[s] = (x1[(size_t)s * NP + q] - mu) / (g[s] * g[s]);
+      for (int u = 0; u < TVBX_LPG; ++u) {
+        sb[u][q] = sn[u][q];
+#pragma unroll
+        for (int s = 0; s < TVBX_S; ++s) xb[u][s][q] = xn[u][s][q];
       }
-      tvbx_dfun_vjp(x, c, lam, jt, muc, gm, lp[q], a, i, p);
-      tvbx_dpost_dparam(sum, gc, lp[q], a);
-#pragma unroll
-      for (int r = 0; r < TVBX_NGM; ++r)
-        tvbx_csum_add(gm_acc[q][r], gm_err[q][r], gm[r]);
-#pragma unroll
-      for (int r = 0; r < TVBX_NGC; ++r)
-        tvbx_csum_add(gc_acc[q][r], gc_err[q][r], muc[0] * gc[r]);
     }
   }
   // into the planes of the earlier windows' sums: plane 0 += the window's

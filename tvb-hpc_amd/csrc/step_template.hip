@@ -251,6 +251,10 @@ __device__ __forceinline__ void tvbx_accum(float (&acc)[TVBX_IPL], float w,
 #endif
 }
 
+// a condition that most launches' step loops find false: its code is laid out
+// past the loop, which then has fewer taken branches
+#define TVBX_RARE(x) __builtin_expect(!!(x), 0)
+
 // the factor that turns a coupling accumulator into the sum
 __device__ __forceinline__ float tvbx_acc_unscale(const tvbx_step_args &a) {
 #if TVBX_RING_T == 3
@@ -988,7 +992,7 @@ __device__ __forceinline__ void tvbx_coupling_from_sums(
       acc[q] = cs[kk][q] * tvbx_acc_unscale(a);
       c[q][kk] = tvbx_post(kk, acc[q], lp[q], a);
     }
-    if (a.rec_sum != nullptr)
+    if (TVBX_RARE(a.rec_sum != nullptr))
       tvbx_stf(a.rec_sum + ((size_t)(n - a.rec_step0) * TVBX_C + kk) * NP + ip,
                acc);
   }
@@ -1044,7 +1048,7 @@ __device__ __forceinline__ void tvbx_advance(
     const tvbx_lane_params (&lp)[TVBX_IPL], float (&x)[TVBX_IPL][TVBX_S],
     const float (&c)[TVBX_IPL][TVBX_C], float (&yo)[TVBX_R][TVBX_IPL],
     const float (&xf)[TVBX_S][TVBX_IPL], float (&ls)[TVBX_IPL],
-    float (&lc)[TVBX_IPL], unsigned &bad, bool check) {
+    float (&lc)[TVBX_IPL], unsigned &bad, bool check, bool forced) {
   const size_t NP = (size_t)a.n_node * a.pitch;
   const size_t ip = (size_t)i * a.pitch + pb;
 #pragma unroll
@@ -1060,7 +1064,7 @@ __device__ __forceinline__ void tvbx_advance(
     tvbx_dfun(x[q], c[q], f, g, lp[q], a, i, p);
 #if TVBX_EM
     float xi[TVBX_S];
-    if (a.force != nullptr) {
+    if (forced) {
       // forced step: the transition log density of the given x(n + 1)
       // (scheme.py:42-48, mu = x + dt f, sd = sqrt(dt) g), accumulated as a
       // compensated sum; the state then takes the given value
@@ -1085,7 +1089,7 @@ __device__ __forceinline__ void tvbx_advance(
           for (int r = 0; r < 4; ++r)
             if (s0 + r < TVBX_S) xi[s0 + r] = z[r];
         }
-      } else if (a.noise_mode == 2) {
+      } else if (TVBX_RARE(a.noise_mode == 2)) {
         const float *nz = a.noise + (size_t)k * a.noise_tstride;
 #pragma unroll
         for (int s = 0; s < TVBX_S; ++s) xi[s] = nz[s * NP + ip + q];
@@ -1117,7 +1121,7 @@ __device__ __forceinline__ void tvbx_advance(
       yo[r][q] = v;
     }
     // compatibility outputs of the last step of the launch
-    if (a.out_input != nullptr && k == a.n_steps - 1) {
+    if (TVBX_RARE(a.out_input != nullptr && k == a.n_steps - 1)) {
 #pragma unroll
       for (int kk = 0; kk < TVBX_C; ++kk)
         a.out_input[kk * NP + ip + q] = c[q][kk];
@@ -1153,7 +1157,7 @@ __device__ __forceinline__ void tvbx_monitor(const tvbx_step_args &a,
   const size_t NP = (size_t)a.n_node * a.pitch;
 #pragma unroll
   for (int q = 0; q < TVBX_IPL; ++q) acc_t[q] = acc_t[q] + y_mon[q];
-  if (due) {
+  if (TVBX_RARE(due)) {
     float out[TVBX_IPL];
 #pragma unroll
     for (int q = 0; q < TVBX_IPL; ++q) {
@@ -1276,7 +1280,8 @@ tvbx_step(const tvbx_step_args a) {
         tvbx_ldf(a.logp + ip, ls);
         tvbx_ldf(a.logp + NP + ip, lc);
       }
-      tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad, true);
+      tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad, true,
+                   a.force != nullptr);
       if (a.force != nullptr) {
         tvbx_stf(a.logp + ip, ls);
         tvbx_stf(a.logp + NP + ip, lc);
@@ -1509,8 +1514,13 @@ struct tvbx_split {
 // kernel (csum); 2: the gathers and pre() by K waves (tvbx_split<G, K>); all
 // of them add the terms up and advance the node, so that none waits for
 // another's state, and one more wave, which gathers nothing and so has no
-// loads behind its stores to wait for, stores the results.
-template <int MODE, int G = 1, int K = 1>
+// loads behind its stores to wait for, stores the results.  Modes 1 and 2 are
+// compiled with forced steps (FORCE) and without: what a loop skips costs it
+// a taken branch each, which shows in so short a step (32 steps from given
+// sums, MPR N = 84, P = 1024: 33.5 us with all conditions in one loop, 28.6
+// without the forced steps and with the rare ones moved out, 26.9 with one
+// comparison for the priority; P = 512, forced: 22.1, 18.7).
+template <int MODE, int G = 1, int K = 1, bool FORCE = true>
 __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
                                                  int bx, int i,
                                                  int *pace_on = nullptr,
@@ -1533,6 +1543,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const bool gathers = MODE != 2 || wave < K;
   const bool lead = MODE != 2 || (wave == K && lane < 64 / G);
+  const bool forced = MODE != 0 ? FORCE : a.force != nullptr;
 
   tvbx_lane_params lp[TVBX_IPL];
 #pragma unroll
@@ -1565,7 +1576,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   float cs[TVBX_C][TVBX_IPL], xf[TVBX_S][TVBX_IPL], ls[TVBX_IPL],
       lc[TVBX_IPL];
   if (SUMS) tvbx_load_sums(a, ip, 0, cs);
-  if (a.force != nullptr) {
+  if (forced) {
     tvbx_load_frame(a, ip, n0 + 1, xf);
     tvbx_ldf(a.logp + ip, ls);
     tvbx_ldf(a.logp + NP + ip, lc);
@@ -1574,7 +1585,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     tvbx_settle(x);
     if (a.tavg_period > 0) tvbx_settle(acc_t);
     if (SUMS) tvbx_settle(cs);
-    if (a.force != nullptr) {
+    if (forced) {
       tvbx_settle(xf);
       tvbx_settle(ls);
       tvbx_settle(lc);
@@ -1613,21 +1624,27 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
 #endif
 #if TVBX_EMAJ
   // all the launch's coupling sums first, edges outer and steps inner
-  const bool emaj = !SUMS && a.ring32 && a.force == nullptr &&
+  const bool emaj = !SUMS && a.ring32 && !forced &&
                     a.rec_sum == nullptr && a.n_steps <= TVBX_EMAJ;
   float ce[TVBX_EMAJ][TVBX_IPL][TVBX_C];
   if (emaj) tvbx_coupling_launch(a, cd, wt, rw, ring, t, pb, a.n_steps, lp, ce);
 #endif
 
+  int kp = 0;
   for (int k = 0; k < a.n_steps; ++k) {
-    tvbx_progress_prio(k, a.n_steps);
+    if (MODE == 0)
+      tvbx_progress_prio(k, a.n_steps);
+    else if (TVBX_RARE(k == kp)) {  // one comparison a step
+      tvbx_progress_prio(k, a.n_steps);
+      kp += (a.n_steps + 3) / 4;
+    }
     const long long n = n0 + k;
     const int t1 = (t + 1 == H) ? 0 : t + 1;
     float cn[TVBX_C][TVBX_IPL], xn[TVBX_S][TVBX_IPL];
     if (SUMS) tvbx_load_sums(a, ip, min(k + 1, a.n_steps - 1), cn);
-    if (SUMS && a.force != nullptr)
+    if (SUMS && forced)
       tvbx_load_frame(a, ip, n + (k + 1 < a.n_steps ? 2 : 1), xn);
-    if (lead && a.rec_x != nullptr) tvbx_record_state(a, ip, n, x);
+    if (TVBX_RARE(lead && a.rec_x != nullptr)) tvbx_record_state(a, ip, n, x);
     float y_mon[TVBX_IPL];
     if (a.tavg_period > 0) tvbx_monitor_obs(a, i, pb, lp, x, y_mon);
     float c[TVBX_IPL][TVBX_C];
@@ -1684,8 +1701,8 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     }
     float yo[TVBX_R][TVBX_IPL];
     tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad,
-                 a.force != nullptr);
-    if (!SUMS && a.force != nullptr)
+                 forced, forced);
+    if (!SUMS && forced)
       tvbx_load_frame(a, ip, n + (k + 1 < a.n_steps ? 2 : 1), xf);
 #if TVBX_SPLIT
     if (MODE == 2) {
@@ -1714,7 +1731,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
 #pragma unroll
         for (int q = 0; q < TVBX_IPL; ++q) cs[kk][q] = cn[kk][q];
     }
-    if (SUMS && a.force != nullptr) {
+    if (SUMS && forced) {
       tvbx_settle(xn);
 #pragma unroll
       for (int s = 0; s < TVBX_S; ++s)
@@ -1729,7 +1746,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   // non-finite during it; forced steps, which replace the state, were
   // checked at every step.
   if (!lead) return;
-  if (a.force == nullptr) tvbx_flag_nonfinite(a, pb, x, bad);
+  if (!forced) tvbx_flag_nonfinite(a, pb, x, bad);
 #pragma unroll
   for (int s = 0; s < TVBX_S; ++s) {
     float v[TVBX_IPL];
@@ -1738,7 +1755,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     tvbx_stf(a.state + s * NP + ip, v);
   }
   if (a.tavg_period > 0) tvbx_stf(a.tavg + ip, acc_t);
-  if (a.force != nullptr) {
+  if (forced) {
     tvbx_stf(a.logp + ip, ls);
     tvbx_stf(a.logp + NP + ip, lc);
   }
@@ -1807,7 +1824,11 @@ tvbx_step_sums(const tvbx_step_args a) {
   tvbx_block(a, bx, by);
   const int i = __builtin_amdgcn_readfirstlane(by * a.node_block +
                                                (int)(threadIdx.x >> 6));
-  if (i < a.n_node) tvbx_blocked_run<1>(a, bx, i);
+  if (i >= a.n_node) return;
+  if (a.force != nullptr)
+    tvbx_blocked_run<1, 1, 1, true>(a, bx, i);
+  else
+    tvbx_blocked_run<1, 1, 1, false>(a, bx, i);
 }
 
 #if TVBX_SPLIT
@@ -1816,7 +1837,10 @@ tvbx_step_sums(const tvbx_step_args a) {
 extern "C" __global__ void __launch_bounds__(192, 4)
 tvbx_step_split(const tvbx_step_args a) {
   __shared__ tvbx_split<4, 2>::lds sh;
-  tvbx_blocked_run<2, 4, 2>(a, blockIdx.x, blockIdx.y, nullptr, &sh);
+  if (a.force != nullptr)
+    tvbx_blocked_run<2, 4, 2, true>(a, blockIdx.x, blockIdx.y, nullptr, &sh);
+  else
+    tvbx_blocked_run<2, 4, 2, false>(a, blockIdx.x, blockIdx.y, nullptr, &sh);
 }
 #endif
 

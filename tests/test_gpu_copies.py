@@ -37,3 +37,32 @@ def test_ring_and_state_round_trip(ring, P):
     x = rng.standard_normal((6, N, P)).astype(np.float32)
     sim.set_state(x)
     assert np.array_equal(sim.get_state(), x)
+
+
+def test_threads_sharing_a_context_read_their_own_states():
+    """Each thread's strided copies go through the context's one workspace."""
+    import threading
+    N, P = 50, 300
+    csr = CSR(N, np.arange(N + 1), np.arange(N)[::-1].copy(), np.ones(N),
+              np.full(N, 3))
+    m = M.JansenRit()
+    sims, xs, bad = [], [], []
+    for k in range(4):
+        sims.append(Simulation(m, CF.Sigmoidal(m), SC.EulerStep(0.05), csr, P,
+                               horizon=8))
+        xs.append(np.random.default_rng(k).standard_normal(
+            (6, N, P)).astype(np.float32))
+        sims[k].set_state(xs[k])
+
+    def work(k):
+        for _ in range(60):
+            if not np.array_equal(sims[k].get_state(), xs[k]):
+                bad.append(k)
+            sims[k].set_state(xs[k])
+
+    ts = [threading.Thread(target=work, args=(k, )) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad

@@ -141,9 +141,13 @@ struct tvbx_ctx {
   hipStream_t stream = nullptr;
   hipDeviceProp_t prop{};
   // device workspace of the calls that leave nothing in it (tvbx_fc_loss,
-  // tvbx_sim_fc_sc_error), grown on demand and kept until tvbx_ctx_destroy
+  // tvbx_sim_fc_sc_error, strided host copies), grown on demand and kept
+  // until tvbx_ctx_destroy; a call holds the lock from ctx_work until it has
+  // enqueued its last use, on the context's stream, so that calls of several
+  // threads follow each other there
   void *work = nullptr;
   size_t work_bytes = 0;
+  std::mutex work_lock;
 };
 
 struct tvbx_module {
@@ -1056,8 +1060,14 @@ static int copy_rows(tvbx_ctx *c, void *dst, size_t dp, const void *src,
         "host rows must be contiguous");
   const size_t step =
       std::min(rows, std::max<size_t>(1, (32u << 20) / width));
-  const int rc = ctx_work(c, step * width);
-  if (rc != TVBX_OK) return rc;
+  std::lock_guard<std::mutex> hold(c->work_lock);
+  if (ctx_work(c, step * width) != TVBX_OK) {
+    // no workspace: row by row, slower
+    (void)hipGetLastError();
+    HIPCHK(hipMemcpy2DAsync(dst, dp, src, sp, width, rows, hipMemcpyDefault,
+                            st));
+    return TVBX_OK;
+  }
   for (size_t r = 0; r < rows; r += step) {
     const size_t n = std::min(step, rows - r);
     char *d = (char *)dst + r * dp;
@@ -2105,6 +2115,7 @@ extern "C" int tvbx_sim_fc_sc_error(tvbx_sim *s, const float *sc, int p0,
   const int N = d.n_node;
   // the context's workspace: sc, one partial per (row, instance), the sums
   const size_t nn = ((size_t)N * N * 4 + 255) / 256 * 256;
+  std::lock_guard<std::mutex> hold(s->ctx->work_lock);
   rc = ctx_work(s->ctx, nn + ((size_t)N + 1) * s->pitch * 8);
   if (rc != TVBX_OK) return rc;
   float *dsc = (float *)s->ctx->work;
@@ -2716,6 +2727,7 @@ extern "C" int tvbx_fc_loss(tvbx_ctx *c, const float *samples, long long n,
   CHECK(fc_fits(f, pitch), "FC problem too large for one launch");
   CHECK((unsigned long long)N * pitch * 4ull < (1ull << 32),
         "one sample must stay under 4 GiB for the FC merge");
+  std::lock_guard<std::mutex> hold(c->work_lock);
   int rc = ctx_work(c, used);
   if (rc != TVBX_OK) return rc;
   char *base = static_cast<char *>(c->work);

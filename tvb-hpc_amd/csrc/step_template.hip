@@ -1782,8 +1782,8 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
 // (source, delay) meet there.
 //   Bound: many gathers with little reuse by HBM (Jansen-Rit N = 998, P =
 // 1024, float32: 5.8 TB/s); with 32 delay bins by the L2 and the issue of the
-// gathers (bfloat16, 256-byte rows: 17.9 us per step, 11.3 TB/s of gathered
-// bytes, against 23 us of the one-kernel launch's 27).
+// gathers (bfloat16, 256-byte rows: 17.8 us per step, 11.4 TB/s of gathered
+// bytes of which 5.9 TB/s miss the L2; 23 us of the one-kernel launch's 27).
 extern "C" __global__ void __launch_bounds__(64 * TVBX_SUMS_WAVES)
 tvbx_sums(const tvbx_step_args a) {
   const int lane = threadIdx.x & 63;

@@ -278,14 +278,18 @@ static double gather_reuse(const tvbx_sim_desc &d, const unsigned *cd) {
 // several times in a step and the sums' step-by-step order lets the L2 serve
 // the repeats; else the sums' round trip through memory costs more.
 // Measured, us per step, one kernel against two:
-//   few waves: MPR N = 84, P = 64 (84 waves) 2.59 / 1.09, P = 1024 (1344)
-//   5.45 / 2.24, P = 2048 (2688) 3.69 / 3.70, P = 4096 (5376) 7.21 / 7.27;
-//   two-dimensional oscillator, 12 edges a row, 2100 waves 2.04 / 1.78, 4200
-//   waves 2.78 / 3.31; Jansen-Rit N = 379 8-bit, 1137 waves 4.50 / 2.58;
+//   few waves: MPR N = 84, P = 1024 (1344 waves) 2.37 / 1.59, P = 2048 (2688)
+//   3.27 / 2.89, P = 3072 (4032) 4.51 / 4.49, P = 4096 at 2 instances a lane
+//   (2688) 6.22 / 6.37; two-dimensional oscillator, 33 edges a row, 11 steps
+//   a launch, 1344 waves 3.07 / 2.42, 2688 4.05 / 4.14; 12 edges a row, 2688
+//   2.13 / 2.06, 5376 4.13 / 4.14; Jansen-Rit N = 379 8-bit, 1137 waves 4.45
+//   / 2.29, 1895 6.60 / 4.98;
 //   reuse (N = 998, P = 1024): 4.2 edges per value (32 bins) float32 66.4 /
-//   36.3, 16 bits 28.1 / 21.8 (P = 4096: 148 / 87), 8 bits 13.84 / 13.58;
+//   36.3, 16 bits 28.2 / 21.4 (P = 4096: 148 / 87), 8 bits 13.84 / 13.58;
 //   1.4 (128 bins) float32 73.4 / 59.1, 16 bits 35.2 / 32.7, 8 bits 16.6 /
 //   18.8; 1.06 (exact delays) 16 bits 36.4 / 40.0, 8 bits 17.6 / 20.7.
+//   Short launches of wide lanes gain least: 16 bits, 4 instances a lane, 8
+//   steps 24.8 / 26.4 (16 steps 25.6 / 25.4).
 static bool sums_ahead(const tvbx_sim *s, const unsigned *cd) {
   const tvbx_sim_desc &d = s->d;
   if (!is_blocked(d) || !s->mod->sums || !s->mod->step_sums) return false;

@@ -121,8 +121,8 @@ def default_ipl(cfg):
     and where a history value is gathered several times in a step they keep
     the rows that an XCD reads at a time small enough for its L2 (256-byte
     rows won: us per step at N = 998, P = 1024, 32 delay bins, 1 / 2 / 4
-    instances per lane: float32 36.3 / 42.5 / 49.5, bfloat16 28.0 / 21.8 /
-    23.7, 8 bits 27.8 / 16.5 / 13.6).  Without reuse 2 lanes' worth of
+    instances per lane: float32 36.6 / 42.8 / 52.6, bfloat16 26.9 / 21.4 /
+    24.2, 8 bits 26.3 / 15.9 / 13.9).  Without reuse 2 lanes' worth of
     float32 and 4 of the narrower types suffice.  Below that, the widest with
     enough waves (float32: MPR N = 84, P = 2048 3.7 at 2,688 waves against
     4.2 and 5.1 at 1,344 and 672; P = 4096 6.8 at 2,688, 7.2 at 5,376, 8.4

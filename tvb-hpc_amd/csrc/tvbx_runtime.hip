@@ -1195,13 +1195,16 @@ static unsigned sums_grid(const tvbx_sim *s) {
 
 // Whether a blocked launch gives each node and 16 instances a workgroup of 3
 // waves (tvbx_step_split) instead of each node and 64 instances a wave: while
-// that leaves the chip idle (Kuramoto N = 76, us per step, a wave against a
-// workgroup: 76 waves 3.35 / 1.38, 152 3.36 / 1.48, 304 3.42 / 2.58, 608
-// 3.50 / 3.95).
+// that leaves the chip idle and the workgroups are all resident at once.  us
+// per step, a wave against a workgroup: Kuramoto, 22 edges a row, 76 pairs
+// 3.35 / 1.38, 152 3.36 / 1.48; 60 edges, 64 pairs 5.25 / 1.92, 256 5.23 /
+// 2.18; differences (no sine), 20 edges, 64 pairs 1.62 / 0.87, 256 1.55 /
+// 1.07; 60 edges, 256 pairs 2.56 / 1.71; 70 edges (two blocks) 152 pairs
+// 2.94 / 2.66, 304 2.92 / 3.15, 380 3.54 / 5.11.
 static bool split_launch(const tvbx_sim *s, const tvbx_step_args &a) {
   const tvbx_sim_desc &d = s->d;
   return is_blocked(d) && s->mod->split && !a.csum && !a.pace && a.ring32 &&
-         (long long)(s->pitch / 64) * d.n_node <= 384;
+         (long long)(s->pitch / 64) * d.n_node <= 256;
 }
 
 // One forward launch of a.n_steps steps: the step kernel of the launch

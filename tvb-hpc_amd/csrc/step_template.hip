@@ -1415,11 +1415,11 @@ struct tvbx_split {
   };
 
   // the lane's edges of block c: delay, and byte offset of the column's row
-  // in a slot; the block's weights to LDS
-  static __device__ __forceinline__ void row(
+  // in a slot; returns the block's weight of edge threadIdx.x (threads < BLK)
+  static __device__ __forceinline__ float row(
       const tvbx_step_args &a, const unsigned *__restrict__ cd,
       const float *__restrict__ wt, int e0, int cnt, int c, unsigned lane_off,
-      int (&d)[E], unsigned (&col)[E], float *__restrict__ w) {
+      int (&d)[E], unsigned (&col)[E]) {
     const int wave = threadIdx.x >> 6, g = (threadIdx.x & 63) / Q;
     unsigned x[E];
 #pragma unroll
@@ -1433,8 +1433,8 @@ struct tvbx_split {
                lane_off;
       asm volatile("" : "+v"(d[u]), "+v"(col[u]));
     }
-    for (int l = threadIdx.x; l < BLK; l += 64 * (K + 1))
-      w[l] = c * BLK + l < cnt ? wt[e0 + c * BLK + l] : 0.0f;
+    const int l = c * BLK + (int)threadIdx.x;
+    return threadIdx.x < BLK && l < cnt ? wt[e0 + l] : 0.0f;
   }
 
   static __device__ __forceinline__ void fetch(
@@ -1614,10 +1614,10 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
       post[kk] = ring[tvbx_ring_off(t, kk, i, a) + pb];
     tvbx_settle(post);
     if (nc > 0) {
-      split::row(a, cd, wt, e0, cnt, 0, lane_off, sd, sc, sh.w[0]);
+      const float w0 = split::row(a, cd, wt, e0, cnt, 0, lane_off, sd, sc);
       // a row of one block keeps its weights in both buffers
-      for (int l = threadIdx.x; nc == 1 && l < split::BLK; l += 64 * (K + 1))
-        sh.w[1][l] = l < cnt ? wt[e0 + l] : 0.0f;
+      if (threadIdx.x < split::BLK)
+        sh.w[0][threadIdx.x] = sh.w[1][threadIdx.x] = w0;
       if (gathers) split::fetch(a, t, 0, sd, sc, gv);
     }
   }
@@ -1658,9 +1658,10 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
           if (gathers)
             split::pre(a, lp[0], kk, n8, post[kk], gv, sh.term[bf]);
           const bool more = cc + 1 < nc, last = kk + 1 == TVBX_C;
+          float wn = 0.0f;
           if (nc > 1)
-            split::row(a, cd, wt, e0, cnt, more ? cc + 1 : 0, lane_off, sd, sc,
-                       sh.w[1 - bf]);
+            wn = split::row(a, cd, wt, e0, cnt, more ? cc + 1 : 0, lane_off,
+                            sd, sc);
           // (after the launch's last exchange: a slot that the launch writes,
           // read and not used)
           if (gathers)
@@ -1668,8 +1669,12 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
                          more ? kk : (last ? 0 : kk + 1), sd, sc, gv);
           __syncthreads();
           acc = split::sum(sh.term[bf], sh.w[bf], n8, acc);
-          // no barrier after the reads: the block's terms are written again
-          // two exchanges on, past the next one's barrier
+          // No barrier after the reads.  The block's terms are written again
+          // two exchanges on, past the next one's barrier; the next block's
+          // weights here, past the barrier behind which every wave has done
+          // with the buffer (the exchange before read it).
+          if (nc > 1 && threadIdx.x < split::BLK)
+            sh.w[1 - bf][threadIdx.x] = wn;
           bf ^= 1;
         }
         acc = acc * tvbx_acc_unscale(a);

@@ -1797,18 +1797,20 @@ static int fc_flush(tvbx_sim *s) {
   CHECK(fc_fits(f, s->pitch), "FC problem too large for one launch");
   CHECK((unsigned long long)N * s->pitch * 4ull < (1ull << 32),
         "one monitor sample must stay under 4 GiB for the FC merge");
-  if (!s->fc_tiles.p) {
-    int rc = dalloc(s->fc_tiles, (size_t)f.n_tiles * 8);
-    if (rc == TVBX_OK) rc = dalloc(s->fc_shift, s->NP * 4);
-    if (rc == TVBX_OK) rc = dalloc(s->fc_s1, s->NP * 8);
-    if (rc == TVBX_OK) rc = dalloc(s->fc_u, s->NP * 8);
+  int rc = dalloc(s->fc_shift, s->NP * 4);
+  if (rc == TVBX_OK) rc = dalloc(s->fc_s1, s->NP * 8);
+  if (rc == TVBX_OK) rc = dalloc(s->fc_u, s->NP * 8);
+  if (rc != TVBX_OK) return rc;
+  if (!s->fc_tiles.p) {  // allocated is written: the table comes last
+    rc = dalloc(s->fc_tiles, (size_t)f.n_tiles * 8);
     if (rc != TVBX_OK) return rc;
     fc_tile_table(st, f, (int2 *)s->fc_tiles.p);
   }
   const long long first = (s->sample_base + s->samples_used) % d.sample_slots;
   const double n_prev = (double)s->samples_used;
   fc_merge(st, f, (const float *)s->samples.p,
-           s->smp_ld ? s->smp_ld : s->pitch, d.sample_slots, first, (int)pending, N, s->pitch, n_prev, (const int2 *)s->fc_tiles.p,
+           s->smp_ld ? s->smp_ld : s->pitch, d.sample_slots, first,
+           (int)pending, N, s->pitch, n_prev, (const int2 *)s->fc_tiles.p,
            (const double *)s->fc_mean.p, (float *)s->fc_shift.p,
            (double *)s->fc_s1.p, (double *)s->fc_u.p, (double *)s->fc_m2.p);
   hipLaunchKernelGGL(k_fc_mean, dim3(s->pitch / 64, N), dim3(64), 0, st, N,

@@ -33,6 +33,7 @@ const char *host_hip_log() {
 }
 // the n'th allocation from now fails (0: the next; < 0: none)
 void host_hip_fail(long n) { g_fail = n; }
+long host_hip_left() { return g_fail; }
 long host_hip_held() {
   long n = 0;
   for (auto &m : g_mem) n += (long)m.second;

@@ -1027,6 +1027,28 @@ static int fill_f32(tvbx_sim *s, DevBuf &b, float v) {
   return TVBX_OK;
 }
 
+static void drop_graphs(tvbx_sim *s) {
+  for (auto &g : s->graphs) hipGraphExecDestroy(g.second);
+  s->graphs.clear();
+}
+
+// Device memory of a simulation's calls.  Where there is none left, the sums
+// of its two-kernel launches are given back first: one kernel needs none and
+// gives the same results.
+static int sim_alloc(tvbx_sim *s, DevBuf &b, size_t bytes) {
+  const int rc = dalloc(b, bytes);
+  const bool sums = s->ahead && !s->mfma;
+  if (rc == TVBX_OK || (!sums && !s->msum.p)) return rc;
+  (void)hipGetLastError();
+  (void)hipStreamSynchronize(s->ctx->stream);
+  if (s->aux) (void)hipStreamSynchronize(s->aux);
+  drop_graphs(s);
+  dfree(s->msum);
+  if (sums) dfree(s->csum);
+  s->ahead = false;
+  return dalloc(b, bytes);
+}
+
 // host [rows][P] <-> device [rows][pitch]
 // true when p is device memory that kernels can read and write directly
 static bool on_device(const void *p) {
@@ -1391,10 +1413,6 @@ extern "C" int tvbx_sim_destroy(tvbx_sim *s) {
   return TVBX_OK;
 }
 
-static void drop_graphs(tvbx_sim *s) {
-  for (auto &g : s->graphs) hipGraphExecDestroy(g.second);
-  s->graphs.clear();
-}
 
 extern "C" int tvbx_sim_set_exec(tvbx_sim *s, int use_graph, int graph_window,
                                  int profile) {
@@ -1797,12 +1815,12 @@ static int fc_flush(tvbx_sim *s) {
   CHECK(fc_fits(f, s->pitch), "FC problem too large for one launch");
   CHECK((unsigned long long)N * s->pitch * 4ull < (1ull << 32),
         "one monitor sample must stay under 4 GiB for the FC merge");
-  int rc = dalloc(s->fc_shift, s->NP * 4);
-  if (rc == TVBX_OK) rc = dalloc(s->fc_s1, s->NP * 8);
-  if (rc == TVBX_OK) rc = dalloc(s->fc_u, s->NP * 8);
+  int rc = sim_alloc(s, s->fc_shift, s->NP * 4);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->fc_s1, s->NP * 8);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->fc_u, s->NP * 8);
   if (rc != TVBX_OK) return rc;
   if (!s->fc_tiles.p) {  // allocated is written: the table comes last
-    rc = dalloc(s->fc_tiles, (size_t)f.n_tiles * 8);
+    rc = sim_alloc(s, s->fc_tiles, (size_t)f.n_tiles * 8);
     if (rc != TVBX_OK) return rc;
     fc_tile_table(st, f, (int2 *)s->fc_tiles.p);
   }
@@ -1957,7 +1975,7 @@ extern "C" int tvbx_sim_run(tvbx_sim *s, long long n_steps,
     CHECK(tstride == 0 || tstride == (long long)d.n_svar * d.n_node * d.n_inst,
           "noise_tstride must be 0 or S*N*P");
     size_t steps_up = tstride ? (size_t)n_steps : 1;
-    int rc = dalloc(s->noise, steps_up * SNP * 4);
+    int rc = sim_alloc(s, s->noise, steps_up * SNP * 4);
     if (rc != TVBX_OK) return rc;
     rc = up2d(s, s->noise.p, noise, steps_up * d.n_svar * d.n_node);
     if (rc != TVBX_OK) return rc;
@@ -2098,7 +2116,7 @@ extern "C" int tvbx_sim_fc(tvbx_sim *s, int p0, int np, float *corr,
   // linear copy (a strided copy of the triangle's N (N + 1) / 2 rows per
   // call took seconds at N = 998)
   const size_t nn = (size_t)N * N;
-  rc = dalloc(s->corr, (size_t)np * nn * 4);
+  rc = sim_alloc(s, s->corr, (size_t)np * nn * 4);
   if (rc != TVBX_OK) return rc;
   fc_corr(s->ctx->stream, (const double *)s->fc_m2.p, N, s->pitch, p0, np,
           (float *)s->corr.p);
@@ -2199,18 +2217,19 @@ extern "C" int tvbx_sim_logp(tvbx_sim *s, const float *traj,
   const size_t SNP = (size_t)d.n_svar * s->NP;
   const size_t frame = (size_t)d.n_svar * d.n_node * d.n_inst;
   const int ngc = std::max(n_gc, 1), ngm = std::max(n_gm, 1);
-  int rc = dalloc(s->force, d.n_inst == s->pitch && on_device(traj)
-                                ? 4
-                                : (size_t)(W + 1) * SNP * 4);
+  int rc = sim_alloc(s, s->force, d.n_inst == s->pitch && on_device(traj)
+                                      ? 4
+                                      : (size_t)(W + 1) * SNP * 4);
   // compensated float32 sums: two planes (sum, carried rounding error)
-  if (rc == TVBX_OK) rc = dalloc(s->logp, 2 * s->NP * 4);
-  if (rc == TVBX_OK) rc = dalloc(s->logp_sum, 2 * (size_t)s->pitch * 4);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->logp, 2 * s->NP * 4);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->logp_sum, 2 * (size_t)s->pitch * 4);
   if (rc == TVBX_OK) rc = fill_f32(s, s->force, 0.0f);
   if (rc == TVBX_OK) rc = fill_f32(s, s->logp, 0.0f);
   if (grads) {
-    if (rc == TVBX_OK) rc = dalloc(s->rec_sum, (size_t)W * d.n_coupled * s->NP * 4);
-    if (rc == TVBX_OK) rc = dalloc(s->lg_c, 2 * (size_t)ngc * s->NP * 4);
-    if (rc == TVBX_OK) rc = dalloc(s->lg_m, 2 * (size_t)ngm * s->NP * 4);
+    if (rc == TVBX_OK)
+      rc = sim_alloc(s, s->rec_sum, (size_t)W * d.n_coupled * s->NP * 4);
+    if (rc == TVBX_OK) rc = sim_alloc(s, s->lg_c, 2 * (size_t)ngc * s->NP * 4);
+    if (rc == TVBX_OK) rc = sim_alloc(s, s->lg_m, 2 * (size_t)ngm * s->NP * 4);
     if (rc == TVBX_OK) rc = fill_f32(s, s->lg_c, 0.0f);
     if (rc == TVBX_OK) rc = fill_f32(s, s->lg_m, 0.0f);
   }
@@ -3248,9 +3267,9 @@ static int build_csc(tvbx_sim *s) {
       CHECK(dl >= 1, "the adjoint needs delays >= 1 (edge %d has 0)", perm[k]);
       crow[(size_t)g * nnz + k] = ((unsigned)dl << 16) | (unsigned)tgt[k];
     }
-  int rc = dalloc(s->ccol, (size_t)(N + 1) * 4);
-  if (rc == TVBX_OK) rc = dalloc(s->crow, crow.size() * 4);
-  if (rc == TVBX_OK) rc = dalloc(s->cw, cw.size() * 4);
+  int rc = sim_alloc(s, s->ccol, (size_t)(N + 1) * 4);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->crow, crow.size() * 4);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->cw, cw.size() * 4);
   if (rc != TVBX_OK) return rc;
   HIPCHK(hipMemcpyAsync(s->ccol.p, cnt.data(), (size_t)(N + 1) * 4,
                         hipMemcpyHostToDevice, s->ctx->stream));
@@ -3279,9 +3298,9 @@ extern "C" int tvbx_sim_checkpoint_run(tvbx_sim *s, long long n_steps,
   if (window == 0) {
     // record the whole run: no checkpoints, no replay in the adjoint
     CHECK(n_steps <= 0x7fffffffLL, "too many steps to record");
-    rc = dalloc(s->rec_x, (size_t)n_steps * d.n_svar * s->NP * 4);
+    rc = sim_alloc(s, s->rec_x, (size_t)n_steps * d.n_svar * s->NP * 4);
     if (rc == TVBX_OK)
-      rc = dalloc(s->rec_sum, (size_t)n_steps * d.n_coupled * s->NP * 4);
+      rc = sim_alloc(s, s->rec_sum, (size_t)n_steps * d.n_coupled * s->NP * 4);
     if (rc != TVBX_OK) return rc;
     s->ck_step0 = s->step;
     s->ck_T = n_steps;
@@ -3303,8 +3322,8 @@ extern "C" int tvbx_sim_checkpoint_run(tvbx_sim *s, long long n_steps,
     s->ck_ring.assign(K, DevBuf());
   }
   for (long long k = 0; k < K; ++k) {
-    rc = dalloc(s->ck_state[k], sb);
-    if (rc == TVBX_OK) rc = dalloc(s->ck_ring[k], rb);
+    rc = sim_alloc(s, s->ck_state[k], sb);
+    if (rc == TVBX_OK) rc = sim_alloc(s, s->ck_ring[k], rb);
     if (rc != TVBX_OK) return rc;
   }
   s->ck_step0 = s->step;
@@ -3351,7 +3370,7 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
   const int ngc = std::max(n_gc, 1), ngm = std::max(n_gm, 1);
   int r2 = TVBX_OK;
 #define AL(buf, bytes) \
-  if (r2 == TVBX_OK) r2 = dalloc(s->buf, (size_t)(bytes));
+  if (r2 == TVBX_OK) r2 = sim_alloc(s, s->buf, (size_t)(bytes));
   AL(lam, (size_t)S * NP * 4);
   AL(mu, (size_t)d.horizon * NP * 4);
   AL(rec_x, (size_t)W * S * NP * 4);
@@ -3360,9 +3379,6 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
   AL(g_c, (size_t)ngc * NP * 4);
   AL(g_m, (size_t)ngm * NP * 4);
   AL(g_out, (size_t)ngc * pitch * 4);
-  // reverse launches as two kernels where the forward ones are
-  const bool ahead = s->ahead && s->mod->adj_sums;
-  if (ahead) AL(msum, (size_t)d.steps_per_launch * NP * 4);
   // replaying inside the checkpoints leaves the end-of-run state and ring
   // untouched: nothing to save
   const bool consume = !s->ck_recorded && !s->ck_keep;
@@ -3413,8 +3429,8 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
   const bool overlap = replay && K > 1;
   hipStream_t sa = s->ctx->stream, sb = sa;
   if (overlap) {
-    rc = dalloc(s->rec_x2, (size_t)W * S * NP * 4);
-    if (rc == TVBX_OK) rc = dalloc(s->rec_sum2, (size_t)W * NP * 4);
+    rc = sim_alloc(s, s->rec_x2, (size_t)W * S * NP * 4);
+    if (rc == TVBX_OK) rc = sim_alloc(s, s->rec_sum2, (size_t)W * NP * 4);
     if (rc != TVBX_OK) return rc;
     if (!s->aux) HIPCHK(hipStreamCreateWithFlags(&s->aux, hipStreamNonBlocking));
     sb = s->aux;
@@ -3427,6 +3443,12 @@ extern "C" int tvbx_sim_adjoint(tvbx_sim *s, const float *dsamples,
     HIPCHK(hipEventRecord(s->adj_ev[2 * K], sa));
     HIPCHK(hipStreamWaitEvent(sb, s->adj_ev[2 * K], 0));
   }
+  // reverse launches as two kernels where the forward ones are; what the call
+  // cannot do without is allocated by now
+  const bool ahead =
+      s->ahead && s->mod->adj_sums &&
+      dalloc(s->msum, (size_t)d.steps_per_launch * NP * 4) == TVBX_OK;
+  if (!ahead) (void)hipGetLastError();
   auto rec_x_of = [&](long long kw) {
     return (float *)((overlap && (kw & 1)) ? s->rec_x2.p : s->rec_x.p);
   };

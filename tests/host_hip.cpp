@@ -16,6 +16,7 @@ static std::map<const void *, std::string> g_kernels;
 static std::map<char *, size_t> g_mem;
 static std::vector<std::string> g_log, *g_capture;
 static long g_fail = -1;  // allocations until the one that fails
+static bool g_fail_on;    // and all after it
 
 static void note(const std::string &name, unsigned gx, unsigned gy) {
   (g_capture ? *g_capture : g_log)
@@ -32,7 +33,15 @@ const char *host_hip_log() {
   return s.c_str();
 }
 // the n'th allocation from now fails (0: the next; < 0: none)
-void host_hip_fail(long n) { g_fail = n; }
+void host_hip_fail(long n) {
+  g_fail = n;
+  g_fail_on = false;
+}
+// it and all after it
+void host_hip_fail_from(long n) {
+  g_fail = n;
+  g_fail_on = true;
+}
 long host_hip_left() { return g_fail; }
 long host_hip_held() {
   long n = 0;
@@ -100,6 +109,7 @@ hipError_t hipFuncGetAttribute(int *v, hipFunction_attribute, hipFunction_t) {
 }
 
 hipError_t hipMalloc(void **p, size_t n) {
+  if (g_fail == 0 && g_fail_on) return hipErrorOutOfMemory;
   if (g_fail >= 0 && g_fail-- == 0) return hipErrorOutOfMemory;
   *p = calloc(1, n ? n : 1);
   g_mem[(char *)*p] = n;

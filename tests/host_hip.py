@@ -22,7 +22,7 @@ sys.path[:0] = [%(pkg)r, %(tests)r]
 H = ctypes.CDLL(%(lib)r, ctypes.RTLD_GLOBAL)
 H.host_hip_log.restype = ctypes.c_char_p
 H.host_hip_held.restype = H.host_hip_left.restype = ctypes.c_long
-H.host_hip_fail.argtypes = [ctypes.c_long]
+H.host_hip_fail.argtypes = H.host_hip_fail_from.argtypes = [ctypes.c_long]
 import numpy as np
 from tvb_hpc import coupling as CF, hip, model as M, scheme as SC
 from tvb_hpc.network import CSR

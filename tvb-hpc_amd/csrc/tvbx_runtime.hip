@@ -3267,9 +3267,10 @@ static int build_csc(tvbx_sim *s) {
       CHECK(dl >= 1, "the adjoint needs delays >= 1 (edge %d has 0)", perm[k]);
       crow[(size_t)g * nnz + k] = ((unsigned)dl << 16) | (unsigned)tgt[k];
     }
-  int rc = sim_alloc(s, s->ccol, (size_t)(N + 1) * 4);
-  if (rc == TVBX_OK) rc = sim_alloc(s, s->crow, crow.size() * 4);
+  // ccol last: its pointer says that the transpose is there
+  int rc = sim_alloc(s, s->crow, crow.size() * 4);
   if (rc == TVBX_OK) rc = sim_alloc(s, s->cw, cw.size() * 4);
+  if (rc == TVBX_OK) rc = sim_alloc(s, s->ccol, (size_t)(N + 1) * 4);
   if (rc != TVBX_OK) return rc;
   HIPCHK(hipMemcpyAsync(s->ccol.p, cnt.data(), (size_t)(N + 1) * 4,
                         hipMemcpyHostToDevice, s->ctx->stream));

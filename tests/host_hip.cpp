@@ -5,6 +5,8 @@
 // kernel names that it holds.
 #include <hip/hip_runtime.h>
 
+#include <sys/mman.h>
+
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -15,6 +17,7 @@
 static std::map<const void *, std::string> g_kernels;
 static std::map<char *, size_t> g_mem;
 static std::vector<std::string> g_log, *g_capture;
+static const size_t BIG = 1u << 30;
 static long g_fail = -1;  // allocations until the one that fails
 static bool g_fail_on;    // and all after it
 
@@ -111,13 +114,21 @@ hipError_t hipFuncGetAttribute(int *v, hipFunction_attribute, hipFunction_t) {
 hipError_t hipMalloc(void **p, size_t n) {
   if (g_fail == 0 && g_fail_on) return hipErrorOutOfMemory;
   if (g_fail >= 0 && g_fail-- == 0) return hipErrorOutOfMemory;
-  *p = calloc(1, n ? n : 1);
+  // large memory is address space only, until it is touched
+  *p = n < BIG ? calloc(1, n ? n : 1)
+               : mmap(nullptr, n, PROT_READ | PROT_WRITE,
+                      MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
   g_mem[(char *)*p] = n;
   return hipSuccess;
 }
 hipError_t hipFree(void *p) {
+  if (!p) return hipSuccess;
+  const size_t n = g_mem[(char *)p];
   g_mem.erase((char *)p);
-  free(p);
+  if (n < BIG)
+    free(p);
+  else
+    munmap(p, n);
   return hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void **p, const void *) {

@@ -3052,7 +3052,7 @@ k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
 
 // node[k][c] = roi[rmap[k]][c], a thread per W consecutive columns of a row
 // (W = 4 where the rows are multiples of 16 bytes), I the type that counts
-// the output's words: every lane busy whatever the row's length (a wave per
+// the words of both arrays: every lane busy whatever the row's length (a wave per
 // vertex and 64 instances took 57.6 us for 515,056 x 128 where this takes
 // 41, 6.5 TB/s, and 4.1 us for 20,484 x 2 where this takes 2.2).
 template <int W, typename I>
@@ -3171,7 +3171,9 @@ static int rmap_run(tvbx_rmap *r, bool to_avg, int nvar, int n_inst,
       const long long row = wide ? C / 4 : C, total = row * r->nnode;
       const unsigned grid = grid1d((size_t)total, 256);
       const int *map = (const int *)r->rmap.p;
-      if (total < (1ll << 32)) {
+      // 32-bit indices: into the vertices and into the regions, of which
+      // there may be more
+      if (std::max(total, row * r->nroi) < (1ll << 32)) {
         auto fn = wide ? k_rmap_from_avg<4, unsigned>
                        : k_rmap_from_avg<1, unsigned>;
         hipLaunchKernelGGL(fn, dim3(grid), dim3(256), 0, st, map,

@@ -2931,7 +2931,14 @@ struct tvbx_rmap {
   DevBuf rmap;     // [nnode] region of each vertex
   DevBuf rptr;     // [nroi + 1] CSR of the vertices of each region
   DevBuf members;  // [nnode] vertices by region, ascending within a region
+  int longest = 0; // vertices of the largest region
 };
+
+// whether region sums of C columns go to k_rmap_to_avg_short (which tells why)
+static bool rmap_short(const tvbx_rmap *r, long long C) {
+  const double groups = (double)r->nroi * (double)((C + 63) / 64);
+  return r->longest <= 0.25 * groups + 1e-5 * (double)r->nnode * (double)C;
+}
 
 // roi[r][c] = sum of node[k][c] over the vertices k of region r, c one of the
 // row's C = nvar n_inst columns, added in ascending k from 0 (the reference
@@ -3050,6 +3057,45 @@ k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
   }
 }
 
+// The same for short regions: a wave per region and 64 columns, the loads of
+// RMAP_UNROLL vertices in flight together and added in order.  A region costs
+// it its chain, 27 ns a vertex, and next to nothing beside that, where a
+// workgroup of the kernel above costs 5 ns of the chip whatever its region's
+// length and its chain 3 ns a vertex.  Which one is taken (rmap_short): the
+// longest region against a quarter of the workgroups, and against the reads,
+// which the waves of short regions overlap better (515,056 vertices x 128).
+// Whole calls, us, this kernel against the one above, the longest region in
+// parentheses: 20,484 vertices x 1 in 300 regions (89) 23.4 / 22.6, 600 (55)
+// 22.6 / 23.9, 20,000 (6) 24.6 / 110; x 128 in 200 (129) 25.8 / 24.0, 400
+// (71) 24.5 / 25.2; 515,056 x 1 in 1500 (406) 36.7 / 29.0, 3000 (220) 32.1 /
+// 36.7, 100,000 (19) 51 / 593; x 128 in 300 (1835) 116 / 87, 1000 (591) 68 /
+// 80; uneven, 20,484 x 1 in 1000 (268) 27.1 / 25.6, 2000 (142) 24.2 / 30.7.
+// grid (nroi, y, z) with y z >= ceil(C / 64), block 64.
+#define RMAP_UNROLL 32
+__global__ void __launch_bounds__(64)
+k_rmap_to_avg_short(const int *__restrict__ rptr,
+                    const int *__restrict__ members, long long C,
+                    const float *__restrict__ node, float *__restrict__ roi) {
+  const int r = blockIdx.x;
+  const long long cb = (long long)blockIdx.z * gridDim.y + blockIdx.y;
+  const long long col = cb * 64 + threadIdx.x;
+  const bool on = col < C;
+  const int m0 = rptr[r], m1 = rptr[r + 1];
+  const float *__restrict__ src = node + (on ? col : 0);
+  float acc = 0.0f;
+  int m = m0;
+  for (; m1 - m >= RMAP_UNROLL; m += RMAP_UNROLL) {
+    float v[RMAP_UNROLL];
+#pragma unroll
+    for (int u = 0; u < RMAP_UNROLL; ++u)
+      v[u] = src[(size_t)members[m + u] * C];
+#pragma unroll
+    for (int u = 0; u < RMAP_UNROLL; ++u) acc += v[u];
+  }
+  for (; m < m1; ++m) acc += src[(size_t)members[m] * C];
+  if (on) roi[(size_t)r * C + col] = acc;
+}
+
 // node[k][c] = roi[rmap[k]][c], a thread per W consecutive columns of a row
 // (W = 4 where the rows are multiples of 16 bytes), I the type that counts
 // the words of both arrays: every lane busy whatever the row's length (a wave per
@@ -3090,6 +3136,8 @@ extern "C" int tvbx_rmap_create(tvbx_ctx *c, const int *rmap, int nnode,
   r->ctx = c;
   r->nnode = nnode;
   r->nroi = nroi;
+  for (int k = 0; k < nroi; ++k)
+    r->longest = std::max(r->longest, cnt[(size_t)k + 1] - cnt[k]);
   int rc = dalloc(r->rmap, (size_t)nnode * 4);
   if (rc == TVBX_OK) rc = dalloc(r->rptr, ((size_t)nroi + 1) * 4);
   if (rc == TVBX_OK) rc = dalloc(r->members, (size_t)nnode * 4);
@@ -3153,7 +3201,9 @@ static int rmap_run(tvbx_rmap *r, bool to_avg, int nvar, int n_inst,
   if (rc == TVBX_OK && e == hipSuccess) {
     const long long C = (long long)nvar * n_inst;
     if (to_avg) {
-      auto fn = C > 32  ? k_rmap_to_avg<64>
+      const bool few = rmap_short(r, C);
+      auto fn = few      ? k_rmap_to_avg_short
+                : C > 32 ? k_rmap_to_avg<64>
                 : C > 16 ? k_rmap_to_avg<32>
                 : C > 8  ? k_rmap_to_avg<16>
                 : C > 4  ? k_rmap_to_avg<8>
@@ -3163,7 +3213,7 @@ static int rmap_run(tvbx_rmap *r, bool to_avg, int nvar, int n_inst,
       const long long nb = (C + 63) / 64, gy = std::min<long long>(nb, 65535);
       hipLaunchKernelGGL(fn, dim3((unsigned)r->nroi, (unsigned)gy,
                                   (unsigned)((nb + gy - 1) / gy)),
-                         dim3(RM_T), 0, st, (const int *)r->rptr.p,
+                         dim3(few ? 64 : RM_T), 0, st, (const int *)r->rptr.p,
                          (const int *)r->members.p, C, s, d);
     } else {
       const bool wide =

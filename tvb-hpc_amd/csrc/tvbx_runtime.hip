@@ -256,12 +256,12 @@ static bool is_blocked(const tvbx_sim_desc &d) {
   return d.steps_per_launch > 1 && d.node_block < d.n_node;
 }
 
-// How often a history value is gathered in a step: edges per distinct
-// (delay, source), of the first delay group (1 when there are too many
-// (delay, source) pairs to count).
-static double gather_reuse(const tvbx_sim_desc &d, const unsigned *cd) {
+// Distinct (delay, source) pairs of the first delay group's edges: the history
+// values of an instance that a step gathers (all edges where there are too
+// many pairs to count).
+static size_t gather_distinct(const tvbx_sim_desc &d, const unsigned *cd) {
   const size_t bits = (size_t)d.horizon * d.n_node;
-  if (d.nnz == 0 || bits > (1ull << 28)) return 1.0;
+  if (bits > (1ull << 28)) return (size_t)d.nnz;
   std::vector<bool> seen(bits, false);
   size_t distinct = 0;
   for (int e = 0; e < d.nnz; ++e) {
@@ -269,33 +269,55 @@ static double gather_reuse(const tvbx_sim_desc &d, const unsigned *cd) {
     distinct += !seen[b];
     seen[b] = true;
   }
-  return (double)d.nnz / (double)distinct;
+  return distinct;
 }
 
 // Whether a blocked launch runs as two kernels, all its coupling sums ahead
-// of its updates (tvbx_sums, tvbx_step_sums), or as one.  Two kernels win
-// where one would leave the chip idle, and where a history value is gathered
-// several times in a step and the sums' step-by-step order lets the L2 serve
-// the repeats; else the sums' round trip through memory costs more.
-// Measured, us per step, one kernel against two:
-//   few waves: MPR N = 84, P = 1024 (1344 waves) 2.37 / 1.59, P = 2048 (2688)
-//   3.27 / 2.89, P = 3072 (4032) 4.51 / 4.49, P = 4096 at 2 instances a lane
-//   (2688) 6.22 / 6.37; two-dimensional oscillator, 33 edges a row, 11 steps
-//   a launch, 1344 waves 3.07 / 2.42, 2688 4.05 / 4.14; 12 edges a row, 2688
-//   2.13 / 2.06, 5376 4.13 / 4.14; Jansen-Rit N = 379 8-bit, 1137 waves 4.45
-//   / 2.29, 1895 6.60 / 4.98;
-//   reuse (N = 998, P = 1024): 4.2 edges per value (32 bins) float32 66.4 /
-//   36.3, 16 bits 28.2 / 21.4 (P = 4096: 148 / 87), 8 bits 13.84 / 13.58;
-//   1.4 (128 bins) float32 73.4 / 59.1, 16 bits 35.2 / 32.7, 8 bits 16.6 /
-//   18.8; 1.06 (exact delays) 16 bits 36.4 / 40.0, 8 bits 17.6 / 20.7.
-//   Short launches of wide lanes gain least: 16 bits, 4 instances a lane, 8
-//   steps 24.8 / 26.4 (16 steps 25.6 / 25.4).
+// of its updates (tvbx_sums, tvbx_step_sums), or as one.  The sums' round trip
+// through memory and the second launch have to be earned, so a launch of few
+// steps stays one kernel, and a longer one is split
+//  1. where little is gathered in a step: the slot of one step's history is
+//     small, one kernel is bound by each wave's serial chain and leaves the
+//     chip idle.  us per step, one kernel / two, 32 steps a launch: float32
+//     MPR N = 84, 20 edges a row, P = 256 (86 KB) 1.51 / 0.68, 1024 (344 KB)
+//     1.68 / 1.06, 2048 (688 KB) 1.87 / 1.65; Jansen-Rit N = 998, 100 edges, P
+//     = 64 (255 KB) 5.13 / 4.09, 128 (511 KB) 6.85 / 7.81; N = 400, 40 edges,
+//     P = 512 (819 KB) at 2 instances a lane 3.70 / 4.31; 8 bits N = 998, P =
+//     256 (255 KB) 6.08 / 5.50, 512 (511 KB) 7.89 / 9.61.  With fewer steps,
+//     N = 84, P = 256: 8 steps 1.81 / 1.38, 4 2.18 / 2.08, 2 2.79 / 3.43; P =
+//     1024: 2.09 / 1.94, 2.59 / 2.76, 3.37 / 4.19; with 60 edges a row 3.34 /
+//     2.68, 3.86 / 3.67, 4.64 / 5.23;
+//  2. where history values are gathered several times in a step (edges per
+//     distinct value) and the distinct rows of an instance tile fit the 4 MB
+//     L2 of an XCD, which the sums' step-by-step order then hits, 8 / 32 steps
+//     a launch: float32 N = 400, 80 edges a row, P = 1024, 4.1 edges a value
+//     (2.0 MB) 10.9 / 9.6 and 12.4 / 8.9; N = 998, P = 512, 6.3 (4.1 MB) 19.1
+//     / 18.5 and 22.0 / 17.2; P = 256, 3.1 (8.2 MB) 11.1 / 12.4 and 12.1 /
+//     11.5; N = 2000, 2.7 (9.4 MB) 12.6 / 13.2 and 12.4 / 12.3;
+//  3. where they are and the ring is well beyond the 256 MB of the last level
+//     cache, so that every repeat saved is a read of HBM.  By ring bytes times
+//     edges a value, N = 998, 8 steps: float32 P = 1024, 1.4 (2.6 GB) 71.8 /
+//     64.7; 16 bits at 2 instances a lane, 1.4, P = 1024 (1.3 GB) 32.9 / 36.5,
+//     P = 2048 (2.6 GB) 74.5 / 70.2; 3.1, P = 1024 (2.8 GB) 27.7 / 26.1, with
+//     4 steps 26.6 / 28.5; 8 bits at 4, 1.9, P = 1024 (0.9 GB) 15.6 / 18.5, P
+//     = 4096 (3.4 GB), 4 steps, 91 / 73.  Without repeats 16 bits 31.5 / 35.4.
 static bool sums_ahead(const tvbx_sim *s, const unsigned *cd) {
   const tvbx_sim_desc &d = s->d;
-  if (!is_blocked(d) || !s->mod->sums || !s->mod->step_sums) return false;
-  const long long waves = (long long)(s->pitch / (64 * d.ipl)) * d.n_node;
-  return waves < 2400 ||
-         gather_reuse(d, cd) >= (d.ring_type == 3 ? 2.0 : 1.25);
+  const int L = d.steps_per_launch;
+  if (!is_blocked(d) || !s->mod->sums || !s->mod->step_sums || L < 4)
+    return false;
+  const double slot = (double)s->NP * s->esz, edges = (double)d.nnz;
+  if (slot <= 450e3 &&
+      (L >= 8 || edges >= 50.0 * d.n_node || slot <= 100e3))
+    return true;
+  if (slot <= 450e3 || d.nnz == 0) return false;
+  const double distinct = (double)gather_distinct(d, cd);
+  const double reuse = edges / distinct;
+  const double tile = distinct * 64.0 * d.ipl * s->esz;
+  const double ring = slot * d.horizon;
+  if (L >= 8 && reuse >= 1.5 && tile <= 4.2e6) return true;
+  return reuse >= 1.25 && ring >= 600e6 &&
+         ring * reuse >= (L >= 8 ? 1.8e9 : 3.2e9);
 }
 
 // advance the device clock by w steps (last node of a captured window)

@@ -55,6 +55,10 @@ RULE = [
     ((998, 100, 1024, 'bf16', 2, 32, 100, 400), ONE),
     ((998, 100, 1024, 'bf16', 4, 8, 25, 400), TWO),
     ((998, 100, 1024, 'u8', 4, 8, 50, 400), ONE),    # 2.2, ring 0.45 GB
+    ((998, 100, 2048, 'u8', 4, 16, 30, 400), ONE),   # 3.4, ring 0.9 GB
+    ((998, 100, 2048, 'u8', 4, 32, 20, 400), TWO),   # 5
+    ((400, 40, 2048, 'u8', 4, 8, 30, 60), ONE),      # 1.8 edges a value
+    ((400, 80, 2048, 'u8', 4, 8, 15, 60), TWO),      # 4, 2 MB
 ]
 
 

@@ -301,6 +301,10 @@ static size_t gather_distinct(const tvbx_sim_desc &d, const unsigned *cd) {
 //     P = 2048 (2.6 GB) 74.5 / 70.2; 3.1, P = 1024 (2.8 GB) 27.7 / 26.1, with
 //     4 steps 26.6 / 28.5; 8 bits at 4, 1.9, P = 1024 (0.9 GB) 15.6 / 18.5, P
 //     = 4096 (3.4 GB), 4 steps, 91 / 73.  Without repeats 16 bits 31.5 / 35.4.
+//     Values of 8 bits gain least, their sums being four times their size, and
+//     are split later in 2. and 3.: N = 400, P = 4096, 1.8 edges a value 0.87
+//     times as fast, N = 84, P = 8192, 2.3 1.12; N = 998, P = 1024, 6.3 (2.7
+//     GB) 0.97, P = 2048, 3.1 (2.8 GB), 4, 8 and 32 steps 0.97, 1.01, 1.08.
 static bool sums_ahead(const tvbx_sim *s, const unsigned *cd) {
   const tvbx_sim_desc &d = s->d;
   const int L = d.steps_per_launch;
@@ -315,9 +319,10 @@ static bool sums_ahead(const tvbx_sim *s, const unsigned *cd) {
   const double reuse = edges / distinct;
   const double tile = distinct * 64.0 * d.ipl * s->esz;
   const double ring = slot * d.horizon;
-  if (L >= 8 && reuse >= 1.5 && tile <= 4.2e6) return true;
+  const bool bytes = d.ring_type == 3;
+  if (L >= 8 && reuse >= (bytes ? 2.0 : 1.5) && tile <= 4.2e6) return true;
   return reuse >= 1.25 && ring >= 600e6 &&
-         ring * reuse >= (L >= 8 ? 1.8e9 : 3.2e9);
+         ring * reuse >= (L >= 8 && !bytes ? 1.8e9 : 3.2e9);
 }
 
 // advance the device clock by w steps (last node of a captured window)

@@ -251,9 +251,13 @@ __device__ __forceinline__ void tvbx_accum(float (&acc)[TVBX_IPL], float w,
 #endif
 }
 
-// a condition that most launches' step loops find false: its code is laid out
-// past the loop, which then has fewer taken branches
-#define TVBX_RARE(x) __builtin_expect(!!(x), 0)
+// A condition that most launches' step loops find false: where RARE, its code
+// is laid out past the loop, which then has fewer taken branches.  The loops
+// that also gather leave it where it is: there the hint, and what the loop
+// carries along, cost spilled registers where registers are short (Jansen-Rit
+// N = 998, P = 1024, 16 bits at 4 instances a lane, one kernel: 70 with it
+// and 37.8 us a step, 31 and 35.3 without).
+#define TVBX_RARE(x) (RARE ? __builtin_expect(!!(x), 0) : !!(x))
 
 // the factor that turns a coupling accumulator into the sum
 __device__ __forceinline__ float tvbx_acc_unscale(const tvbx_step_args &a) {
@@ -992,7 +996,7 @@ __device__ __forceinline__ void tvbx_coupling_from_sums(
       acc[q] = cs[kk][q] * tvbx_acc_unscale(a);
       c[q][kk] = tvbx_post(kk, acc[q], lp[q], a);
     }
-    if (TVBX_RARE(a.rec_sum != nullptr))
+    if (__builtin_expect(a.rec_sum != nullptr, 0))
       tvbx_stf(a.rec_sum + ((size_t)(n - a.rec_step0) * TVBX_C + kk) * NP + ip,
                acc);
   }
@@ -1042,7 +1046,9 @@ __device__ __forceinline__ void tvbx_settle(float (&v)[A][B]) {
 // wrap, non-finite flags (every step with `check`) and the ring values of
 // x(n + 1).  x is updated in place; k is the step's index within the launch.
 // Forced steps take x(n + 1) from xf and add their log density to the
-// compensated sum ls + lc.
+// compensated sum ls + lc, both loaded by the caller; unless RARE they load
+// and store their own.
+template <bool RARE>
 __device__ __forceinline__ void tvbx_advance(
     const tvbx_step_args &a, int i, int pb, long long n, int k,
     const tvbx_lane_params (&lp)[TVBX_IPL], float (&x)[TVBX_IPL][TVBX_S],
@@ -1068,17 +1074,28 @@ __device__ __forceinline__ void tvbx_advance(
       // forced step: the transition log density of the given x(n + 1)
       // (scheme.py:42-48, mu = x + dt f, sd = sqrt(dt) g), accumulated as a
       // compensated sum; the state then takes the given value
+      const float *__restrict__ xn =
+          RARE ? nullptr
+               : a.force + (size_t)(n + 1 - a.force_step0) * TVBX_S * NP + ip +
+                     q;
       float lp_step = 0.0f;
 #pragma unroll
       for (int s = 0; s < TVBX_S; ++s) {
         const float mu = x[q][s] + a.dt * f[s];
-        const float xs1 = xf[s][q];
+        const float xs1 = RARE ? xf[s][q] : xn[(size_t)s * NP];
         const float r = xs1 - mu;
         const float sd2 = a.dt * g[s] * g[s];
         lp_step -= r * r / (2.0f * sd2);
         x[q][s] = xs1;
       }
-      tvbx_csum_add(ls[q], lc[q], lp_step);
+      if (RARE) {
+        tvbx_csum_add(ls[q], lc[q], lp_step);
+      } else {
+        float l0 = a.logp[ip + q], l1 = a.logp[NP + ip + q];
+        tvbx_csum_add(l0, l1, lp_step);
+        a.logp[ip + q] = l0;
+        a.logp[NP + ip + q] = l1;
+      }
     } else {
       if (a.noise_mode == 1) {
 #pragma unroll
@@ -1150,6 +1167,7 @@ __device__ __forceinline__ void tvbx_monitor_obs(
 // time average over tavg_period steps; at the period's last step (due) the
 // average (optionally through Balloon-Windkessel) goes to sample slot
 // m mod sample_slots and the accumulator restarts
+template <bool RARE>
 __device__ __forceinline__ void tvbx_monitor(const tvbx_step_args &a,
                                              size_t ip, bool due, long long m,
                                              const float (&y_mon)[TVBX_IPL],
@@ -1275,17 +1293,8 @@ tvbx_step(const tvbx_step_args a) {
 
       float yo[TVBX_R][TVBX_IPL], xf[TVBX_S][TVBX_IPL], ls[TVBX_IPL],
           lc[TVBX_IPL];
-      if (a.force != nullptr) {
-        tvbx_load_frame(a, ip, n + 1, xf);
-        tvbx_ldf(a.logp + ip, ls);
-        tvbx_ldf(a.logp + NP + ip, lc);
-      }
-      tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad, true,
-                   a.force != nullptr);
-      if (a.force != nullptr) {
-        tvbx_stf(a.logp + ip, ls);
-        tvbx_stf(a.logp + NP + ip, lc);
-      }
+      tvbx_advance<false>(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad, true,
+                          a.force != nullptr);
 #pragma unroll
       for (int s = 0; s < TVBX_S; ++s) {
         float v[TVBX_IPL];
@@ -1313,8 +1322,8 @@ tvbx_step(const tvbx_step_args a) {
       if (a.tavg_period > 0) {
         float acc_t[TVBX_IPL];
         tvbx_ldf(a.tavg + ip, acc_t);
-        tvbx_monitor(a, ip, (n + 1) % a.tavg_period == 0,
-                     (n + 1) / a.tavg_period - 1, y_mon, acc_t);
+        tvbx_monitor<false>(a, ip, (n + 1) % a.tavg_period == 0,
+                            (n + 1) / a.tavg_period - 1, y_mon, acc_t);
         tvbx_stf(a.tavg + ip, acc_t);
       }
     }
@@ -1539,11 +1548,11 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   const tvbx_rt *__restrict__ ring = (const tvbx_rt *)a.ring;
   tvbx_rt *ring_w = (tvbx_rt *)a.ring;
   const size_t ip = (size_t)i * a.pitch + pb;
-  constexpr bool SUMS = MODE == 1;
+  constexpr bool SUMS = MODE == 1, RARE = MODE != 0;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const bool gathers = MODE != 2 || wave < K;
   const bool lead = MODE != 2 || (wave == K && lane < 64 / G);
-  const bool forced = MODE != 0 ? FORCE : a.force != nullptr;
+  const bool forced = TVBX_EM && (MODE != 0 ? FORCE : a.force != nullptr);
 
   tvbx_lane_params lp[TVBX_IPL];
 #pragma unroll
@@ -1565,18 +1574,21 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   if (a.tavg_period > 0) tvbx_ldf(a.tavg + ip, acc_t);
 #pragma unroll
   for (int q = 0; q < TVBX_IPL; ++q) tvbx_load_node(lp[q], a, i, pb + q);
-  // the monitor's period: steps into it, and the sample it ends with
+  // the monitor's period: steps into it, and the sample it ends with (where
+  // the wave also gathers, by division at each step)
   int ph = 0;
   long long mo = 0;
-  if (a.tavg_period > 0) {
+  if (MODE != 0 && a.tavg_period > 0) {
     mo = n0 / a.tavg_period;
     ph = (int)(n0 - mo * a.tavg_period);
   }
-  // given sums and forced frames are loaded one step ahead
+  // given sums and forced frames are loaded one step ahead, the log density
+  // stays in registers; where the wave also gathers there are none to spare,
+  // and a forced step loads and stores its own
   float cs[TVBX_C][TVBX_IPL], xf[TVBX_S][TVBX_IPL], ls[TVBX_IPL],
       lc[TVBX_IPL];
   if (SUMS) tvbx_load_sums(a, ip, 0, cs);
-  if (forced) {
+  if (MODE != 0 && forced) {
     tvbx_load_frame(a, ip, n0 + 1, xf);
     tvbx_ldf(a.logp + ip, ls);
     tvbx_ldf(a.logp + NP + ip, lc);
@@ -1705,9 +1717,9 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
       tvbx_coupling(a, cd, wt, rw, ring, nullptr, i, t, pb, n, lp, c);
     }
     float yo[TVBX_R][TVBX_IPL];
-    tvbx_advance(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad,
-                 forced, forced);
-    if (!SUMS && forced)
+    tvbx_advance<RARE>(a, i, pb, n, k, lp, x, c, yo, xf, ls, lc, bad, forced,
+                       forced);
+    if (MODE == 2 && forced)
       tvbx_load_frame(a, ip, n + (k + 1 < a.n_steps ? 2 : 1), xf);
 #if TVBX_SPLIT
     if (MODE == 2) {
@@ -1721,9 +1733,12 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
         tvbx_str(ring_w + tvbx_ring_off(t1, r, i, a) + pb, yo[r]);
     }
     if (lead && a.tavg_period > 0) {
-      const bool due = ++ph == a.tavg_period;
-      tvbx_monitor(a, ip, due, mo, y_mon, acc_t);
-      if (due) {
+      const bool due =
+          MODE == 0 ? (n + 1) % a.tavg_period == 0 : ++ph == a.tavg_period;
+      tvbx_monitor<RARE>(a, ip, due,
+                         MODE == 0 ? (n + 1) / a.tavg_period - 1 : mo, y_mon,
+                         acc_t);
+      if (MODE != 0 && due) {
         ph = 0;
         ++mo;
       }
@@ -1760,7 +1775,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
     tvbx_stf(a.state + s * NP + ip, v);
   }
   if (a.tavg_period > 0) tvbx_stf(a.tavg + ip, acc_t);
-  if (forced) {
+  if (MODE != 0 && forced) {
     tvbx_stf(a.logp + ip, ls);
     tvbx_stf(a.logp + NP + ip, lc);
   }

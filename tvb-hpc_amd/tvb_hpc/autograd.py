@@ -144,12 +144,51 @@ def fc_loss(samples, fc_target):
     return 1.0 - r
 
 
+def _grad_by_bmm(M, N, P):
+    """Whether the FC loss's gradient takes one batched product between two
+    transposes instead of tvbx_fc_loss_grad.
+
+    The kernel's lanes are instances and each wave walks the nodes one after
+    the other: 0.7 us a node, or the arithmetic of instances rounded up to 64.
+    Few instances of many nodes leave it idle or padded, and a large product
+    alone runs faster in the library; the transposes and the scaling of S cost
+    a product per instance and node pair.  us of a backward pass, kernel /
+    product: M = 1000 samples, N = 998, P = 1 2189 / 227, P = 16 2364 / 709,
+    P = 65 6227 / 3056; M = 200, N = 400, P = 8 292 / 156, P = 48 326 / 310;
+    M = 100, N = 400, P = 1024 1114 / 3867; M = 2000, N = 600, P = 128 4953 /
+    3553; N = 250, M = 1000, P = 24 241 / 242; up to 150 nodes the kernel is
+    the faster one throughout (M = 500, N = 84, P = 1024 356 / 751)."""
+    if N < 160:
+        return False
+    kernel = max(0.7 * N, 5.0e-8 * 64 * -(-P // 64) * M * N * N)
+    product = 160.0 + P * N * N * (2.5e-8 * M + 1.5e-5)
+    return product < kernel
+
+
+def _grad_product(hctx, x, s, mean, g):
+    "The gradient as one product per instance, batched over the instances."
+    M, N, P = x.shape
+    dev = x.device
+    xt = torch.empty((P, M * N), dtype=torch.float32, device=dev)
+    sp = (s.permute(2, 0, 1) * g[:, None, None]).contiguous()
+    dx = torch.empty((M, N, P), dtype=torch.float32, device=dev)
+    torch.cuda.current_stream(dev).synchronize()
+    hctx.transpose(x.data_ptr(), M * N, P, xt.data_ptr(), mean.data_ptr(), N)
+    hctx.sync()
+    y = torch.bmm(xt.view(P, M, N), sp)
+    torch.cuda.current_stream(dev).synchronize()
+    hctx.transpose(y.data_ptr(), P, M * N, dx.data_ptr())
+    hctx.sync()
+    return dx
+
+
 class _FcLossDevice(torch.autograd.Function):
     """fc_loss of device samples on the HIP kernels: the FP64 co-moments
     and the loss with its derivative in libtvbx (tvbx_fc_loss), the samples'
     gradient as one float32 product per instance, dL_p/dx_p = gout_p (x_p -
-    mean_p) S_p, with the instances innermost throughout
-    (tvbx_fc_loss_grad)."""
+    mean_p) S_p: with the instances innermost throughout (tvbx_fc_loss_grad),
+    or, where ``_grad_by_bmm`` says so, batched between two transposes
+    (tvbx_transpose) that take the instance axis outermost and back."""
 
     @staticmethod
     def forward(ctx, samples, fc_target, hctx):
@@ -180,6 +219,12 @@ class _FcLossDevice(torch.autograd.Function):
         hctx = ctx.hctx
         dev = x.device
         g = gout.detach().float().contiguous()
+        if _grad_by_bmm(M, N, P):
+            try:
+                return _grad_product(hctx, x, s, mean, g).to(ctx.dtype), \
+                    None, None
+            except torch.cuda.OutOfMemoryError:
+                pass                # the kernel needs no workspace
         dx = torch.empty((M, N, P), dtype=torch.float32, device=dev)
         torch.cuda.current_stream(dev).synchronize()
         hctx.fc_loss_grad(x.data_ptr(), M, N, P, s.data_ptr(),

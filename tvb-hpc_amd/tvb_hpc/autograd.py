@@ -156,12 +156,12 @@ def _grad_by_bmm(M, N, P):
     product: M = 1000 samples, N = 998, P = 1 2189 / 227, P = 16 2364 / 709,
     P = 65 6227 / 3056; M = 200, N = 400, P = 8 292 / 156, P = 48 326 / 310;
     M = 100, N = 400, P = 1024 1114 / 3867; M = 2000, N = 600, P = 128 4953 /
-    3553; N = 250, M = 1000, P = 24 241 / 242; up to 150 nodes the kernel is
-    the faster one throughout (M = 500, N = 84, P = 1024 356 / 751)."""
+    3553; M = 50, N = 200, P = 1 on two devices 166 / 172 and 204 / 132, N =
+    100 116 / 168 and 148 / 131; M = 500, N = 84, P = 1024 356 / 751."""
     if N < 160:
         return False
-    kernel = max(0.7 * N, 5.0e-8 * 64 * -(-P // 64) * M * N * N)
-    product = 160.0 + P * N * N * (2.5e-8 * M + 1.5e-5)
+    kernel = max(0.75 * N, 5.0e-8 * 64 * -(-P // 64) * M * N * N)
+    product = 120.0 + P * N * N * (2.5e-8 * M + 1.5e-5)
     return product < kernel
 
 

@@ -149,7 +149,8 @@ def _grad_by_bmm(M, N, P):
     transposes instead of tvbx_fc_loss_grad.
 
     The kernel's lanes are instances and each wave walks the nodes one after
-    the other: 0.7 us a node, or the arithmetic of instances rounded up to 64.
+    the other: 0.6 to 0.9 us a node, or the arithmetic of instances rounded up
+    to 64.
     Few instances of many nodes leave it idle or padded, and a large product
     alone runs faster in the library; the transposes and the scaling of S cost
     a product per instance and node pair.  us of a backward pass, kernel /

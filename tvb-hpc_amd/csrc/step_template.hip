@@ -1528,8 +1528,11 @@ struct tvbx_split {
 // a taken branch each, which shows in so short a step (32 steps from given
 // sums, MPR N = 84, P = 1024: 33.5 us with all conditions in one loop, 28.6
 // without the forced steps and with the rare ones moved out, 26.9 with one
-// comparison for the priority; P = 512, forced: 22.1, 18.7).
-template <int MODE, int G = 1, int K = 1, bool FORCE = true>
+// comparison for the priority; P = 512, forced: 22.1, 18.7).  So are mode 2's
+// rows of several blocks of edges (MULTI), whose exchange of weights would
+// cost the others too (Kuramoto, 22 edges a row, 1.73 us a step, 1.58 apart).
+template <int MODE, int G = 1, int K = 1, bool FORCE = true,
+          bool MULTI = false>
 __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
                                                  int bx, int i,
                                                  int *pace_on = nullptr,
@@ -1620,7 +1623,7 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
   if (MODE == 2) {
     e0 = a.row[i];
     cnt = a.row[i + 1] - e0;
-    nc = (cnt + split::BLK - 1) / split::BLK;
+    nc = MULTI ? (cnt + split::BLK - 1) / split::BLK : min(cnt, 1);
 #pragma unroll
     for (int kk = 0; kk < TVBX_C; ++kk)
       post[kk] = ring[tvbx_ring_off(t, kk, i, a) + pb];
@@ -1669,11 +1672,13 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
           const int n8 = (min(split::BLK, cnt - split::BLK * cc) + 7) & ~7;
           if (gathers)
             split::pre(a, lp[0], kk, n8, post[kk], gv, sh.term[bf]);
-          const bool more = cc + 1 < nc, last = kk + 1 == TVBX_C;
-          float wn = 0.0f;
-          if (nc > 1)
-            wn = split::row(a, cd, wt, e0, cnt, more ? cc + 1 : 0, lane_off,
-                            sd, sc);
+          const bool more = MULTI && cc + 1 < nc, last = kk + 1 == TVBX_C;
+          float wn[1];
+          if (MULTI) {
+            wn[0] = split::row(a, cd, wt, e0, cnt, more ? cc + 1 : 0, lane_off,
+                               sd, sc);
+            tvbx_settle(wn);  // here, not behind the gathers that follow
+          }
           // (after the launch's last exchange: a slot that the launch writes,
           // read and not used)
           if (gathers)
@@ -1685,8 +1690,8 @@ __device__ __forceinline__ void tvbx_blocked_run(const tvbx_step_args &a,
           // two exchanges on, past the next one's barrier; the next block's
           // weights here, past the barrier behind which every wave has done
           // with the buffer (the exchange before read it).
-          if (nc > 1 && threadIdx.x < split::BLK)
-            sh.w[1 - bf][threadIdx.x] = wn;
+          if (MULTI && threadIdx.x < split::BLK)
+            sh.w[1 - bf][threadIdx.x] = wn[0];
           bf ^= 1;
         }
         acc = acc * tvbx_acc_unscale(a);
@@ -1857,10 +1862,20 @@ tvbx_step_sums(const tvbx_step_args a) {
 extern "C" __global__ void __launch_bounds__(192, 4)
 tvbx_step_split(const tvbx_step_args a) {
   __shared__ tvbx_split<4, 2>::lds sh;
-  if (a.force != nullptr)
-    tvbx_blocked_run<2, 4, 2, true>(a, blockIdx.x, blockIdx.y, nullptr, &sh);
-  else
-    tvbx_blocked_run<2, 4, 2, false>(a, blockIdx.x, blockIdx.y, nullptr, &sh);
+  const int bx = blockIdx.x, i = blockIdx.y;
+  // (rows of one block of edges apart from longer ones)
+  const bool multi = a.row[i + 1] - a.row[i] > tvbx_split<4, 2>::BLK;
+  if (TVBX_EM && a.force != nullptr) {
+    if (multi)
+      tvbx_blocked_run<2, 4, 2, true, true>(a, bx, i, nullptr, &sh);
+    else
+      tvbx_blocked_run<2, 4, 2, true, false>(a, bx, i, nullptr, &sh);
+  } else {
+    if (multi)
+      tvbx_blocked_run<2, 4, 2, false, true>(a, bx, i, nullptr, &sh);
+    else
+      tvbx_blocked_run<2, 4, 2, false, false>(a, bx, i, nullptr, &sh);
+  }
 }
 #endif
 

@@ -77,21 +77,6 @@ def log(*a):
           flush=True)
 
 
-def step_kernel(sim, cfg):
-    """The kernels of a launch: a blocked one with few waves, or with history
-    values gathered several times in a step, runs as two (the rule of
-    libtvbx's sums_ahead)."""
-    from tvb_hpc.autotune import gather_reuse
-    if not sim.blocked:
-        return 'tvbx_step'
-    waves = cfg.csr.nnode * -(-cfg.n_inst // (64 * sim.spec.ipl))
-    reuse = 2.0 if cfg.ring_dtype == 'u8' else 1.25
-    if cfg.coupling != 'mfma' and (waves < 2400 or
-                                   gather_reuse(cfg.csr) >= reuse):
-        return 'tvbx_sums + tvbx_step_sums'
-    return 'tvbx_step_blocked'
-
-
 def traffic_from_profile(kernel, workload, launch):
     """HBM bytes per dispatch of `kernel` on `workload` from the committed
     PMC summary (profiles/<kernel>_<workload>_pmc.txt), if it was measured
@@ -168,7 +153,7 @@ def time_sweep(cfg, launch, K, W, graph_window, profile_steps):
     per_s = steps_per_launch / (launch_ms * 1e-3)
     achieved = bytes_inst_step * P * per_s / 1e9
     comp = comp_inst_step * P * per_s / 1e9
-    kernel = step_kernel(sim, cfg)
+    kernel = sim.kernels()
     del sim
     return dict(value=P * K / el, ms_per_step=el / K * 1e3, steps=K,
                 roofline={

@@ -171,6 +171,11 @@ int tvbx_sim_init_history(tvbx_sim *sim, int mode);
 /* noise source for Euler-Maruyama: 0 none, 1 Philox4x32-10 with the given
  * 64-bit seed (counter = step, node | svar/4 << 24, instance, step >> 32) */
 int tvbx_sim_set_noise(tvbx_sim *sim, int mode, unsigned long long seed);
+/* The kernels of one of the simulation's launches, in order and joined by
+ * " + ", as a string into buf (len bytes): "tvbx_step", "tvbx_step_blocked",
+ * "tvbx_step_split", "tvbx_sums + tvbx_step_sums" or "tvbx_mfma_sums +
+ * tvbx_step_sums".  No counterpart in the reference. */
+int tvbx_sim_kernels(tvbx_sim *sim, char *buf, size_t len);
 /* execution mode of tvbx_sim_run: use_graph != 0 replays hipGraph-captured
  * windows of graph_window steps (the step counter lives on the device, so
  * one capture serves every window; runs with injected noise, remainders and

@@ -28,7 +28,7 @@ for N, deg, P, ring, ipl, L, bins, span in %r:
                        horizon=34 + span + L)
     log()
     s.run(L)
-    out.append(' + '.join(n for n, _ in log()))
+    out.append([' + '.join(n for n, _ in log()), s.kernels()])
     del s
 print(json.dumps(out))
 '''
@@ -64,5 +64,5 @@ RULE = [
 
 def test_kernels_of_a_launch():
     got = run(CODE % ([r[0] for r in RULE], ))
-    for (shape, want), kernels in zip(RULE, got):
-        assert kernels == want, (shape, kernels)
+    for (shape, want), (kernels, told) in zip(RULE, got):
+        assert kernels == want and told == want, (shape, kernels, told)

@@ -1256,9 +1256,17 @@ static bool split_launch(const tvbx_sim *s, const tvbx_step_args &a) {
          (long long)(s->pitch / 64) * d.n_node <= 256;
 }
 
-// One forward launch of a.n_steps steps: the step kernel of the launch
-// shape, or the kernel that forms the launch's sums (by gathers, or on the
-// matrix cores) and then the blocked updates from them.
+// The kernels of a forward launch: the step kernel of the launch shape, or the
+// kernel that forms the launch's sums (by gathers, or on the matrix cores) and
+// then the blocked updates from them.
+enum launch_kind { L_STEP, L_BLOCKED, L_SPLIT, L_SUMS, L_MFMA };
+static launch_kind launch_of(const tvbx_sim *s, const tvbx_step_args &a) {
+  if (split_launch(s, a)) return L_SPLIT;
+  if (a.csum) return s->mfma ? L_MFMA : L_SUMS;
+  return is_blocked(s->d) ? L_BLOCKED : L_STEP;
+}
+
+// One forward launch of a.n_steps steps.
 static hipError_t launch_steps(tvbx_sim *s, tvbx_step_args &a,
                                hipStream_t st) {
   const tvbx_sim_desc &d = s->d;
@@ -1266,23 +1274,47 @@ static hipError_t launch_steps(tvbx_sim *s, tvbx_step_args &a,
   const unsigned gy = (d.n_node + d.node_block - 1) / d.node_block;
   const unsigned bx = 64u * d.waves;
   void *params[] = {&a};
-  hipFunction_t fn = is_blocked(d) ? s->mod->blocked : s->mod->step;
-  if (split_launch(s, a))
-    return hipModuleLaunchKernel(s->mod->split, (unsigned)(s->pitch / 16),
-                                 (unsigned)d.n_node, 1, 192, 1, 1, 0, st,
-                                 params, nullptr);
-  if (a.csum) {
-    const hipError_t e =
-        s->mfma ? hipModuleLaunchKernel(s->mod->mfma, (d.n_node + 15) / 16, gx,
-                                        1, 256, 1, 1, 0, st, params, nullptr)
-                : hipModuleLaunchKernel(
-                      s->mod->sums, sums_grid(s), (unsigned)a.n_steps, 1, 256,
-                      1, 1, 0, st, params, nullptr);
-    if (e != hipSuccess) return e;
-    fn = s->mod->step_sums;
+  hipFunction_t fn = s->mod->step;
+  hipError_t e = hipSuccess;
+  switch (launch_of(s, a)) {
+    case L_STEP:
+      break;
+    case L_BLOCKED:
+      fn = s->mod->blocked;
+      break;
+    case L_SPLIT:
+      return hipModuleLaunchKernel(s->mod->split, (unsigned)(s->pitch / 16),
+                                   (unsigned)d.n_node, 1, 192, 1, 1, 0, st,
+                                   params, nullptr);
+    case L_SUMS:
+      e = hipModuleLaunchKernel(s->mod->sums, sums_grid(s),
+                                (unsigned)a.n_steps, 1, 256, 1, 1, 0, st,
+                                params, nullptr);
+      fn = s->mod->step_sums;
+      break;
+    case L_MFMA:
+      e = hipModuleLaunchKernel(s->mod->mfma, (d.n_node + 15) / 16, gx, 1, 256,
+                                1, 1, 0, st, params, nullptr);
+      fn = s->mod->step_sums;
+      break;
   }
+  if (e != hipSuccess) return e;
   return hipModuleLaunchKernel(fn, gx, gy, 1, bx, 1, 1, 0, st, params,
                                nullptr);
+}
+
+extern "C" int tvbx_sim_kernels(tvbx_sim *s, char *buf, size_t len) {
+  CHECK(s && buf && len, "null argument");
+  CHECK(s->have_connectome, "set the connectome first");
+  static const char *const names[] = {
+      "tvbx_step", "tvbx_step_blocked", "tvbx_step_split",
+      "tvbx_sums + tvbx_step_sums", "tvbx_mfma_sums + tvbx_step_sums"};
+  tvbx_step_args a;
+  fill_args(s, a);
+  const char *n = names[launch_of(s, a)];
+  CHECK(strlen(n) < len, "buffer too small");
+  strcpy(buf, n);
+  return TVBX_OK;
 }
 
 // reference ordering: the stale block read by step `step`
@@ -1919,9 +1951,6 @@ static long long graph_len(tvbx_sim *s) {
 // step / slot are offsets from the device clock, then the clock tick
 static int capture_window(tvbx_sim *s, long long W, hipGraphExec_t *out) {
   const tvbx_sim_desc &d = s->d;
-  const unsigned gx = s->pitch / (64 * d.ipl);
-  const unsigned gy = (d.n_node + d.node_block - 1) / d.node_block;
-  const unsigned bx = 64u * d.waves;
   hipStream_t st = s->ctx->stream;
   HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
   hipError_t e = hipSuccess;
@@ -2007,9 +2036,6 @@ extern "C" int tvbx_sim_run(tvbx_sim *s, long long n_steps,
     rc = up2d(s, s->noise.p, noise, steps_up * d.n_svar * d.n_node);
     if (rc != TVBX_OK) return rc;
   }
-  const unsigned gx = s->pitch / (64 * d.ipl);
-  const unsigned gy = (d.n_node + d.node_block - 1) / d.node_block;
-  const unsigned bx = 64u * d.waves;
   const long long W =
       (noise || s->forced_run || s->rec_forward) ? 0 : graph_len(s);
   long long done = 0;

@@ -100,6 +100,7 @@ _SIGS = {
     'tvbx_sim_init_history': [_P, _I],
     'tvbx_sim_set_noise': [_P, _I, ctypes.c_ulonglong],
     'tvbx_sim_run': [_P, _LL, _P, _LL],
+    'tvbx_sim_kernels': [_P, _P, _SZ],
     'tvbx_sim_set_exec': [_P, _I, _I, _I],
     'tvbx_sim_set_coupling': [_P, _I],
     'tvbx_sim_set_pacing': [_P, _I],
@@ -669,6 +670,12 @@ class Simulation:
             check(lib().tvbx_sim_set_noise(self.h, 0, 0))
         else:
             check(lib().tvbx_sim_set_noise(self.h, 1, int(seed)))
+
+    def kernels(self):
+        "The kernels of one launch, in order and joined by ' + '."
+        buf = ctypes.create_string_buffer(128)
+        check(lib().tvbx_sim_kernels(self.h, buf, 128))
+        return buf.value.decode()
 
     def set_exec(self, graph=True, window=100, profile=False):
         """graph: replay hipGraph windows of `window` steps (launches of 8

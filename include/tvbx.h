@@ -369,8 +369,9 @@ int tvbx_fc_loss_grad(tvbx_ctx *ctx, const float *samples, long long n, int N,
                       const float *gout, float *dsamples);
 /* out[c][r] = in[r][c] - sub[r % sub_rows][c] (sub may be null): device
  * arrays, in [rows][cols] -> out [cols][rows].  No counterpart in the
- * reference: it moves the FC-loss gradient's operands between the
- * instance-innermost layout and the instance-major one of batched products. */
+ * reference: where batched products form the FC loss's gradient, it moves
+ * their operands between the instance-innermost layout and the
+ * instance-major one. */
 int tvbx_transpose(tvbx_ctx *ctx, const float *in, long long rows,
                    long long cols, const float *sub, int sub_rows, float *out);
 

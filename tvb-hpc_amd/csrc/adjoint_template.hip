@@ -66,46 +66,46 @@ __device__ __forceinline__ void tvbx_adj_gather(
   const int deg = crw.e1 - crw.e0;
 #define TVBX_ADJ_SRC(C)                                                       \
   reinterpret_cast<const float *>(                                            \
-  reinterpret_cast<const char *>(                                         \
-      mu_r + ((size_t)(t + (int)((C) >> 16) -                             \
-                       ((t + (int)((C) >> 16)) >= H ? H : 0)) * N +       \
-              ((C) & 0xffffu)) * a.pitch) +                               \
-  tvbx_lane_offset(lane_off))
+      reinterpret_cast<const char *>(                                         \
+          mu_r + ((size_t)(t + (int)((C) >> 16) -                             \
+                           ((t + (int)((C) >> 16)) >= H ? H : 0)) * N +       \
+                  ((C) & 0xffffu)) * a.pitch) +                               \
+      tvbx_lane_offset(lane_off))
 // the same with buffer loads at the byte offsets OV (read back per edge)
 #define TVBX_ADJ_BRANGE(NE, OV, WV)                                           \
   {                                                                           \
     int u0 = 0;                                                               \
     for (; u0 + TVBX_ADJ_UNROLL <= (NE); u0 += TVBX_ADJ_UNROLL) {             \
-  unsigned so[TVBX_ADJ_UNROLL];                                           \
-  float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
-      tvbx_lane_u((OV), u0 + u);                                          \
-  __builtin_amdgcn_sched_barrier(0);                                      \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
-      tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
-  __builtin_amdgcn_sched_barrier(0);                                      \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-    const float we = tvbx_lane_f((WV), u0 + u);                           \
-    _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
-        fmaf(we, v[u][q], accm[q]);                                       \
-  }                                                                       \
+      unsigned so[TVBX_ADJ_UNROLL];                                           \
+      float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
+          tvbx_lane_u((OV), u0 + u);                                          \
+      __builtin_amdgcn_sched_barrier(0);                                      \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
+          tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
+      __builtin_amdgcn_sched_barrier(0);                                      \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+        const float we = tvbx_lane_f((WV), u0 + u);                           \
+        _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
+            fmaf(we, v[u][q], accm[q]);                                       \
+      }                                                                       \
     }                                                                         \
     if (u0 < (NE)) {                                                          \
-  /* the remainder as one group: a slot past the row reads the row's */   \
-  /* last edge again, with the weight 0 its lane holds (adds nothing) */  \
-  unsigned so[TVBX_ADJ_UNROLL];                                           \
-  float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
-      tvbx_lane_u((OV), min(u0 + u, (NE) - 1));                           \
-  __builtin_amdgcn_sched_barrier(0);                                      \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
-      tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
-  __builtin_amdgcn_sched_barrier(0);                                      \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-    const float we = tvbx_lane_f((WV), u0 + u);                           \
-    _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
-        fmaf(we, v[u][q], accm[q]);                                       \
-  }                                                                       \
+      /* the remainder as one group: a slot past the row reads the row's */   \
+      /* last edge again, with the weight 0 its lane holds (adds nothing) */  \
+      unsigned so[TVBX_ADJ_UNROLL];                                           \
+      float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) so[u] =     \
+          tvbx_lane_u((OV), min(u0 + u, (NE) - 1));                           \
+      __builtin_amdgcn_sched_barrier(0);                                      \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u)             \
+          tvbx_bloadf(mrs, lane_off, so[u], v[u]);                            \
+      __builtin_amdgcn_sched_barrier(0);                                      \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+        const float we = tvbx_lane_f((WV), u0 + u);                           \
+        _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
+            fmaf(we, v[u][q], accm[q]);                                       \
+      }                                                                       \
     }                                                                         \
   }
 // TVBX_ADJ_UNROLL gathers in flight, accumulated in CSC order
@@ -113,24 +113,24 @@ __device__ __forceinline__ void tvbx_adj_gather(
   {                                                                           \
     int u0 = 0;                                                               \
     for (; u0 + TVBX_ADJ_UNROLL <= (NE); u0 += TVBX_ADJ_UNROLL) {             \
-  float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-    const unsigned c = tvbx_lane_u((CV), u0 + u);                         \
-    tvbx_ldf(TVBX_ADJ_SRC(c), v[u]);                                      \
-  }                                                                       \
-  _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
-    const float we = tvbx_lane_f((WV), u0 + u);                           \
-    _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
-        fmaf(we, v[u][q], accm[q]);                                       \
-  }                                                                       \
+      float v[TVBX_ADJ_UNROLL][TVBX_IPL];                                     \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+        const unsigned c = tvbx_lane_u((CV), u0 + u);                         \
+        tvbx_ldf(TVBX_ADJ_SRC(c), v[u]);                                      \
+      }                                                                       \
+      _Pragma("unroll") for (int u = 0; u < TVBX_ADJ_UNROLL; ++u) {           \
+        const float we = tvbx_lane_f((WV), u0 + u);                           \
+        _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =        \
+            fmaf(we, v[u][q], accm[q]);                                       \
+      }                                                                       \
     }                                                                         \
     for (; u0 < (NE); ++u0) {                                                 \
-  const unsigned c = tvbx_lane_u((CV), u0);                               \
-  float v[TVBX_IPL];                                                      \
-  tvbx_ldf(TVBX_ADJ_SRC(c), v);                                           \
-  const float we = tvbx_lane_f((WV), u0);                                 \
-  _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =          \
-      fmaf(we, v[q], accm[q]);                                            \
+      const unsigned c = tvbx_lane_u((CV), u0);                               \
+      float v[TVBX_IPL];                                                      \
+      tvbx_ldf(TVBX_ADJ_SRC(c), v);                                           \
+      const float we = tvbx_lane_f((WV), u0);                                 \
+      _Pragma("unroll") for (int q = 0; q < TVBX_IPL; ++q) accm[q] =          \
+          fmaf(we, v[q], accm[q]);                                            \
     }                                                                         \
   }
   if (mu32) {

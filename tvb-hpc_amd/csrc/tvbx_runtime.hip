@@ -581,9 +581,9 @@ __host__ __device__ inline size_t tri_index(int i, int j, int N) {
 // With d_k = x_k - shift for any per-(node, instance) shift,
 //   sum_k (x_ki - mb_i)(x_kj - mb_j) = sum_k d_ki d_kj - S1_i S1_j / m,
 //   S1 = sum_k d_k,
-// so no second pass over the block needs its mean.  The shift is the running mean rounded to
-// float (the block's first sample before the first merge), which keeps d
-// small and makes x - shift exact in double.
+// so no second pass over the block needs its mean.  The shift is the running
+// mean rounded to float (the block's first sample before the first merge),
+// which keeps d small and makes x - shift exact in double.
 
 // per (node, instance): shift, S1 and u of the block; rows of ld >= the
 // instances in use.  The 4 waves of a workgroup take a quarter of the samples
@@ -656,8 +656,9 @@ typedef double fc_d4 __attribute__((ext_vector_type(4)));
 // x[pl][k * 48 + r] (r < 16: row node I0 + r, else column node J0 + r - 16;
 // 16 dwords of padding per sample and one per instance; "sample" 4 holds the
 // 32 nodes' shifts, written once), so the operand reads (lanes = (k, node))
-// fall in distinct banks; a wave stages half of one sample's node rows, and the next 4 samples' global loads are in flight while the current ones
-// are multiplied.  d = x - shift is formed in FP64 at the operand (exact, as
+// fall in distinct banks; a wave stages half of one sample's node rows, and the
+// next 4 samples' global loads are in flight while the current ones are
+// multiplied.  d = x - shift is formed in FP64 at the operand (exact, as
 // the shift is the float running mean).  With PB = 32 (128-byte loads,
 // 31 KB of LDS) 3 workgroups of 8 waves share a CU; PB = 16 gives twice the
 // workgroups, 4 to a CU, for problems that would not fill the chip (the rule
@@ -1076,7 +1077,6 @@ static int sim_alloc(tvbx_sim *s, DevBuf &b, size_t bytes) {
   return dalloc(b, bytes);
 }
 
-// host [rows][P] <-> device [rows][pitch]
 // true when p is device memory that kernels can read and write directly
 static bool on_device(const void *p) {
   hipPointerAttribute_t at;
@@ -1087,8 +1087,6 @@ static bool on_device(const void *p) {
   return at.type == hipMemoryTypeDevice;
 }
 
-// [rows][P] float32 arrays in host or device memory (the copy kind is
-// inferred from the addresses) <-> pitched device rows
 // `rows` rows of `width` bytes from src (row pitch sp) to dst (dp), queued on
 // the context's stream; host memory has rows side by side.  One copy where
 // both sides are contiguous; else the device's side is packed or unpacked on

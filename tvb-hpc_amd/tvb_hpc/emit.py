@@ -284,7 +284,6 @@ class KernelSpec:
             lines.append('#define TVBX_PIPE 1')
         lines.append('#define TVBX_PRIO %d' % int(self.prio))
         lines.append('#define TVBX_EMAJ %d' % self.emaj)
-        lines.append('#define TVBX_ADJOINT %d' % int(self.adjoint))
         # lane parameters
         fields = self._lane_fields()
         lines.append('struct tvbx_lane_params {')

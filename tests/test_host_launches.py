@@ -66,3 +66,29 @@ def test_kernels_of_a_launch():
     got = run(CODE % ([r[0] for r in RULE], ))
     for (shape, want), (kernels, told) in zip(RULE, got):
         assert kernels == want and told == want, (shape, kernels, told)
+
+
+SPLIT = r'''
+out = []
+for N, deg, P, L in %r:
+    m = M.Kuramoto()
+    s = hip.Simulation(m, CF.Kuramoto(m), SC.EulerStep(0.05), csr(N, deg, 12),
+                       P, params={'c:a': np.full(P, 0.1, np.float32)},
+                       kinds={'c:a': 'inst'}, waves=1, node_block=1,
+                       steps_per_launch=L, horizon=300)
+    log()
+    s.run(L)
+    out.append([n for n, _ in log()] + [s.kernels()])
+print(json.dumps(out))
+'''
+
+
+@pytest.mark.parametrize('shape,split', [
+    ((76, 22, 64, 10), True), ((256, 20, 64, 2), True),
+    ((257, 20, 64, 8), False),                    # more than 256 pairs
+    ((128, 20, 128, 8), True), ((129, 20, 128, 8), False),
+    ((200, 5, 64, 8), True), ((200, 5, 64, 4), False),   # short rows
+    ((128, 5, 64, 4), True), ((128, 5, 64, 3), False)])
+def test_split_launches(shape, split):
+    name = 'tvbx_step_split' if split else 'tvbx_step_blocked'
+    assert run(SPLIT % ([shape], )) == [[name, name]]

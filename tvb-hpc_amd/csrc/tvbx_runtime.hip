@@ -1247,11 +1247,19 @@ static unsigned sums_grid(const tvbx_sim *s) {
 // 3.35 / 1.38, 152 3.36 / 1.48; 60 edges, 64 pairs 5.25 / 1.92, 256 5.23 /
 // 2.18; differences (no sine), 20 edges, 64 pairs 1.62 / 0.87, 256 1.55 /
 // 1.07; 60 edges, 256 pairs 2.56 / 1.71; 70 edges (two blocks) 152 pairs
-// 2.94 / 2.66, 304 2.92 / 3.15, 380 3.54 / 5.11.
+// 2.94 / 2.66, 304 2.92 / 3.15, 380 3.54 / 5.11.  Short launches of short rows
+// do not pay for a workgroup's start, the less the more of them there are:
+// Kuramoto, 5 edges a row, 256 pairs, 2, 3, 4, 5 and 8 steps 3.23 / 3.74, 2.75
+// / 3.01, 2.50 / 2.63, 2.35 / 2.36 and 2.13 / 1.99; 76 pairs, 2, 3 and 4 steps
+// 3.14 / 3.32, 2.67 / 2.66, 2.44 / 2.32; 20 edges, 256 pairs, 2 steps 4.67 /
+// 4.21.
 static bool split_launch(const tvbx_sim *s, const tvbx_step_args &a) {
   const tvbx_sim_desc &d = s->d;
+  const long long pairs = (long long)(s->pitch / 64) * d.n_node;
   return is_blocked(d) && s->mod->split && !a.csum && !a.pace && a.ring32 &&
-         (long long)(s->pitch / 64) * d.n_node <= 256;
+         pairs <= 256 &&
+         ((double)d.steps_per_launch * d.nnz >= 24.0 * d.n_node ||
+          (d.steps_per_launch >= 4 && pairs <= 128));
 }
 
 // The kernels of a forward launch: the step kernel of the launch shape, or the

@@ -3037,8 +3037,10 @@ k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
   const int r = blockIdx.x;
   const long long cb = (long long)blockIdx.z * gridDim.y + blockIdx.y;
   if (cb * 64 >= C) return;  // whole workgroup
-  const int m0 = rptr[r], m1 = rptr[r + 1];
-  const int nt = (m1 - m0 + V - 1) / V;
+  // (unsigned: an index past the last tile, before it is cut off, may be past
+  // 2^31)
+  const unsigned m0 = (unsigned)rptr[r], m1 = (unsigned)rptr[r + 1];
+  const int nt = (int)((m1 - m0 + V - 1) / V);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (wave == 0) {
     // the sums; lanes past CP or C repeat a column and store nothing
@@ -3048,7 +3050,7 @@ k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
       __syncthreads();  // tile t is in buffer t & 1
       const float4 *__restrict__ t4 =
           reinterpret_cast<const float4 *>(tile[t & 1] + c * LD);
-      const int n4 = (min(V, m1 - m0 - t * V) + 3) / 4;
+      const int n4 = ((int)min((unsigned)V, m1 - m0 - (unsigned)t * V) + 3) / 4;
       // two batches of B reads by turns, whole batches (V is a multiple of
       // 8 B): what lies past the region in the tile is zeros
       float4 q[2][B];
@@ -3087,7 +3089,7 @@ k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
   auto index = [&](int t) {
 #pragma unroll
     for (int u = 0; u < RM_V; ++u)
-      k[u] = members[min(m0 + t * V + u * RV + row, m1 - 1)];
+      k[u] = members[min(m0 + (unsigned)t * V + u * RV + row, m1 - 1u)];
   };
   auto fetch = [&]() {
 #pragma unroll
@@ -3103,7 +3105,8 @@ k_rmap_to_avg(const int *__restrict__ rptr, const int *__restrict__ members,
 #pragma unroll
       for (int u = 0; u < RM_V; ++u) {
         const int x = u * RV + row;
-        tile[t & 1][c * LD + x] = m0 + t * V + x < m1 ? v[u] : 0.0f;
+        tile[t & 1][c * LD + x] =
+            m0 + (unsigned)t * V + x < m1 ? v[u] : 0.0f;
       }
       if (t + RM_D < nt) {
         fetch();
